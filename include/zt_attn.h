@@ -336,7 +336,9 @@ int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_til
  *   ZT_DQDS_K 1|2 (key parts of the dq-from-dS product), ZT_ATTN_RSCORES
  *   0|1 (the row-split dk/dv kernel reading the forward's scores for head
  *   groups that cannot be halved; 0 = it forms S again and the forward keeps
- *   none).
+ *   none), ZT_ATTN_FSHAPE 11|12|14|21|22 (the forward's wave shape on split
+ *   operands, 16-row blocks per wave then key parts; one the kernel does not
+ *   hold falls back to one it does).
  * Returns 0, or 1 (reason on stderr) for an unknown name or value.  The
  * process environment is never read.  Not synchronised with launches in
  * flight on other threads: set before launching. */

@@ -1,0 +1,76 @@
+"""The kernels that form f32 products from three bf16 parts per operand
+(csrc/kernels/split.h): every wave shape of the forward against a float64
+reference, at tile edges and remainders, and operands too large for the split
+(infinities, magnitudes of 2^60 and more), which take f32 products instead.
+
+Gate: an output is a convex combination of V rows (|V| up to about 5 here), so
+an error of 2^-22 in a weight's exponent and 2^-22 in its product are below
+5e-6 in it; the score error is a few 2^-24 of a sum of d products of order
+sqrt(d) before the 1/sqrt(d) scale.  2e-5 covers the sum of both at d = 256.
+"""
+import numpy as np
+import pytest
+
+from gpuhelp import SEED_K, SEED_Q, SEED_V, dev_normal, host
+from npref import attention_f64
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-5
+
+
+def _forward(gpu, zt, q, k, v, T, H, Hkv, D):
+    out = gpu.full((T * H * D,), float("nan"), device="cuda")
+    zt.forward(q, k, v, out, T, H, Hkv, D)
+    gpu.cuda.synchronize()
+    return host(out)
+
+
+def _inputs(gpu, zt, T, H, Hkv, D):
+    return (dev_normal(gpu, zt, T * H * D, SEED_Q), dev_normal(gpu, zt, T * Hkv * D, SEED_K),
+            dev_normal(gpu, zt, T * Hkv * D, SEED_V))
+
+
+@pytest.mark.parametrize("shape", [11, 12, 14, 21, 22])
+@pytest.mark.parametrize("T,H,Hkv,D", [(2, 4, 2, 32), (33, 4, 2, 32), (129, 4, 1, 64), (257, 3, 1, 64), (63, 2, 2, 36),
+                                       (65, 4, 1, 96), (100, 4, 4, 128), (161, 8, 2, 128), (97, 2, 1, 192),
+                                       (70, 4, 1, 256), (31, 2, 2, 256)])
+def test_every_wave_shape(gpu, zt, tune, shape, T, H, Hkv, D):
+    """(A shape a width does not have falls back to one it has.)"""
+    tune({"ZT_ATTN_FSHAPE": shape})
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    want = attention_f64(host(q), host(k), host(v), T, H, Hkv, D).ravel()
+    assert np.max(np.abs(_forward(gpu, zt, q, k, v, T, H, Hkv, D) - want)) <= TOL
+
+
+@pytest.mark.parametrize("shape", [12, 21])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("where", ["k", "v", "q", "kq"])
+def test_large_finite_operands_take_the_f32_products(gpu, zt, tune, shape, D, where):
+    """An entry of 2^70 in one row of K, V or Q (and in both K and Q, at
+    different columns, so no product of two of them): its own products are
+    formed in f32, and rows and columns it does not reach keep their bits."""
+    tune({"ZT_ATTN_FSHAPE": shape})
+    T, H, Hkv, S = 150, 4, 2, 70
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    good = _forward(gpu, zt, q, k, v, T, H, Hkv, D).reshape(T, H, D)
+    big = 2.0 ** 70
+    if "k" in where:
+        k = k.clone()
+        k.view(T, Hkv, D)[S, 1, 3] = -big
+    if "q" in where:
+        q = q.clone()
+        q.view(T, H, D)[S, 2, 5] = big
+    if "v" in where:
+        v = v.clone()
+        v.view(T, Hkv, D)[S, 1, 3] = big
+    got = _forward(gpu, zt, q, k, v, T, H, Hkv, D).reshape(T, H, D)
+    want = attention_f64(host(q), host(k), host(v), T, H, Hkv, D).reshape(T, H, D)
+    scale = np.maximum(1.0, np.abs(want))
+    assert np.max(np.abs(got - want) / scale) <= TOL
+    assert np.array_equal(got[:, :2].view(np.uint32), good[:, :2].view(np.uint32))      # the other kv head
+    if where != "kq":  # (a tile with both is formed in f32 throughout)
+        assert np.array_equal(got[:S].view(np.uint32), good[:S].view(np.uint32))        # earlier rows
+    if where == "v":
+        keep = [c for c in range(D) if c != 3]
+        assert np.array_equal(got[..., keep].view(np.uint32), good[..., keep].view(np.uint32))

@@ -22,7 +22,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 KERNELS = [("fwd", "attn_fwd.hip"), ("bwd", "attn_bwd.hip"), ("dec", "attn_decode.hip"), ("misc", "norm_rope.hip"),
            ("cal", "calibrate.hip"), ("gemm", "gemm.hip")]
-HIP_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
+HIP_FLAGS = ["-O3", "-std=c++20", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-Wall"]
 LIB = os.path.join(BUILD, "libzt_attn.so")
 

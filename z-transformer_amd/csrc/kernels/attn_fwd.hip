@@ -19,6 +19,7 @@
 // spreads across the XCDs -- keep one kv group's K/V per XCD L2.
 #include "common.h"
 #include "args.h"
+#include "split.h"
 
 
 // KS > 1 (key split): the workgroup's waves are KS key parts x (NW / KS) row
@@ -301,6 +302,499 @@ __device__ __forceinline__ void attn_fwd_body(const FwdArgs &a) {
     }
 }
 
+// ---- The forward on split operands (split.h) --------------------------------
+//
+// The schedule of the wide-row kernels (dim % 4 == 0): the same two products
+// S^T = K Q^T and O^T += V^T P^T and the same softmax as attn_fwd_tile, on the
+// bf16 matrix cores.  A wave owns NQ blocks of 16 query rows of one head, the
+// workgroup HW heads of one kv group x RB row blocks x KS key parts x DS column
+// halves of waves.
+//   * K and V tiles of 32 keys (per key part) are split once while they are
+//     staged and shared by the workgroup's waves, row-major in LDS; the V^T
+//     operand comes from the same layout through the transposing LDS read.
+//   * Two phases per step, a barrier after each: scores, then softmax and
+//     output product.  Eight waves, where two buffers each of K and V fit in
+//     LDS (ALT): the second four waves, one per SIMD, run half a step behind
+//     the first, so that on every SIMD one wave's softmax and staging run
+//     beside the other's MFMAs; the score phase stages the next K and the
+//     output phase the next V.  Otherwise one buffer each: the waves write this
+//     step's V while they multiply K and the next K while they multiply V.
+//   * Q's split stays in registers (12 per 32 columns and row block), P's is
+//     formed from the score registers.
+//   * O accumulates 32-key sums with f32 adds: four vector adds beside six
+//     MFMAs, and a long row takes T / 32 roundings instead of 6 T / 32.
+// What bounds it: on a full chip, power -- operands like these hold a loop of
+// nothing but these MFMAs to 1.8 PFLOP/s, 300 TFLOP/s of f32 products -- and the
+// vector work beside it (a 16 x 16 score block at d = 128 is 48 MFMAs of 16
+// cycles; its softmax and split about 70 vector instructions).  32 over 8 heads,
+// d = 128, T = 4096: 1012 us on f32 MFMAs, 614 us here (224 TFLOP/s), with the
+// scores kept 1053 / 705 us; d = 256, 2 x 2048 rows of 16 over 4 heads 538 / 437 us.
+// On small grids, the latency of a step (fetch, split, barrier, two dependent
+// products): 512 rows of that first shape 70 / 34 us.  Two row blocks per wave (NQ = 2) read each K and V
+// operand from LDS once for 32 rows: at one block the operand reads alone
+// (49 KB per wave and tile at d = 128) would take as long as the MFMAs.
+template <int DP, int DS, int NW, int NQ, int KS>
+struct FwdSplit {
+    static constexpr int DW = DP / DS;      // columns per wave
+    static constexpr int NT = DW / 16;      // 16-wide output tiles per wave
+    static constexpr int NKS = DW / 32;     // 32-wide contraction steps of the score product
+    static constexpr int ROWS = 32 * KS;    // keys staged per step
+    static constexpr int TILE = split_bytes<DP>(ROWS);
+    static constexpr int XCHG = DS > 1 ? NW * 2 * NQ * 1024 : 0;  // partial scores of the column halves
+    static constexpr int MERGE = (KS - 1) * (NW / KS) * 64 * (4 * NQ * NT + 2 * NQ) * 4;
+    // Alternating wave halves (below): two buffers each for K and V.
+    static constexpr bool ALT = NW == 8 && DS == 1 && 4 * TILE + 16 <= 160 * 1024;
+    static constexpr int BUFS = ALT ? 2 : 1;
+    static constexpr int FLAGS = 2 * BUFS * TILE + XCHG;  // offset of the big-value flags
+    static constexpr int BYTES = FLAGS + 16;
+    static_assert(MERGE <= 2 * BUFS * TILE, "the key parts merge in the tiles' space");
+    static_assert(BYTES <= 160 * 1024, "LDS");
+};
+
+// 4 x 4 transpose within each group of four lanes: lane i ends with element i
+// of the group's lanes 0..3.
+DEVI f4 quad_transpose(f4 x, int lane) {
+    const bool o1 = lane & 1, o2 = lane & 2;
+    // (The lane exchanges are outside the selects: every lane takes part.)
+    auto xor1 = [](float v) { return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0xb1, 0xf, 0xf, true)); };
+    auto xor2 = [](float v) { return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x4e, 0xf, 0xf, true)); };
+    const float x0 = xor1(x.x), x1 = xor1(x.y), x2 = xor1(x.z), x3 = xor1(x.w);
+    const float a0 = o1 ? x1 : x.x, a1 = o1 ? x.y : x0, a2 = o1 ? x3 : x.z, a3 = o1 ? x.w : x2;
+    const float y0 = xor2(a0), y1 = xor2(a1), y2 = xor2(a2), y3 = xor2(a3);
+    return f4{o2 ? y2 : a0, o2 ? y3 : a1, o2 ? a2 : y0, o2 ? a3 : y1};
+}
+
+template <int DP, int DS, int NW, int NQ, int KS, int SC>
+DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int &sid) {
+    using C = FwdSplit<DP, DS, NW, NQ, KS>;
+    constexpr int DW = C::DW, NT = C::NT, NKS = C::NKS, ROWS = C::ROWS, NTH = 64 * NW, NWR = NW / (KS * DS);
+    constexpr bool ALT = C::ALT;
+    char *const xchg = smem + 2 * C::BUFS * C::TILE;
+    // The K (V) tile of a step, and the flag that holds the step's id if the tile has a big value.
+    auto ktile = [&](int id) { return smem + (ALT ? (id & 1) * 2 * C::TILE : 0); };
+    auto vtile = [&](int id) { return ktile(id) + C::TILE; };
+    auto kflag = [&](int id) { return reinterpret_cast<int *>(smem + C::FLAGS) + (ALT ? (id & 1) * 2 : 0); };
+    auto vflag = [&](int id) { return kflag(id) + 1; };
+
+    const int tid = opaque((int)threadIdx.x), lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kh = w / (NW / KS);       // key part
+    const int dh = (w / NWR) % DS;      // column half
+    const int wr = w % NWR;             // (head, row block) slot
+    const int RB = NWR / a.HW;
+    const int per_tile = a.n_head_blocks * a.B;
+    const int rem = (int)blockIdx.x % per_tile;
+    const int hb = rem % a.n_head_blocks, b = rem / a.n_head_blocks;
+    const int h = hb * a.HW + (wr % a.HW);
+    const int kvh = ZT_PLANT == 2 ? 0 : h / (a.H / a.Hkv);
+    const int wg_row0 = tile * 16 * NQ * RB;
+    const int row0 = wg_row0 + 16 * NQ * (wr / a.HW);
+    const size_t qld = (size_t)a.H * a.dim, kld = (size_t)a.Hkv * a.dim;
+    const float *qb = a.q + (size_t)b * a.T * qld + (size_t)h * a.dim;
+    const float *kb = a.k + (size_t)b * a.kv_rows * kld + (size_t)kvh * a.dim;
+    const float *vb = a.v + (size_t)b * a.kv_rows * kld + (size_t)kvh * a.dim;
+    const float qscale = ZT_PLANT == 4 ? kLog2e : a.scale_log2e;
+
+    // Staging: thread tid takes the 8-column chunks e = tid + n NTH of the
+    // step's ROWS x DP tile.  Loads are unconditional and in bounds: rows past
+    // n_keys load row n_keys - 1 (masked scores, weight 0), columns past dim
+    // the row's last floats (replaced by 0).
+    constexpr int CPR = DP / 8, CH = ROWS * CPR, NP = (CH + NTH - 1) / NTH;
+    constexpr bool EVEN = CH % NTH == 0;
+    // Byte offsets within a tile's rows, fixed for the kernel; a fetch clamps
+    // them (one min) to row n_keys - 1 counted within the tile.  ROWS kld 4 <
+    // 2^32 at every width and head count admitted (ROWS DP <= 8192).
+    constexpr int NC = NTH % CPR == 0 ? 1 : NP;  // distinct columns among a thread's chunks
+    unsigned voff[NP], vcol[NC], vcol2[NC];
+#pragma unroll
+    for (int n = 0; n < NP; ++n) voff[n] = (unsigned)((tid + n * NTH) / CPR) * (unsigned)kld * 4u;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+        const int c = (tid + n * NTH) % CPR * 8;
+        vcol[n] = (unsigned)min(c, a.dim - 4) * 4u;
+        // The chunk's second half; past dim it is replaced by 0, so anything in bounds will do.
+        vcol2[n] = c + 4 < a.dim ? vcol[n] + 16u : vcol[n];
+    }
+    auto fetch = [&](f4 (&x)[NP][2], const float *base, int k0) {
+        const unsigned last = (unsigned)min(a.n_keys - 1 - k0, ROWS - 1) * (unsigned)kld * 4u;
+        const char *p = reinterpret_cast<const char *>(base + (size_t)k0 * kld);
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            if (!EVEN && tid + n * NTH >= CH) break;  // wave-uniform: CH is a multiple of 64
+            const unsigned r = min(voff[n], last);
+            x[n][0] = *reinterpret_cast<const f4 *>(p + (r + vcol[n % NC]));
+            x[n][1] = *reinterpret_cast<const f4 *>(p + (r + vcol2[n % NC]));
+        }
+    };
+    auto put = [&](const f4 (&x)[NP][2], char *t, int *flag, int id) {
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            const int e = tid + n * NTH;
+            if (!EVEN && e >= CH) break;
+            const int c = (e % CPR) * 8;
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = x[n][i / 4][i % 4];
+            if (a.dim < DP) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = c + (i & 4) < a.dim ? y[i] : 0.f;
+            }
+            if (any_big(max_abs(y))) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+                if (lane == 0) *flag = id;
+            }
+            put_tri<DP>(t, ROWS, e / CPR, c, split8(y));
+        }
+    };
+
+    // Q: the B operand of the score product, lane l16 = row, k slot = column.
+    Tri q[NKS][NQ];
+    float qmax = 0.f;
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+        const int row = row0 + 16 * n + l16;
+        const float *qrow = qb + (size_t)min(row, a.T - 1) * qld;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const int c = dh * DW + 32 * ks + 8 * grp;
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; i += 4) {
+                // Unconditional and in bounds; rows past T and columns past dim are 0.
+                const f4 x = *reinterpret_cast<const f4 *>(qrow + min(c + i, a.dim - 4));
+                const bool in = row < a.T && c + i < a.dim;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[i + e] = in ? x[e] * qscale : 0.f;
+            }
+            const float mx = max_abs(y);
+            qmax = vmax(qmax, mx);
+            if (any_big(mx)) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+            }
+            q[ks][n] = split8(y);
+        }
+    }
+    const bool qbig = any_big(qmax);
+
+    f4 o[NT][NQ];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) o[i][n] = zero4();
+    float m[NQ], lsum[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) { m[n] = -INFINITY; lsum[n] = 0.f; }
+    const int kend_wg = min(a.n_keys, a.q_offset + min(a.T, wg_row0 + 16 * NQ * RB));
+    const int kend_w = row0 < a.T ? min(a.n_keys, a.q_offset + min(a.T, row0 + 16 * NQ)) : 0;
+
+    // Scores (kept if SC) to weights in s, the row state updated.
+    f4 s[2 * NQ];  // s[j NQ + n]: keys k0 + 16 j + 4 grp + r of row block n
+    auto softmax = [&](const int k0) {
+        if (SC == 1 || (SC == 2 && a.s_out)) {
+        // Element (t = row + l16, s = k0 + 16 j + 4 grp + r) belongs at lane
+        // (s & 15) + 16 ((t & 15) >> 2), element t & 3 of its tile: after the
+        // quad transpose a lane holds four consecutive rows of one key, and
+        // the wave's 16-byte stores cover the tile's 1 KB (nontemporal: the
+        // tiles would displace the K/V rows the workgroups share in L2).
+        const int nt = (a.T + 15) >> 4;
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+            if (DS > 1 && n % DS != dh) continue;
+            const int r0 = row0 + 16 * n;
+            const int kend = r0 < a.T ? min(a.n_keys, min(a.T, r0 + 16)) : 0;
+            float *srow = a.s_out +
+                          (((size_t)b * a.H + h) * zt_tri_count(nt) + zt_tri_index(r0 >> 4, k0 >> 4)) * 256 +
+                          (4 * grp + (l16 & 3) + 16 * (l16 >> 2)) * 4;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if (k0 + 16 * j >= kend) continue;  // wave-uniform: above the diagonal
+                f4 x = quad_transpose(s[j * NQ + n], lane);
+                if (ZT_PLANT == 5) x = x / a.scale_log2e;
+                __builtin_nontemporal_store(x, reinterpret_cast<f4 *>(srow + j * 256));
+            }
+        }
+        }
+        if (k0 + 31 > a.q_offset + row0 || k0 + 32 > a.n_keys) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < 2 * NQ; ++i) {
+            const int qpos = a.q_offset + row0 + 16 * (i % NQ) + l16;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = k0 + 16 * (i / NQ) + 4 * grp + r;
+                if ((ZT_PLANT != 1 && key > qpos) || key >= a.n_keys) s[i][r] = -INFINITY;
+            }
+        }
+        }
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = s[(i / 4) * NQ + n][i % 4];
+        const float mt = max4grp(vmax_n(y));
+        // Lazy rescaling, per row (attn_fwd_tile).
+        if (ZT_PLANT == 3 || mt > m[n] + 8.f) {
+            const float mnew = fmaxf(m[n], mt);
+            const float corr = fast_exp2(m[n] - mnew);
+            m[n] = mnew;
+            lsum[n] = ZT_PLANT == 3 ? lsum[n] : lsum[n] * corr;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) o[i][n] *= ZT_PLANT == 3 ? 1.f : corr;
+        }
+        // A row whose every key so far is masked (a later row block, or a
+        // key part past the first) keeps base -inf, taken as 0 here so that
+        // exp2(-inf) = 0.
+        const float mb = m[n] == -INFINITY ? 0.f : m[n];
+        float ps = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            y[i] = fast_exp2(y[i] - mb);
+            s[(i / 4) * NQ + n][i % 4] = y[i];
+            ps = i == 0 ? y[0] : ps + y[i];
+        }
+        lsum[n] += ps;
+        }
+    };
+    // Where registers allow (DEEP) a tile is fetched a whole step before it is
+    // written to LDS, else in the phase that writes it, which is shorter than the
+    // loads' latency for small tiles.
+    constexpr bool DEEP = NQ == 1 || DW <= 64;
+    f4 px[NP][2], py[DEEP ? NP : 1][2];
+    auto stage_k = [&](int id) { put(px, ktile(id), kflag(id), id); };
+    auto stage_v = [&](int id) {
+        if constexpr (DEEP) put(py, vtile(id), vflag(id), id);
+        else put(px, vtile(id), vflag(id), id);
+    };
+    const int klast = (kend_wg - 1) / ROWS * ROWS;  // the last step's first key
+    fetch(px, kb, 0);
+    stage_k(sid + 1);
+    if constexpr (DEEP) fetch(py, vb, 0);
+    if constexpr (ALT) {
+        if constexpr (!DEEP) fetch(px, vb, 0);
+        stage_v(sid + 1);
+        if constexpr (DEEP) fetch(py, vb, min(ROWS, klast));
+    }
+    if constexpr (DEEP) fetch(px, kb, min(ROWS, klast));
+    __syncthreads();
+    // Half a step behind: the second half's waves meet one barrier more here, the first half's one more at the end.
+    if (ALT && w >= NW / 2) __syncthreads();
+    for (int ks0 = 0; ks0 < kend_wg; ks0 += ROWS) {
+        ++sid;
+        // The steps after this one (the last loads itself again, unused).
+        const int kn = min(ks0 + ROWS, klast), kn2 = min(ks0 + 2 * ROWS, klast);
+        const int k0 = ks0 + 32 * kh;
+        const bool active = k0 < kend_w;  // wave-uniform
+        // Phase A: scores; this step's V (ALT: the next K) into LDS.
+        if constexpr (!DEEP) fetch(px, ALT ? kb : vb, ALT ? kn : ks0);
+        const char *const Ks = ktile(sid), *const Vs = vtile(sid);
+        if (active) {
+#pragma unroll
+            for (int i = 0; i < 2 * NQ; ++i) s[i] = zero4();
+            // One 16-key block at a time: step (j, ks) = (i / NKS, i % NKS).
+            stream_parts<2 * NKS, 3>(
+                [&](int i, int part) {
+                    return get_row<DP>(Ks, ROWS, 32 * kh + 16 * (i / NKS), dh * DW + 32 * (i % NKS), l16, grp, part);
+                },
+                [&](int i, auto part, u4 x) {
+                    f4 t[NQ];
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n) t[n] = s[(i / NKS) * NQ + n];
+                    mfma_parts<part>(t, x, [&](int n) -> const Tri & { return q[i % NKS][n]; });
+#pragma unroll
+                    for (int n = 0; n < NQ; ++n) s[(i / NKS) * NQ + n] = t[n];
+                });
+            const bool kbig = __builtin_amdgcn_readfirstlane(*kflag(sid)) == sid;
+            if (kbig || qbig) {
+                // Products with a big operand, from the full values.
+                if (kbig && qbig) {  // both sides: the whole product in f32
+#pragma unroll
+                    for (int i = 0; i < 2 * NQ; ++i) s[i] = zero4();
+                }
+                const int ll = opaque(lane), lrow = ll & 15, lgrp = ll >> 4;
+#pragma unroll 1
+                for (int cc = 0; cc < 8 * NKS; ++cc) {
+                        const int c = dh * DW + 32 * (cc >> 3) + 8 * lgrp + (cc & 7);
+                        float kv[2], qv[NQ];
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) {
+                            const int key = min(k0 + 16 * j + lrow, a.n_keys - 1);
+                            kv[j] = c < a.dim ? kb[(size_t)key * kld + c] : 0.f;
+                            if (!qbig) kv[j] = big_part(kv[j]);
+                        }
+#pragma unroll
+                        for (int n = 0; n < NQ; ++n) {
+                            const int row = row0 + 16 * n + lrow;
+                            qv[n] = row < a.T && c < a.dim ? qb[(size_t)row * qld + c] * qscale : 0.f;
+                            if (!kbig) qv[n] = big_part(qv[n]);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 2 * NQ; ++i) s[i] = mfma16(kv[i / NQ], qv[i % NQ], s[i]);
+                    }
+            }
+            if constexpr (DS == 1) {
+                softmax(k0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 2 * NQ; ++i)
+                    *reinterpret_cast<f4 *>(xchg + ((w * 2 * NQ + i) * 64 + lane) * 16) = s[i];
+            }
+        }
+        if constexpr (ALT) {
+            stage_k(sid + 1);
+            if constexpr (DEEP) fetch(px, kb, kn2);
+        } else {
+            stage_v(sid);
+            if constexpr (DEEP) fetch(py, vb, kn);
+        }
+        __syncthreads();
+
+        // Phase B: softmax and the output product; the next K (ALT: V) into LDS.
+        if constexpr (!DEEP) fetch(px, ALT ? vb : kb, kn);
+        if (active) {
+            if constexpr (DS > 1) {  // f32 addition commutes: both halves get the same scores
+                const int other = w ^ NWR;
+#pragma unroll
+                for (int i = 0; i < 2 * NQ; ++i)
+                    s[i] += *reinterpret_cast<const f4 *>(xchg + ((other * 2 * NQ + i) * 64 + lane) * 16);
+            }
+            if constexpr (DS > 1) softmax(k0);
+            Tri p[NQ];
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+                float y[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = s[(i / 4) * NQ + n][i % 4];
+                p[n] = split8(y);
+            }
+            f4 t[NQ];
+            stream_parts<NT, 3>(
+                [&](int i, int part) { return get_col<DP>(Vs, ROWS, 32 * kh, dh * DW + 16 * i, lane, part); },
+                [&](int i, auto part, u4 x) {
+                    if constexpr (part == 0) {
+#pragma unroll
+                        for (int n = 0; n < NQ; ++n) t[n] = zero4();
+                    }
+                    mfma_parts<part>(t, x, [&](int n) -> const Tri & { return p[n]; });
+                    if constexpr (part == 2) {
+#pragma unroll
+                        for (int n = 0; n < NQ; ++n) o[i][n] += t[n];
+                    }
+                });
+            if (__builtin_amdgcn_readfirstlane(*vflag(sid)) == sid) {
+                // V's big values, from the full rows (P is at most 2^8, or NaN).
+                const int ll = opaque(lane), lcol = ll & 15, lgrp = ll >> 4;
+#pragma unroll 1
+                for (int jr = 0; jr < 8; ++jr) {
+                        const int key = min(k0 + 16 * (jr >> 2) + 4 * lgrp + (jr & 3), a.n_keys - 1);
+                        float pv[NQ];
+#pragma unroll
+                        for (int n = 0; n < NQ; ++n) {
+                            unsigned ph = p[n].h.x, pm = p[n].m.x, pl = p[n].l.x;
+#pragma unroll
+                            for (int e = 1; e < 4; ++e) {
+                                ph = jr >> 1 == e ? p[n].h[e] : ph;
+                                pm = jr >> 1 == e ? p[n].m[e] : pm;
+                                pl = jr >> 1 == e ? p[n].l[e] : pl;
+                            }
+                            pv[n] = join_bf16(ph, pm, pl, jr & 1);
+                        }
+#pragma unroll
+                        for (int i = 0; i < NT; ++i) {
+                            const int c = dh * DW + 16 * i + lcol;
+                            const float vv = c < a.dim ? big_part(vb[(size_t)key * kld + c]) : 0.f;
+#pragma unroll
+                            for (int n = 0; n < NQ; ++n) o[i][n] = mfma16(vv, pv[n], o[i][n]);
+                        }
+                    }
+            }
+        }
+        if constexpr (ALT) {
+            stage_v(sid + 1);
+            if constexpr (DEEP) fetch(py, vb, kn2);
+        } else {
+            stage_k(sid + 1);
+            if constexpr (DEEP) fetch(px, kb, kn2);
+        }
+        __syncthreads();
+    }
+    if (ALT && w < NW / 2) __syncthreads();
+    ++sid;  // the last step staged tiles for the step that does not follow
+
+    if constexpr (KS > 1) {
+        // Merge the key parts, as in attn_fwd_tile.  (The loop ended with a barrier.)
+        constexpr int SF = 4 * NQ * NT + 2 * NQ;
+        auto slot = [&](int part) {
+            return reinterpret_cast<float *>(smem) + (((part - 1) * (NW / KS) + (w % (NW / KS))) * SF) * 64 + lane * 4;
+        };
+        if (kh > 0) {
+            float *mb = slot(kh);
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) *reinterpret_cast<f4 *>(mb + (i * NQ + n) * 256) = o[i][n];
+            float *ml = mb + 4 * NQ * NT * 64 - lane * 4 + lane;
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) { ml[(2 * n) * 64] = m[n]; ml[(2 * n + 1) * 64] = lsum[n]; }
+        }
+        __syncthreads();
+        if (kh == 0) {
+#pragma unroll
+            for (int part = 1; part < KS; ++part) {
+                const float *mb = slot(part);
+                const float *ml = mb + 4 * NQ * NT * 64 - lane * 4 + lane;
+#pragma unroll
+                for (int n = 0; n < NQ; ++n) {
+                    const float m2 = ml[(2 * n) * 64], l2 = ml[(2 * n + 1) * 64];
+                    const float mm = fmaxf(m[n], m2);
+                    const float f1 = ZT_PLANT == 3 ? 1.f : m[n] == -INFINITY ? 0.f : fast_exp2(m[n] - mm);
+                    const float f2 = ZT_PLANT == 3 ? 1.f : m2 == -INFINITY ? 0.f : fast_exp2(m2 - mm);
+                    lsum[n] = lsum[n] * f1 + l2 * f2;
+#pragma unroll
+                    for (int i = 0; i < NT; ++i)
+                        o[i][n] = o[i][n] * f1 + *reinterpret_cast<const f4 *>(mb + (i * NQ + n) * 256) * f2;
+                    m[n] = mm;
+                }
+            }
+        }
+        __syncthreads();  // the merge's reads before the next tile's staging
+        if (kh != 0) return;
+    }
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+        const int el = opaque(lane), egrp = el >> 4;
+        const int row = row0 + 16 * n + (el & 15);
+        const float l = sum4grp(lsum[n]);
+        const float inv = 1.f / l;
+        if (row >= a.T) continue;
+        if (a.lse && egrp == 0 && dh == 0)  // natural log: (m + log2 l) ln 2
+            a.lse[((size_t)b * a.T + row) * a.H + h] = (m[n] + log2f(l)) * 0.69314718055994531f;
+        float *orow = a.out + (size_t)b * a.T * qld + (size_t)row * qld + (size_t)h * a.dim;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int c = dh * DW + 16 * i + 4 * egrp;
+            if (c < a.dim) *reinterpret_cast<f4 *>(orow + c) = o[i][n] * inv;
+        }
+    }
+}
+
+template <int DP, int DS, int NW, int NQ, int KS, int SC>
+DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
+    const int p = (int)blockIdx.x / (a.n_head_blocks * a.B);
+    using C = FwdSplit<DP, DS, NW, NQ, KS>;
+    if (threadIdx.x < 4) reinterpret_cast<int *>(smem + C::FLAGS)[threadIdx.x] = 0;
+    __syncthreads();
+    int sid = 0;
+    // One copy of the tile's code (two cost registers: 43 against 11 spilled at d = 128).
+    const int second = a.n_row_tiles - 1 - p;
+    int tile = second;
+#pragma unroll 1
+    for (;;) {  // workgroup-uniform (every tile ends after a barrier)
+        fwd_split_tile<DP, DS, NW, NQ, KS, SC>(a, tile, smem, sid);
+        if (!a.pair || tile == p || p >= second) break;
+        tile = p;
+    }
+}
 #define ZT_FWD(DP, BK)                                                                             \
     extern "C" __global__ void __launch_bounds__(256) zt_fwd_d##DP##_k##BK(FwdArgs a) {          \
         attn_fwd_body<DP, BK, 4, false>(a);                                                        \
@@ -308,29 +802,51 @@ __device__ __forceinline__ void attn_fwd_body(const FwdArgs &a) {
     extern "C" __global__ void __launch_bounds__(512) zt_fwd8_d##DP##_k##BK(FwdArgs a) {         \
         attn_fwd_body<DP, BK, 8, false>(a);                                                        \
     }
-// Register-prefetched variants (32-key tiles).
+// Kernels on split operands: one per role and width, each holding the wave
+// shapes (NQ, KS) the launcher picks from by the grid (FwdArgs::nq, ks).
+template <int DP, int DS, int NW, int NQ, int KS, int SC>
+struct FwdShape {
+    static constexpr int BYTES = FwdSplit<DP, DS, NW, NQ, KS>::BYTES;
+    DEVI static bool run(const FwdArgs &a, char *smem) {
+        if (a.nq != NQ || a.ks != KS || blockDim.x != 64 * NW) return false;  // workgroup-uniform
+        fwd_split_body<DP, DS, NW, NQ, KS, SC>(a, smem);
+        return true;
+    }
+};
+template <class... S>
+constexpr int fwd_shapes_bytes() {
+    int m = 0;
+    ((m = S::BYTES > m ? S::BYTES : m), ...);
+    return m;
+}
+template <class... S>
+DEVI void fwd_shapes(const FwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[fwd_shapes_bytes<S...>()];
+    (void)(S::run(a, smem) || ...);
+}
+// SC: 0 never keeps the scores, 1 always, 2 where s_out is set.
+// Roles: several heads of a kv group per workgroup; the same keeping the scores
+// (its own name, so that a profile tells the two apart); one head per workgroup
+// (also four waves, where forced); one head per workgroup on small grids.
+#define ZT_FWD_P8(NAME, DP, ...)                                                                     \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME##_d##DP##_k32(FwdArgs a) {          \
+        fwd_shapes<__VA_ARGS__>(a);                                                                  \
+    }
+#define SH(...) FwdShape<__VA_ARGS__>
+#define ZT_FWD_SPLIT_8(NAME, SC)                                                                         \
+    ZT_FWD_P8(NAME, 32, SH(32, 1, 8, 2, 1, SC), SH(32, 1, 8, 2, 2, SC), SH(32, 1, 8, 1, 2, SC), SH(32, 1, 8, 1, 4, SC))                  \
+    ZT_FWD_P8(NAME, 64, SH(64, 1, 8, 2, 1, SC), SH(64, 1, 8, 2, 2, SC), SH(64, 1, 8, 1, 2, SC))                                      \
+    ZT_FWD_P8(NAME, 96, SH(96, 1, 8, 2, 1, SC), SH(96, 1, 8, 1, 2, SC))                                      \
+    ZT_FWD_P8(NAME, 128, SH(128, 1, 8, 2, 1, SC), SH(128, 1, 8, 1, 2, SC))
+
+// Register-prefetched variants on f32 MFMA (32-key tiles; widths whose halves
+// are not whole 32-column groups).
 #define ZT_FWD_PF(DP)                                                                              \
     extern "C" __global__ void __launch_bounds__(256) zt_fwdp_d##DP##_k32(FwdArgs a) {           \
         attn_fwd_body<DP, 32, 4, true>(a);                                                         \
     }                                                                                              \
     extern "C" __global__ void __launch_bounds__(512, (DP) <= 128 ? 4 : 1) zt_fwd8p_d##DP##_k32(FwdArgs a) { \
         attn_fwd_body<DP, 32, 8, true>(a);                                                         \
-    }
-
-// The same eight-wave kernel under its own name for launches that keep the
-// scores (s_out set), so that a profile tells the two roles apart.
-#define ZT_FWD_PFS(DP)                                                                             \
-    extern "C" __global__ void __launch_bounds__(512, 4) zt_fwd8ps_d##DP##_k32(FwdArgs a) {      \
-        attn_fwd_body<DP, 32, 8, true>(a);                                                         \
-    }
-
-// The key-split variant for heads that share no kv group with another (HW =
-// 1) on small grids: eight waves, 4 row blocks x 2 key parts.  (Four key parts
-// in sixteen waves measured no better: C2's forward 51.3 us against 54.1 us,
-// one 16-head sequence of 2048 rows at d = 64 85.5 against 86.7 us.)
-#define ZT_FWD_PFK(DP)                                                                             \
-    extern "C" __global__ void __launch_bounds__(512) zt_fwdpk_d##DP##_k32(FwdArgs a) {          \
-        attn_fwd_body<DP, 32, 8, true, 2>(a);                                                      \
     }
 
 #if ZT_PLANT == 0
@@ -342,12 +858,25 @@ ZT_FWD(160, 32) ZT_FWD(160, 64)
 ZT_FWD(192, 32) ZT_FWD(192, 64)
 ZT_FWD(224, 32) ZT_FWD(224, 64)
 ZT_FWD(256, 32) ZT_FWD(256, 64)
-ZT_FWD_PF(32) ZT_FWD_PF(64) ZT_FWD_PF(96) ZT_FWD_PF(128)
-ZT_FWD_PF(160) ZT_FWD_PF(192) ZT_FWD_PF(224) ZT_FWD_PF(256)
-ZT_FWD_PFS(32) ZT_FWD_PFS(64) ZT_FWD_PFS(96) ZT_FWD_PFS(128)
-ZT_FWD_PFK(32) ZT_FWD_PFK(64) ZT_FWD_PFK(96) ZT_FWD_PFK(128)
+ZT_FWD_PF(160) ZT_FWD_PF(224)
+ZT_FWD_SPLIT_8(zt_fwd8p, 0)
+ZT_FWD_SPLIT_8(zt_fwd8ps, 1)
+ZT_FWD_P8(zt_fwd8p, 192, SH(192, 2, 8, 2, 1, 2), SH(192, 2, 8, 1, 1, 2))
+ZT_FWD_P8(zt_fwd8p, 256, SH(256, 2, 8, 2, 1, 2), SH(256, 2, 8, 1, 1, 2))
+ZT_FWD_P8(zt_fwdp, 32, SH(32, 1, 8, 2, 1, 2), SH(32, 1, 8, 2, 2, 2), SH(32, 1, 8, 1, 2, 2), SH(32, 1, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdp, 64, SH(64, 1, 8, 2, 1, 2), SH(64, 1, 8, 2, 2, 2), SH(64, 1, 8, 1, 2, 2), SH(64, 1, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdp, 96, SH(96, 1, 8, 2, 1, 2), SH(96, 1, 8, 1, 2, 2), SH(96, 1, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdp, 128, SH(128, 1, 8, 2, 1, 2), SH(128, 1, 8, 1, 2, 2), SH(128, 1, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdp, 192, SH(192, 2, 8, 2, 1, 2), SH(192, 2, 8, 1, 1, 2), SH(192, 2, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdp, 256, SH(256, 2, 8, 2, 1, 2), SH(256, 2, 8, 1, 1, 2), SH(256, 2, 4, 2, 1, 2))
+ZT_FWD_P8(zt_fwdpk, 32, SH(32, 1, 8, 1, 2, 2), SH(32, 1, 8, 1, 4, 2))
+ZT_FWD_P8(zt_fwdpk, 64, SH(64, 1, 8, 1, 2, 2), SH(64, 1, 8, 1, 4, 2))
+ZT_FWD_P8(zt_fwdpk, 96, SH(96, 1, 8, 1, 2, 2))
+ZT_FWD_P8(zt_fwdpk, 128, SH(128, 1, 8, 1, 2, 2))
 #else
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
-ZT_FWD_PF(32) ZT_FWD_PF(128) ZT_FWD_PFS(128)
+ZT_FWD_P8(zt_fwd8p, 32, SH(32, 1, 8, 2, 1, 0), SH(32, 1, 8, 1, 2, 0), SH(32, 1, 8, 1, 4, 0))
+ZT_FWD_P8(zt_fwd8p, 128, SH(128, 1, 8, 2, 1, 0), SH(128, 1, 8, 1, 2, 0))
+ZT_FWD_P8(zt_fwd8ps, 128, SH(128, 1, 8, 2, 1, 1), SH(128, 1, 8, 1, 2, 1))
 #endif

@@ -166,7 +166,7 @@ int launch(DeviceState *st, const char *name, unsigned blocks, const Args &args,
 enum Tune {
     kTuneBK, kTuneFwdW, kTuneFPF, kTuneFPair, kTuneQPF, kTuneDqW, kTuneHS, kTuneW8, kTunePF, kTuneDMA, kTuneBPair,
     kTuneDSplit, kTuneRSplit, kTuneDecWgs, kTuneGemmTile, kTuneGemmSk, kTuneGemmSkTile, kTuneDqdsTile, kTuneRowG,
-    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneCount
+    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneFShape, kTuneCount
 };
 struct TuneSpec {
     const char *name;
@@ -197,6 +197,7 @@ const TuneSpec kTuneSpecs[kTuneCount] = {
     {"ZT_ATTN_FKS", {1, 2}, 2},
     {"ZT_DQDS_K", {1, 2}, 2},
     {"ZT_ATTN_RSCORES", {0, 1}, 2},
+    {"ZT_ATTN_FSHAPE", {11, 12, 14, 21, 22}, 5},
 };
 std::atomic<int> g_tune[kTuneCount] = {};  // 0 = unset (no allowed value is 0 except a flag, stored as value + 1)
 
@@ -235,21 +236,18 @@ size_t kv_tile_bytes(int dp, int bk) { return (size_t)2 * bk * (dp + 4) * sizeof
 // it loses for MHA (C2 0.057 -> 0.076 ms); the dq kernel loses at every shape tried.
 int fwd_waves(int hw) { return tuned(kTuneFwdW, hw >= 2 ? 8 : 4); }
 
-// Forward kernel name: waves per workgroup, key tile, and for 32-key tiles the
-// register-prefetched variant (ZT_ATTN_FPF=0 turns it off).  Measured on
-// MI355X: eight waves, C3 1.315 -> 1.225 ms and C5 0.758 -> 0.630 ms; four
-// waves (MHA and head groups of two), C2 0.074 -> 0.057 ms and one 16-head
-// sequence of 2048 rows at d = 128 0.30 -> 0.185 ms.
-void fwd_kernel_name(char *name, size_t len, int dim, int dp, int bk, int nw, int ks = 1) {
-    // The prefetching kernels load 16-byte row chunks unconditionally (dim % 4 == 0).
-    const bool pf = bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1;
-    if (pf && ks > 1)
-        snprintf(name, len, "zt_fwdpk_d%d_k32", dp);
-    else if (pf)
-        snprintf(name, len, nw == 8 ? "zt_fwd8p_d%d_k32" : "zt_fwdp_d%d_k32", dp);
-    else
-        snprintf(name, len, nw == 8 ? "zt_fwd8_d%d_k%d" : "zt_fwd_d%d_k%d", dp, bk);
-}
+// The forward's kernel and the work of its waves.  nw waves per workgroup,
+// hw query heads of one kv group among them; on split operands (split) also nq
+// 16-row blocks per wave, ks key parts and ds column halves.
+struct FwdPlan {
+    bool split, small;  // small: one head per workgroup on a small grid (fwd_key_split)
+    int nw, hw, nq, ks, ds;
+};
+int fwd_rows(const FwdPlan &p) { return 16 * p.nq * (p.nw / (p.ks * p.ds * p.hw)); }
+
+// Widths the split-operand forward is built for (a wave's columns are whole
+// 32-column groups); it loads whole 16-byte row chunks (dim % 4 == 0).
+bool fwd_split_width(int dp) { return dp <= 128 || dp == 192 || dp == 256; }
 
 // Key parts of the forward: 1, or 2 for the key-split kernel (zt_fwdpk_*:
 // eight waves, 4 row blocks x 2 key parts merged at the end) for one query
@@ -265,6 +263,80 @@ int fwd_key_split(int B, int T, int n_heads, int hw, int dp, int dim, int bk, in
     const long long wgs = (tiles + 1) / 2 * (long long)n_heads * B;  // paired
     return able ? tuned(kTuneFKS, wgs <= cus ? 2 : 1) : 1;
 }
+
+// Whether the kernel fwd_kernel_name names for p holds the wave shape p (the
+// lists in kernels/attn_fwd.hip).
+bool fwd_shape_built(const FwdPlan &p, int dp) {
+    if (p.nw == 4) return p.nq == 2 && p.ks == 1;
+    if (p.ds == 2) return p.ks == 1;
+    if (p.small) return p.nq == 1 && (p.ks == 2 || (p.ks == 4 && dp <= 64));
+    return (p.nq == 2 && p.ks == 1) || (p.nq == 1 && p.ks == 2) || (p.nq == 2 && p.ks == 2 && dp <= 64) ||
+           (p.nq == 1 && p.ks == 4 && dp == 32 && p.hw >= 2);
+}
+
+// Wave shapes on split operands, by how many workgroups the widest shape (two
+// row blocks per wave, one key part) gives: past one per CU it shares each K/V
+// operand read between most rows; below that, waves that each hold one row
+// block and split the keys leave fewer rows, so more workgroups, and shorter
+// key loops.  Measured on MI355X (us, widest / chosen): 32 over 8 heads at d =
+// 128, T = 512 79 / 36, T = 1024 145 / 72, 333 rows at 2007 316 / 132, T = 2048
+// 285 / 235, T = 4096 610 / 860 (kept); 4 over 2 heads at d = 32, T = 256
+// 20 / 9.2 (two key parts 11), T = 4096 237 / 64; MHA at d = 64, 4 x 1024 rows x 8
+// heads 56 (two row blocks, two key parts) / 47, one sequence of 512 rows
+// 30 / 16 (four key parts).  Up to d = 64 grids of half to one workgroup per CU
+// keep both row blocks and split the keys: 8 x 2048 rows of 4 over 2 heads at d
+// = 32 125 / 86 (one row block 111), 8 x 1024 of 8 MHA heads at d = 64 85 / 66 (84).
+FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int bk, int cus) {
+    FwdPlan p{};
+    p.hw = heads_per_wg(n_heads / n_kv_heads);
+    const int ks = fwd_key_split(B, T, n_heads, p.hw, dp, dim, bk, cus);
+    p.small = ks > 1;
+    p.nw = ks > 1 ? 8 : fwd_waves(p.hw);
+    p.nq = 1; p.ks = ks; p.ds = 1;
+    p.split = bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1 && fwd_split_width(dp);
+    if (!p.split) return p;
+    p.nw = tuned(kTuneFwdW, 8);  // (C2 at four waves, two workgroups per CU: 77 us against 47)
+    p.small = p.small && p.nw == 8;
+    p.ds = dp > 128 ? 2 : 1;
+    p.nq = 2; p.ks = 1;
+    while (p.nw / p.ds < p.hw) p.hw /= 2;  // (four waves forced, two column halves)
+    const long long wide = (long long)((T + fwd_rows(p) - 1) / fwd_rows(p)) * (n_heads / p.hw) * B;
+    if (p.small) {  // one head per workgroup, keys split
+        const long long rows32 = (long long)((T + 31) / 32) * n_heads * B;
+        p.nq = 1;
+        p.ks = dp <= 64 && rows32 <= cus ? 4 : 2;
+    } else if (p.nw == 8 && wide <= cus) {
+        p.nq = 1;
+        p.ks = p.ds > 1 ? 1 : 2;
+        if (dp <= 64 && 2 * wide > cus) p.nq = 2;
+        if (p.hw == 2 && dp == 32 && (long long)((T + 15) / 16) * (n_heads / p.hw) * B <= 2 * cus) p.ks = 4;
+    }
+    const int shape = tuned(kTuneFShape, 10 * p.nq + p.ks);
+    p.nq = shape / 10;
+    p.ks = shape % 10;
+    if (!fwd_shape_built(p, dp)) {  // a forced shape the kernel does not hold
+        p.nq = p.small ? 1 : 2;
+        p.ks = p.small ? 2 : 1;
+    }
+    while (p.nw / (p.ks * p.ds) < p.hw) p.hw /= 2;
+    return p;
+}
+
+// Forward kernel name: the split-operand kernels, and the f32 MFMA kernels for
+// other widths (32-key tiles with the register prefetch) and rows that are not
+// whole 16-byte chunks or a forced 64-key tile (without).
+void fwd_kernel_name(char *name, size_t len, int dim, int dp, int bk, const FwdPlan &p, bool scores) {
+    const bool pf = bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1;
+    if (p.split && p.nw == 8 && p.hw == 1)
+        snprintf(name, len, p.small ? "zt_fwdpk_d%d_k32" : "zt_fwdp_d%d_k32", dp);
+    else if (pf && p.nw == 8)  // keeping scores: the same kernel, named for its role
+        snprintf(name, len, scores && dp <= 128 ? "zt_fwd8ps_d%d_k32" : "zt_fwd8p_d%d_k32", dp);
+    else if (pf)
+        snprintf(name, len, "zt_fwdp_d%d_k32", dp);
+    else
+        snprintf(name, len, p.nw == 8 ? "zt_fwd8_d%d_k%d" : "zt_fwd_d%d_k%d", dp, bk);
+}
+
 int dq_waves(int dp) {
     const int w = tuned(kTuneDqW, 4);
     return dp > 192 ? 4 : w;  // eight-wave dq spills above d = 192
@@ -473,10 +545,9 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     a.q = q; a.k = k; a.v = v; a.out = out; a.lse = lse; a.s_out = s_out;
     a.B = B; a.T = T; a.H = n_heads; a.Hkv = n_kv_heads; a.dim = dim;
     a.q_offset = q_offset; a.n_keys = n_keys; a.kv_rows = kv_rows;
-    a.HW = heads_per_wg(n_heads / n_kv_heads);
-    const int ks = fwd_key_split(B, T, n_heads, a.HW, dp, dim, bk, st->cus);
-    const int nw = ks > 1 ? 8 : fwd_waves(a.HW);
-    const int rows_per_wg = 16 * (nw / ks / a.HW);
+    const FwdPlan p = fwd_plan(B, T, n_heads, n_kv_heads, dp, dim, bk, st->cus);
+    a.HW = p.hw; a.nq = p.nq; a.ks = p.ks;
+    const int rows_per_wg = fwd_rows(p);
     a.n_row_tiles = (T + rows_per_wg - 1) / rows_per_wg;
     a.n_head_blocks = n_heads / a.HW;
     a.scale_log2e = (float)(1.4426950408889634 / std::sqrt((double)dim));
@@ -487,12 +558,10 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     a.pair = tuned(kTuneFPair, pair_pays((unsigned long long)a.n_row_tiles * a.n_head_blocks * B, st->cus));
     const unsigned long long blocks =
         (unsigned long long)(a.pair ? (a.n_row_tiles + 1) / 2 : a.n_row_tiles) * a.n_head_blocks * B;
-    if (!grid_ok(blocks, 64u * nw)) return 1;
+    if (!grid_ok(blocks, 64u * p.nw)) return 1;
     char name[64];
-    fwd_kernel_name(name, sizeof name, dim, dp, bk, nw, ks);
-    if (s_out && dp <= 128 && strncmp(name, "zt_fwd8p_d", 10) == 0)
-        snprintf(name, sizeof name, "zt_fwd8ps_d%d_k32", dp);  // same kernel, named for its role
-    return launch(st, name, (unsigned)blocks, a, stream, 64u * nw);
+    fwd_kernel_name(name, sizeof name, dim, dp, bk, p, s_out != nullptr);
+    return launch(st, name, (unsigned)blocks, a, stream, 64u * p.nw);
 }
 
 // Validates a backward call and fills the argument block and kernel names.
@@ -1379,8 +1448,7 @@ int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_til
         int G = 0, nw = 0;
         one_row_plan(st, B, n_heads, n_kv_heads, dim, &G, &nw, fwd, len);
     } else {
-        const int hw = heads_per_wg(n_heads / n_kv_heads);
-        fwd_kernel_name(fwd, len, dim, dp, bk, fwd_waves(hw), fwd_key_split(B, T, n_heads, hw, dp, dim, bk, st->cus));
+        fwd_kernel_name(fwd, len, dim, dp, bk, fwd_plan(B, T, n_heads, n_kv_heads, dp, dim, bk, st->cus), false);
     }
     BwdArgs a;
     DeviceState *st2 = nullptr;
@@ -1403,9 +1471,9 @@ int zt_attn_plan_train(int B, int T, int n_heads, int n_kv_heads, int dim, char 
     DeviceState *st = device_state();
     if (!st) return 1;
     if (T == 1) {  // the training forward keeps lse, so one row still takes the forward kernel
-        const int hw = heads_per_wg(n_heads / n_kv_heads), dp = pad32(dim);
+        const int dp = pad32(dim);
         const int bk = key_tile(Tiled::Forward, dp, 64, dim);
-        fwd_kernel_name(fwd, len, dim, dp, bk, fwd_waves(hw), fwd_key_split(B, T, n_heads, hw, dp, dim, bk, st->cus));
+        fwd_kernel_name(fwd, len, dim, dp, bk, fwd_plan(B, T, n_heads, n_kv_heads, dp, dim, bk, st->cus), false);
     }
     const int bt = dqds_tile(B, T, n_heads, dim, st->cus);
     dqds_name(dq, len, bt, dqds_parts(B, T, n_heads, dim, bt, dim % 4 == 0, st->cus));
