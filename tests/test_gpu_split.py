@@ -16,6 +16,58 @@ from npref import attention_f64
 
 pytestmark = pytest.mark.gpu
 
+
+def _product(gpu, zt, op, a, b):
+    """a @ b through zt_matmul ("nn"), zt_weight_grad ("tn": a stored K x M) or zt_input_grad ("nt": b stored N x K)."""
+    (M, K), N = a.shape, b.shape[1]
+    out = gpu.zeros(M * N, device="cuda")
+    aa = (a.t() if op == "tn" else a).contiguous().view(-1)
+    bb = (b.t() if op == "nt" else b).contiguous().view(-1)
+    if op == "nn":
+        zt.matmul(aa, bb, out, M, K, N)
+    elif op == "tn":
+        zt.weight_grad(out, aa, bb, K, M, N)
+    else:
+        zt.input_grad(out, aa, bb, M, K, N)
+    gpu.cuda.synchronize()
+    return out.view(M, N)
+
+
+@pytest.mark.parametrize("op", ["nn", "tn", "nt"])
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("M,K,N", [(128, 32, 128), (256, 96, 128), (129, 33, 127), (1, 65, 130), (200, 257, 68)])
+def test_split_products(gpu, zt, tune, op, tile, M, K, N):
+    """Whole tiles and every kind of remainder.  Per element the six products
+    drop at most 2^-23 of a product and K / 32 + 32 roundings of 2^-24 follow:
+    (2 + K / 32 + 32) 2^-24 of the sum of the products' magnitudes."""
+    tune({"ZT_GEMM_TILE": tile})
+    gen = gpu.Generator(device="cuda").manual_seed(M * 1009 + K)
+    a, b = (gpu.randn(s, device="cuda", generator=gen) for s in ((M, K), (K, N)))
+    want = a.double().cpu() @ b.double().cpu()
+    bound = (a.double().abs().cpu() @ b.double().abs().cpu()) * ((34 + K / 32) * 2.0 ** -24)
+    assert gpu.all((_product(gpu, zt, op, a, b).double().cpu() - want).abs() <= bound)
+
+
+@pytest.mark.parametrize("op", ["nn", "tn", "nt"])
+@pytest.mark.parametrize("which", ["a", "b", "ab"])
+def test_split_products_with_infinities(gpu, zt, tune, op, which):
+    """An infinity in A, B or both gives what f32 arithmetic gives: the same
+    infinities and NaN as float64, and the rest unchanged."""
+    tune({"ZT_GEMM_TILE": 128})
+    M, K, N = 150, 70, 140
+    gen = gpu.Generator(device="cuda").manual_seed(5)
+    a, b = (gpu.randn(s, device="cuda", generator=gen) for s in ((M, K), (K, N)))
+    if "a" in which:
+        a[7, 40] = float("inf")
+        a[140, 2] = -2.0 ** 80
+    if "b" in which:
+        b[41, 133] = float("-inf")
+    want = (a.double().cpu() @ b.double().cpu())
+    got = _product(gpu, zt, op, a, b).double().cpu()
+    fin = gpu.isfinite(want)
+    assert gpu.equal(gpu.isnan(got), gpu.isnan(want)) and gpu.equal(got[~fin & ~gpu.isnan(want)], want[~fin & ~gpu.isnan(want)])
+    assert gpu.all((got[fin] - want[fin]).abs() <= 1e-5 * gpu.clamp(want[fin].abs(), min=1.0))
+
 TOL = 2e-5
 
 

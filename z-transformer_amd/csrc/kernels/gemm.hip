@@ -25,6 +25,7 @@
 // f32 sum only in rounding order.
 #include "common.h"
 #include "args.h"
+#include "split.h"
 
 namespace {
 
@@ -237,6 +238,177 @@ DEVI void gemm_body(const GemmArgs &g) {
                       (!A_KC || (unsigned long long)g.M * (unsigned)g.lda < kOff) &&
                       (!B_KC || (unsigned long long)g.N * (unsigned)g.ldb < kOff);
     if (full) gemm_tile<BT, A_KC, B_KC, true>(g);
+    else gemm_tile<BT, A_KC, B_KC, false>(g);
+}
+
+// The 128 and 64 tiles on split operands (split.h): six bf16 MFMAs per 32-deep
+// slab and 16 x 16 tile instead of eight f32 ones of twice their length.  The
+// same workgroups and waves; a slab is split once while it is written to LDS:
+//   * k-contiguous operand: rows of 32 k, read along the row;
+//   * index-contiguous operand: rows of BT indices, read across the rows by the
+//     transposing LDS read, k slot 8 grp + j then being k = 4 grp + j (j < 4) and
+//     16 + 4 grp + j - 4; a k-contiguous partner is read in the same slots, as
+//     two 8-byte halves.
+// A wave keeps its TW B tiles' parts in registers and streams A's; each slab's
+// tile sums are added to the accumulators on the vector ALU, so that K / 32
+// roundings are made at the accumulators' magnitude and not 6 K / 32.  Two
+// workgroups share a CU and cover each other's barriers.  4096^3: 1064 us on f32
+// MFMAs (129 TFLOP/s), 788 us (174 TFLOP/s); bound by power, as the forward.
+template <int BT, bool KC>
+constexpr int slab_bytes() { return KC ? split_bytes<32>(BT) : split_bytes<BT>(32); }
+
+// Part P of the operand of indices c0 .. c0 + 15 of a slab.
+template <int BT, bool KC, bool HALVES>
+DEVI u4 slab_operand(const char *t, int c0, int lane, int part) {
+    const int l16 = lane & 15, grp = lane >> 4;
+    if constexpr (!KC) return get_col<BT>(t, 32, 0, c0, lane, part);
+    else if constexpr (!HALVES) return get_row<32>(t, BT, c0, 0, l16, grp, part);
+    const char *p = t + ((2 - part) * BT + c0 + l16) * split_stride<32>() + 8 * grp;
+    const u2 x = *reinterpret_cast<const u2 *>(p), y = *reinterpret_cast<const u2 *>(p + 32);
+    return u4{x.x, x.y, y.x, y.y};
+}
+
+template <int BT, bool A_KC, bool B_KC, bool FULL>
+DEVI void gemm_split_tile(const GemmArgs &g, char *smem) {
+    constexpr int TW = Tile<BT>::TW, WT = Tile<BT>::WT, NCH = BT / 64;  // 8-float chunks per thread and operand
+    constexpr bool HALVES = A_KC != B_KC;
+    char *const As = smem, *const Bs = smem + slab_bytes<BT, A_KC>();
+    // The slab id (k0 + 1) whose A (B) holds a big value.
+    int *const flags = reinterpret_cast<int *>(Bs + slab_bytes<BT, B_KC>());
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = WT * (w >> 1), wn = WT * (w & 1);
+    const int tiles_n = (g.N + BT - 1) / BT;
+    const int m0 = (int)(blockIdx.x / tiles_n) * BT, n0 = (int)(blockIdx.x % tiles_n) * BT;
+    if (tid < 2) flags[tid] = 0;
+
+    f4 acc[TW][TW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int j = 0; j < TW; ++j) acc[i][j] = zero4();
+
+    f4 pa[NCH][2], pb[NCH][2];
+    auto fetch8 = [&](f4 (&x)[NCH][2], auto kc, const float *base, int ld, int r0, int rmax, int k0, bool vec) {
+        constexpr bool KC = decltype(kc)::value;
+#pragma unroll
+        for (int n = 0; n < NCH; ++n) {
+            const int e = tid + n * NTHR;
+            const int row = KC ? r0 + e / 4 : k0 + e / (BT / 8), col = KC ? k0 + e % 4 * 8 : r0 + e % (BT / 8) * 8;
+            const float *p = base + (size_t)row * ld + col;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (FULL) {
+                    x[n][h] = *reinterpret_cast<const f4 *>(p + 4 * h);
+                } else {
+                    const bool in = KC ? row < rmax : row < g.K;
+                    x[n][h] = in ? load4(p + 4 * h, (KC ? g.K : rmax) - col - 4 * h, vec) : zero4();
+                }
+            }
+        }
+    };
+    auto put8 = [&](const f4 (&x)[NCH][2], auto kc, char *t, int *flag, int id) {
+        constexpr bool KC = decltype(kc)::value;
+#pragma unroll
+        for (int n = 0; n < NCH; ++n) {
+            const int e = tid + n * NTHR;
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = x[n][i / 4][i % 4];
+            if (any_big(max_abs(y))) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+                if (lane == 0) *flag = id;
+            }
+            if constexpr (KC) put_tri<32>(t, BT, e / 4, e % 4 * 8, split8(y));
+            else put_tri<BT>(t, 32, e / (BT / 8), e % (BT / 8) * 8, split8(y));
+        }
+    };
+    using AK = std::integral_constant<bool, A_KC>;
+    using BK_ = std::integral_constant<bool, B_KC>;
+    fetch8(pa, AK{}, g.a, g.lda, m0, g.M, 0, g.vec_a);
+    fetch8(pb, BK_{}, g.b, g.ldb, n0, g.N, 0, g.vec_b);
+#pragma unroll 1
+    for (int k0 = 0; k0 < g.K; k0 += BK) {
+        __syncthreads();
+        put8(pa, AK{}, As, flags, k0 + 1);
+        put8(pb, BK_{}, Bs, flags + 1, k0 + 1);
+        __syncthreads();
+        if (k0 + BK < g.K) {
+            fetch8(pa, AK{}, g.a, g.lda, m0, g.M, k0 + BK, g.vec_a);
+            fetch8(pb, BK_{}, g.b, g.ldb, n0, g.N, k0 + BK, g.vec_b);
+        }
+        const bool abig = __builtin_amdgcn_readfirstlane(flags[0]) == k0 + 1;
+        const bool bbig = __builtin_amdgcn_readfirstlane(flags[1]) == k0 + 1;
+        if (!(abig && bbig)) {
+            Tri b[TW];
+#pragma unroll
+            for (int j = 0; j < TW; ++j) {
+                b[j].l = slab_operand<BT, B_KC, HALVES>(Bs, wn + 16 * j, lane, 0);
+                b[j].m = slab_operand<BT, B_KC, HALVES>(Bs, wn + 16 * j, lane, 1);
+                b[j].h = slab_operand<BT, B_KC, HALVES>(Bs, wn + 16 * j, lane, 2);
+            }
+            f4 t[TW];
+            stream_parts<TW, 3>([&](int i, int part) { return slab_operand<BT, A_KC, HALVES>(As, wm + 16 * i, lane, part); },
+                                [&](int i, auto part, u4 x) {
+                                    if constexpr (part == 0) {
+#pragma unroll
+                                        for (int j = 0; j < TW; ++j) t[j] = zero4();
+                                    }
+                                    mfma_parts<part>(t, x, [&](int j) -> const Tri & { return b[j]; });
+                                    if constexpr (part == 2) {
+#pragma unroll
+                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j];
+                                    }
+                                });
+        }
+        if (abig || bbig) {
+            // Products with a big operand from the full values (both: the whole slab).
+            const int ll = opaque(lane), li = ll & 15, lg = ll >> 4;
+#pragma unroll 1
+            for (int kk = 0; kk < 8; ++kk) {
+                const int k = k0 + 4 * kk + lg;
+                float av[TW], bv[TW];
+#pragma unroll
+                for (int i = 0; i < TW; ++i) {
+                    const int m = m0 + wm + 16 * i + li, n = n0 + wn + 16 * i + li;
+                    av[i] = m < g.M && k < g.K ? g.a[A_KC ? (size_t)m * g.lda + k : (size_t)k * g.lda + m] : 0.f;
+                    bv[i] = n < g.N && k < g.K ? g.b[B_KC ? (size_t)n * g.ldb + k : (size_t)k * g.ldb + n] : 0.f;
+                    if (!bbig) av[i] = big_part(av[i]);
+                    if (!abig) bv[i] = big_part(bv[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < TW; ++i)
+#pragma unroll
+                    for (int j = 0; j < TW; ++j) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + wm + 16 * i + 4 * grp + r;
+            if (!FULL && m >= g.M) continue;
+            float *crow = g.c + (size_t)m * g.ldc + n0 + wn + l16;
+#pragma unroll
+            for (int j = 0; j < TW; ++j) {
+                if (!FULL && n0 + wn + 16 * j + l16 >= g.N) continue;
+                crow[16 * j] = g.accumulate ? crow[16 * j] + acc[i][j][r] : acc[i][j][r];
+            }
+        }
+}
+// The 64-tile takes the split only for whole tiles (2048 x 4096 x 1024: weightGrad
+// 150 -> 134 us, inputGrad 161 -> 128 us; ragged 1000^3 would lose, 42 -> 47 us and 36
+// -> 45 us), and zt_gemm_nn_64 not at all (142 -> 174 us): its staging is shared by
+// half as many products.
+template <int BT, bool A_KC, bool B_KC>
+DEVI void gemm_split_body(const GemmArgs &g) {
+    __shared__ __attribute__((aligned(16))) char smem[slab_bytes<BT, A_KC>() + slab_bytes<BT, B_KC>() + 16];
+    // Workgroup-uniform: every chunk inside its matrix, 16-byte rows.
+    const bool full = g.vec_a && g.vec_b && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0;
+    if (full) gemm_split_tile<BT, A_KC, B_KC, true>(g, smem);
+    else if constexpr (BT == 128) gemm_split_tile<BT, A_KC, B_KC, false>(g, smem);
     else gemm_tile<BT, A_KC, B_KC, false>(g);
 }
 
@@ -533,8 +705,13 @@ DEVI void dq_ds_body(const DqDsArgs &g) {
     extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_##BT(GemmArgs g) { gemm_body<BT, false, false>(g); } \
     extern "C" __global__ void __launch_bounds__(256) zt_gemm_nt_##BT(GemmArgs g) { gemm_body<BT, true, true>(g); }
 
-ZT_GEMM(128)
-ZT_GEMM(64)
+
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nn_128(GemmArgs g) { gemm_split_body<128, true, false>(g); }
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_128(GemmArgs g) { gemm_split_body<128, false, false>(g); }
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_128(GemmArgs g) { gemm_split_body<128, true, true>(g); }
+extern "C" __global__ void __launch_bounds__(256) zt_gemm_nn_64(GemmArgs g) { gemm_body<64, true, false>(g); }
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_64(GemmArgs g) { gemm_split_body<64, false, false>(g); }
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_64(GemmArgs g) { gemm_split_body<64, true, true>(g); }
 ZT_GEMM(32)
 
 // Split-K kernels: zt_gemm_<op>_sk<16 TW>, 64 NW threads (NW = 4, 8 or 16).
