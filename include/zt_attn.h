@@ -338,7 +338,8 @@ int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_til
  *   groups that cannot be halved; 0 = it forms S again and the forward keeps
  *   none), ZT_ATTN_FSHAPE 11|12|14|21|22 (the forward's wave shape on split
  *   operands, 16-row blocks per wave then key parts; one the kernel does not
- *   hold falls back to one it does).
+ *   hold falls back to one it does), ZT_ATTN_BSHAPE 1|2|4 (16-key blocks per
+ *   workgroup of the score-reading dk/dv kernel, head_dim <= 128).
  * Returns 0, or 1 (reason on stderr) for an unknown name or value.  The
  * process environment is never read.  Not synchronised with launches in
  * flight on other threads: set before launching. */

@@ -11,8 +11,8 @@ sqrt(d) before the 1/sqrt(d) scale.  2e-5 covers the sum of both at d = 256.
 import numpy as np
 import pytest
 
-from gpuhelp import SEED_K, SEED_Q, SEED_V, dev_normal, host
-from npref import attention_f64
+from gpuhelp import SEED_DO, SEED_K, SEED_Q, SEED_V, dev_normal, host
+from npref import attention_backward_f64, attention_f64
 
 pytestmark = pytest.mark.gpu
 
@@ -126,3 +126,50 @@ def test_large_finite_operands_take_the_f32_products(gpu, zt, tune, shape, D, wh
     if where == "v":
         keep = [c for c in range(D) if c != 3]
         assert np.array_equal(got[..., keep].view(np.uint32), good[..., keep].view(np.uint32))
+
+
+def _train(gpu, zt, q, k, v, do, T, H, Hkv, D):
+    out, lse = gpu.empty_like(q), gpu.empty(T * H, device="cuda")
+    dq, dk, dv = (gpu.full_like(x, float("nan")) for x in (q, k, v))
+    ws = gpu.full((zt.backward_train_workspace_bytes(1, T, H, Hkv, D) // 4,), float("nan"), device="cuda")
+    zt.forward_train_ws(q, k, v, out, lse, ws, T, H, Hkv, D)
+    zt.backward_train_ws(q, k, v, out, do, lse, dq, dk, dv, ws, T, H, Hkv, D, stage=3 | zt.ZT_WS_SCORES)
+    gpu.cuda.synchronize()
+    return [host(x) for x in (dq, dk, dv)]
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 4])
+@pytest.mark.parametrize("T,H,Hkv,D", [(2, 4, 2, 32), (33, 4, 2, 32), (161, 4, 1, 32), (65, 4, 2, 64), (97, 3, 1, 64),
+                                       (47, 2, 1, 80), (100, 4, 1, 96), (130, 3, 3, 128), (257, 8, 2, 128)])
+def test_every_dkdv_shape(gpu, zt, tune, blocks, T, H, Hkv, D):
+    """The score-reading dk/dv kernel's shapes (groups that halve, MHA, a group
+    of three).  dk and dv sum up to T H / Hkv terms with 32-term f32 steps, each
+    of a difference of two sums of D products: a few 2^-22 of the gradient's
+    scale; 1e-5 of the largest value leaves a factor of ten."""
+    tune({"ZT_ATTN_BSHAPE": blocks})
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    do = dev_normal(gpu, zt, T * H * D, SEED_DO)
+    want = attention_backward_f64(*(host(x) for x in (q, k, v, do)), T, H, Hkv, D)
+    for got, w in zip(_train(gpu, zt, q, k, v, do, T, H, Hkv, D), want):
+        w = np.asarray(w).ravel()
+        assert np.max(np.abs(got - w)) <= 1e-5 * max(1.0, np.abs(w).max())
+
+
+@pytest.mark.parametrize("where", ["q", "do", "v"])
+def test_dkdv_with_large_operands(gpu, zt, where):
+    """Rows of 2^70 in dO (dv and dk of its keys), or in V or Q where the result
+    stays finite: the gradients follow float64, the other kv head keeps its bits."""
+    T, H, Hkv, D, S = 90, 4, 2, 64, 50
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    do = dev_normal(gpu, zt, T * H * D, SEED_DO)
+    good = _train(gpu, zt, q, k, v, do, T, H, Hkv, D)
+    x = {"q": q, "do": do, "v": v}[where].clone()
+    x.view(T, -1, D)[S, -1, 3] = 2.0 ** 70
+    args = {"q": q, "k": k, "v": v, "do": do, where: x}
+    got = _train(gpu, zt, args["q"], args["k"], args["v"], args["do"], T, H, Hkv, D)
+    want = attention_backward_f64(*(host(args[n]) for n in ("q", "k", "v", "do")), T, H, Hkv, D)
+    for g, w, o, heads in zip(got, want, good, (H, Hkv, Hkv)):
+        g, w, o = (np.asarray(y).reshape(T, heads, D) for y in (g, w, o))
+        assert np.all(np.isfinite(g))
+        assert np.max(np.abs(g - w)) <= 1e-5 * np.abs(w).max()
+        assert np.array_equal(g[:, :heads // 2].view(np.uint32), o[:, :heads // 2].astype(np.float32).view(np.uint32))

@@ -52,6 +52,7 @@ struct BwdArgs {
     float *ds_out;
     int B, T, H, Hkv, dim;
     int HW, n_row_tiles, n_head_blocks;  // dq kernel decomposition (as the forward)
+    int parts, kblocks;                  // dk/dv on split operands: parts and 16-key blocks per workgroup
     int HS, n_key_tiles;                 // dk/dv kernel: head split, ceil(T / (16 * 4/HS))
     int pair;                            // both kernels: a workgroup takes tiles p and n - 1 - p
     float scale, scale_log2e;

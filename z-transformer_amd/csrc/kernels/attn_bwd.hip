@@ -25,6 +25,7 @@
 // dv carries no scale, dk carries 1/sqrt(d) (autograd.zig:829-836).
 #include "common.h"
 #include "args.h"
+#include "split.h"
 
 
 // The K and V tiles of the dq kernels: one allocation per (DP, BK), shared by
@@ -1280,6 +1281,375 @@ __device__ __forceinline__ void bwd_dkdv_dma_body(const BwdArgs &a) {
     }
 }
 
+// ---- dk/dv from the forward's scores, on split operands (split.h) ----------
+//
+// The work of the score-reading kernels above -- dP = dO V^T, P = exp2(S - lse),
+// dS = P (dP - delta), dV += P^T dO, dK += dS^T Q, dS written over S -- for
+// widths to 128 on the bf16 matrix cores.  A wave owns 16 keys (V's split in
+// registers, dK and dV accumulators); the workgroup is NKB key blocks x NPART
+// parts, and a part takes every NPART-th of the (head, 32-row block) items of
+// the kv group, rows from the last down.  Each part stages its item's dO and Q
+// once, split, row-major; the products that contract over the head read rows,
+// those that contract over queries read across them (the transposing LDS read),
+// so neither is stored twice.
+//   * Phase A (dP, P, dS, dV: the dO tile) writes this item's Q to LDS, phase B
+//     (dK: the Q tile) the next item's dO: one buffer of each, and the splitting
+//     runs beside the other waves' products.
+//   * dV and dK take 32-row sums by f32 adds.
+//   * The parts' dK and dV are summed through LDS in part order: deterministic.
+// What bounds it: LDS operand reads and their latency (74 KB per wave and item at
+// d = 128, against 144 MFMAs of 16 cycles).  With delta, against the f32 MFMA
+// kernels before it: 32 over 8 heads, d = 128, T = 4096 1661 -> 1517 us, T = 512 214
+// -> 177; 4 over 2 heads, d = 32, T = 4096 277 -> 130, T = 256 23.8 -> 13.9; MHA d = 64,
+// 4 x 1024 rows x 8 heads 88 -> 78 us.
+template <int DP, int NPART, int NKB>
+struct BwdSplit {
+    static constexpr int NW = NPART * NKB, NT = DP / 16, NKS = DP / 32;
+    static constexpr int TILE = split_bytes<DP>(32);
+    static constexpr int STATS = NPART * 2 * TILE;         // lse log2(e), -delta of the 32 rows, per part
+    static constexpr int FLAGS = STATS + NPART * 64 * 4;   // step ids whose dO (Q) tile holds a big value, per part
+    static constexpr int BYTES = FLAGS + NPART * 8;
+    static_assert((NPART - 1) * NKB * 64 * 2 * NT * 16 <= STATS, "the parts merge in the tiles' space");
+    static_assert(BYTES <= 160 * 1024, "LDS");
+};
+
+template <int DP, int NPART, int NKB>
+DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const int b, char *const smem, int &sid) {
+    using C = BwdSplit<DP, NPART, NKB>;
+    constexpr int NT = C::NT, NKS = C::NKS, NTP = 64 * NKB;
+    const int tid = opaque((int)threadIdx.x), lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int part = w / NKB, kb = w % NKB, ptid = tid - part * NTP;
+    char *const dOs = smem + part * 2 * C::TILE, *const Qs = dOs + C::TILE;
+    float *const st_lse = reinterpret_cast<float *>(smem + C::STATS) + part * 64, *const st_del = st_lse + 32;
+    int *const flags = reinterpret_cast<int *>(smem + C::FLAGS) + 2 * part;
+
+    const int group = a.H / a.Hkv;
+    const size_t qld = (size_t)a.H * a.dim, kld = (size_t)a.Hkv * a.dim;
+    const int s0 = kt * 16 * NKB, key0 = s0 + 16 * kb;
+    const int nt = (a.T + 15) >> 4, nb32 = (a.T + 31) >> 5;
+    const int nrb = nb32 - (s0 >> 5);  // 32-row blocks from the one that holds key s0
+    const int items = group * nrb, steps = (items + NPART - 1) / NPART;
+    const int kvr = ZT_PLANT == 12 ? 0 : kvh;
+
+    // V: the B operand of dP, lane l16 = key, k slot = column.
+    Tri v[NKS];
+    float vmx = 0.f;
+    const float *vrow = a.v + ((size_t)b * a.T + min(key0 + l16, a.T - 1)) * kld + (size_t)kvr * a.dim;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+        const int c = 32 * ks + 8 * grp;
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 8; i += 4) {
+            const f4 x = *reinterpret_cast<const f4 *>(vrow + min(c + i, a.dim - 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[i + e] = c + i < a.dim ? x[e] : 0.f;
+        }
+        const float mx = max_abs(y);
+        vmx = vmax(vmx, mx);
+        if (any_big(mx)) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+        }
+        v[ks] = split8(y);
+    }
+    const bool vbig = any_big(vmx);
+
+    f4 dk[NT], dv[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) dk[i] = dv[i] = zero4();
+
+    // This part's item: head `head` of the group, row block r0; a part past the last item is idle.
+    int it = part, head = part / nrb, rem = part % nrb;
+    auto row_block = [&] { return 32 * (nb32 - 1 - rem); };
+
+    constexpr int CPR = DP / 8, CH = 32 * CPR, NP = (CH + NTP - 1) / NTP;
+    f4 px[NP][2];
+    auto fetch = [&](const float *arr, int r0, int hd) {  // in bounds: rows past T load row T - 1 (P = 0 there)
+        const char *p = reinterpret_cast<const char *>(arr + ((size_t)b * a.T + r0) * qld + (size_t)(kvh * group + hd) * a.dim);
+        const unsigned last = (unsigned)min(a.T - 1 - r0, 31) * (unsigned)qld * 4u;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            const int e = ptid + n * NTP, c = e % CPR * 8;
+            if (CH % NTP != 0 && e >= CH) break;  // wave-uniform
+            const unsigned r = min((unsigned)(e / CPR) * (unsigned)qld * 4u, last);
+            px[n][0] = *reinterpret_cast<const f4 *>(p + (r + (unsigned)min(c, a.dim - 4) * 4u));
+            px[n][1] = *reinterpret_cast<const f4 *>(p + (r + (unsigned)min(c + 4, a.dim - 4) * 4u));
+        }
+    };
+    auto put = [&](char *t, int *flag, int id) {
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            const int e = ptid + n * NTP, c = e % CPR * 8;
+            if (CH % NTP != 0 && e >= CH) break;
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = px[n][i / 4][i % 4];
+            if (a.dim < DP) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = c + (i & 4) < a.dim ? y[i] : 0.f;
+            }
+            if (any_big(max_abs(y))) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+                if (lane == 0) *flag = id;
+            }
+            put_tri<DP>(t, 32, e / CPR, c, split8(y));
+        }
+    };
+    // Row statistics: the part's first wave, lane = row (lse), 32 + row (delta).
+    float stat = 0.f;
+    auto fetch_stats = [&](int r0, int hd) {
+        if (kb != 0) return;  // wave-uniform
+        const size_t o = ((size_t)b * a.T + min(r0 + (lane & 31), a.T - 1)) * a.H + kvh * group + hd;
+        stat = lane < 32 ? a.lse[o] * kLog2e : -a.row_del[o];
+    };
+    auto put_stats = [&] {
+        if (kb == 0) st_lse[lane] = stat;
+    };
+    // The item's two score tiles; one above the diagonal or past the rows loads a written one (P = 0 there).
+    f4 s[2];
+    float *tile_base = nullptr;
+    const int sb = min(key0 >> 4, nt - 1);
+    auto fetch_scores = [&](int r0, int hd) {
+        tile_base = a.ds_out + ((size_t)b * a.H + kvh * group + hd) * zt_tri_count(nt) * 256 + lane * 4;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int tb = max(min((r0 >> 4) + j, nt - 1), sb);
+            s[j] = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(tile_base + zt_tri_index(tb, sb) * 256));
+        }
+    };
+
+    if (it < items) {
+        const int r0 = row_block();
+        fetch(a.dout, r0, head);
+        fetch_stats(r0, head);
+        fetch_scores(r0, head);
+        put(dOs, flags, sid + 1);
+        put_stats();
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int st = 0; st < steps; ++st) {
+        ++sid;
+        const int r0 = row_block(), hd = head;
+        const bool live = it < items, active = live && key0 <= min(r0 + 31, a.T - 1);  // wave-uniform
+        const float *const dOg = a.dout + ((size_t)b * a.T) * qld + (size_t)(kvh * group + hd) * a.dim;
+        const float *const Qg = a.q + ((size_t)b * a.T) * qld + (size_t)(kvh * group + hd) * a.dim;
+        // Phase A: dP, P, dS and dV from the dO tile; this item's Q into LDS.
+        if (live) fetch(a.q, r0, hd);
+        f4 ds[2];
+        if (active) {
+            // dP starts at -delta (C layout: rows 16 j + 4 grp + r).
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ds[j] = *reinterpret_cast<const f4 *>(st_del + 16 * j + 4 * grp);
+            const bool dobig = __builtin_amdgcn_readfirstlane(flags[0]) == sid;
+            if (!(dobig && vbig))
+                stream_parts<2 * NKS, 6>(
+                    [&](int i, int prt) { return get_row<DP>(dOs, 32, 16 * (i & 1), 32 * (i >> 1), l16, grp, prt); },
+                    [&](int i, auto prt, u4 x) {
+                        f4 t[1] = {ds[i & 1]};
+                        mfma_parts<prt>(t, x, [&](int) -> const Tri & { return v[i >> 1]; });
+                        ds[i & 1] = t[0];
+                    });
+            if (dobig || vbig) {  // products with a big operand, from the full values
+                const int ol = opaque(lane), li = ol & 15, lg = ol >> 4;
+                const float *vr = a.v + ((size_t)b * a.T + min(key0 + li, a.T - 1)) * kld + (size_t)kvr * a.dim;
+#pragma unroll 1
+                for (int cc = 0; cc < 8 * NKS; ++cc) {
+                    const int c = 32 * (cc >> 3) + 8 * lg + (cc & 7);
+                    float vv = c < a.dim ? vr[c] : 0.f;
+                    if (!dobig) vv = big_part(vv);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        float ov = c < a.dim ? dOg[(size_t)min(r0 + 16 * j + li, a.T - 1) * qld + c] : 0.f;
+                        if (!vbig) ov = big_part(ov);
+                        ds[j] = mfma16(ov, vv, ds[j]);
+                    }
+                }
+            }
+            float p[8];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const f4 ls = *reinterpret_cast<const f4 *>(st_lse + 16 * j + 4 * grp);
+                const int row = r0 + 16 * j + 4 * grp, key = key0 + l16;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool in = (ZT_PLANT == 11 || key <= row + r) && row + r < a.T;
+                    const float e = in ? fast_exp2(s[j][r] - ls[r]) : 0.f;
+                    p[4 * j + r] = e;
+                    ds[j][r] = in ? (ZT_PLANT == 13 ? e : e * ds[j][r]) : 0.f;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int tb = (r0 >> 4) + j;
+                if (tb < nt && sb <= tb && key0 < a.T)  // wave-uniform: the tile has a slot
+                    __builtin_nontemporal_store(ZT_PLANT == 15 ? ds[1 - j] : ds[j],
+                                                reinterpret_cast<f4 *>(tile_base + zt_tri_index(tb, sb) * 256));
+            }
+            const bool pbig = any_big(max_abs(p));
+            float ps[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ps[i] = p[i];
+            if (pbig) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ps[i] = small_part(ps[i]);
+            }
+            const Tri pt = split8(ps);
+            if (!(dobig && pbig)) {
+                f4 t[1];
+                stream_parts<NT, 6>([&](int i, int prt) { return get_col<DP>(dOs, 32, 0, 16 * i, lane, prt); },
+                                    [&](int i, auto prt, u4 x) {
+                                        if constexpr (prt == 0) t[0] = zero4();
+                                        mfma_parts<prt>(t, x, [&](int) -> const Tri & { return pt; });
+                                        if constexpr (prt == 2) dv[i] += t[0];
+                                    });
+            }
+            if (dobig || pbig) {
+                const int ol = opaque(lane), li = ol & 15, lg = ol >> 4;
+#pragma unroll 1
+                for (int jr = 0; jr < 8; ++jr) {
+                    const float *orow = dOg + (size_t)min(r0 + 16 * (jr >> 2) + 4 * lg + (jr & 3), a.T - 1) * qld;
+                    float pv = p[0];
+#pragma unroll
+                    for (int e = 1; e < 8; ++e) pv = jr == e ? p[e] : pv;
+                    if (!dobig) pv = big_part(pv);
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) {
+                        float ov = 16 * i + li < a.dim ? orow[16 * i + li] : 0.f;
+                        if (!pbig) ov = big_part(ov);
+                        dv[i] = mfma16(ov, pv, dv[i]);
+                    }
+                }
+            }
+        }
+        if (live) put(Qs, flags + 1, sid);
+        __syncthreads();
+
+        // Phase B: dK from the Q tile; the next item's dO, statistics and scores on their way.
+        it += NPART;
+        rem += NPART;
+        while (rem >= nrb) { rem -= nrb; ++head; }
+        const bool next = it < items;
+        if (next) {
+            const int rn = row_block();
+            fetch(a.dout, rn, head);
+            fetch_stats(rn, head);
+            fetch_scores(rn, head);
+        }
+        if (active) {
+            float y[8], ys[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = ys[i] = ds[i / 4][i % 4];
+            const bool dsbig = any_big(max_abs(y)), qbig = __builtin_amdgcn_readfirstlane(flags[1]) == sid;
+            if (dsbig) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ys[i] = small_part(ys[i]);
+            }
+            const Tri dt = split8(ys);
+            if (!(dsbig && qbig)) {
+                f4 t[1];
+                stream_parts<NT, 6>([&](int i, int prt) { return get_col<DP>(Qs, 32, 0, 16 * i, lane, prt); },
+                                    [&](int i, auto prt, u4 x) {
+                                        if constexpr (prt == 0) t[0] = zero4();
+                                        mfma_parts<prt>(t, x, [&](int) -> const Tri & { return dt; });
+                                        if constexpr (prt == 2) dk[i] += t[0];
+                                    });
+            }
+            if (dsbig || qbig) {
+                const int ol = opaque(lane), li = ol & 15, lg = ol >> 4;
+#pragma unroll 1
+                for (int jr = 0; jr < 8; ++jr) {
+                    const float *qrow = Qg + (size_t)min(r0 + 16 * (jr >> 2) + 4 * lg + (jr & 3), a.T - 1) * qld;
+                    float dd = y[0];
+#pragma unroll
+                    for (int e = 1; e < 8; ++e) dd = jr == e ? y[e] : dd;
+                    if (!qbig) dd = big_part(dd);
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) {
+                        float qv = 16 * i + li < a.dim ? qrow[16 * i + li] : 0.f;
+                        if (!dsbig) qv = big_part(qv);
+                        dk[i] = mfma16(qv, dd, dk[i]);
+                    }
+                }
+            }
+        }
+        if (next) {
+            put(dOs, flags, sid + 1);
+            put_stats();
+        }
+        __syncthreads();
+    }
+
+    // Sum the parts in part order; part 0 stores.
+    f4 *const red = reinterpret_cast<f4 *>(smem);
+    if (part > 0) {
+        f4 *const mine = red + ((part - 1) * NKB + kb) * 2 * NT * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) { mine[i * 64] = dk[i]; mine[(NT + i) * 64] = dv[i]; }
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll 1
+        for (int q = 0; q < NPART - 1; ++q) {
+            const f4 *const o = red + (q * NKB + kb) * 2 * NT * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) { dk[i] += o[i * 64]; dv[i] += o[(NT + i) * 64]; }
+        }
+        const int el = opaque(lane), key = key0 + (el & 15);
+        if (key < a.T) {
+            const size_t o = ((size_t)b * a.T + key) * kld + (size_t)kvh * a.dim + 4 * (el >> 4);
+            const float scale = ZT_PLANT == 14 ? 1.f : a.scale;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                if (16 * i + 4 * (el >> 4) >= a.dim) continue;
+                *reinterpret_cast<f4 *>(a.dk + o + 16 * i) = dk[i] * scale;
+                *reinterpret_cast<f4 *>(a.dv + o + 16 * i) = dv[i];
+            }
+        }
+    }
+    __syncthreads();  // the merge's reads before the next tile's staging
+}
+
+// Shapes (NPART, NKB) of one kernel, picked by the launch (BwdArgs::parts, kblocks).
+template <int DP, int NPART, int NKB>
+struct BwdShape {
+    static constexpr int BYTES = BwdSplit<DP, NPART, NKB>::BYTES;
+    DEVI static bool run(const BwdArgs &a, char *smem) {
+        if (a.parts != NPART || a.kblocks != NKB) return false;  // workgroup-uniform
+        if (threadIdx.x < 2 * NPART) reinterpret_cast<int *>(smem + BwdSplit<DP, NPART, NKB>::FLAGS)[threadIdx.x] = 0;
+        __syncthreads();
+        const int per = a.Hkv * a.B, rem = (int)blockIdx.x % per, p = (int)blockIdx.x / per;
+        const int kvh = rem % a.Hkv, b = rem / a.Hkv;
+        int sid = 0, kt = p;
+        const int second = a.n_key_tiles - 1 - p;
+#pragma unroll 1
+        for (;;) {
+            dkdv_split_tile<DP, NPART, NKB>(a, kt, kvh, b, smem, sid);
+            ++sid;  // (ids of one tile's last staging are not met by the next's)
+            if (!a.pair || kt == second || second <= p) break;
+            kt = second;
+        }
+        return true;
+    }
+};
+template <class... S>
+constexpr int bwd_shapes_bytes() {
+    int m = 0;
+    ((m = S::BYTES > m ? S::BYTES : m), ...);
+    return m;
+}
+template <class... S>
+DEVI void bwd_shapes(const BwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[bwd_shapes_bytes<S...>()];
+    (void)(S::run(a, smem) || ...);
+}
+#define ZT_BWD_SPLIT(NAME, ...)                                                                      \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME(BwdArgs a) { bwd_shapes<__VA_ARGS__>(a); }
+#define BS(DP, NPART, NKB) BwdShape<DP, NPART, NKB>
+
 #define ZT_BWD_DQ(DP, BK)                                                                          \
     extern "C" __global__ void __launch_bounds__(256, (DP) <= ((BK) == 32 ? 192 : 128) ? 2 : 1)  \
         zt_bwd_dq_d##DP##_k##BK(BwdArgs a) {                                                       \
@@ -1315,13 +1685,13 @@ __device__ __forceinline__ void bwd_dkdv_dma_body(const BwdArgs &a) {
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8p_d##DP##_hs2(BwdArgs a) {    \
         bwd_dkdv_body<DP, 2, 4, true>(a);                                                          \
     }
-// Eight-wave dk/dv that reads the forward's scores instead of recomputing Q K^T,
-// 32 query rows per stage (without K in registers two 16-row sub-tiles fit:
-// C3 2.09 -> 2.02 ms against one).
-#define ZT_BWD_DKDV8S(DP)                                                                          \
-    extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8s_d##DP##_hs2(BwdArgs a) {    \
-        bwd_dkdv_body<DP, 2, 4, true, 2, true>(a);                                                 \
-    }
+// dk/dv that reads the forward's scores, on split operands: one list of shapes
+// per width under two names, for head groups of two and more (dkdv8s) and for
+// one that cannot be halved (dmars).
+#define ZT_BWD_SPLIT_32(NAME) ZT_BWD_SPLIT(NAME, BS(32, 2, 4), BS(32, 4, 2), BS(32, 8, 1))
+#define ZT_BWD_SPLIT_64(NAME) ZT_BWD_SPLIT(NAME, BS(64, 2, 4), BS(64, 4, 2), BS(64, 4, 1))
+#define ZT_BWD_SPLIT_96(NAME) ZT_BWD_SPLIT(NAME, BS(96, 2, 4), BS(96, 2, 2))
+#define ZT_BWD_SPLIT_128(NAME) ZT_BWD_SPLIT(NAME, BS(128, 2, 4), BS(128, 2, 2))
 #define ZT_BWD_DKDV_DMA(DP, HS)                                                                    \
     extern "C" __global__ void __launch_bounds__(256) zt_bwd_dkdv_dma_d##DP##_hs##HS(BwdArgs a) { \
         bwd_dkdv_dma_body<DP, HS>(a);                                                              \
@@ -1340,7 +1710,10 @@ ZT_BWD_ALL(32)
 ZT_BWD_ALL(64)
 ZT_BWD_ALL(96)
 ZT_BWD_ALL(128)
-ZT_BWD_DKDV8S(32) ZT_BWD_DKDV8S(64) ZT_BWD_DKDV8S(96) ZT_BWD_DKDV8S(128)
+ZT_BWD_SPLIT_32(zt_bwd_dkdv8s_d32_hs2)
+ZT_BWD_SPLIT_64(zt_bwd_dkdv8s_d64_hs2)
+ZT_BWD_SPLIT_96(zt_bwd_dkdv8s_d96_hs2)
+ZT_BWD_SPLIT_128(zt_bwd_dkdv8s_d128_hs2)
 // The 4-way splits: the 160 KB LDS holds 4 parts' tiles (double-buffered for
 // the asynchronous variant) up to d = 128.
 ZT_BWD_DKDV(32, 4)
@@ -1354,13 +1727,11 @@ ZT_BWD_DKDV(128, 4)
         bwd_dkdv_dma_body<DP, 2, false, true>(a);                                                  \
     }
 ZT_BWD_DKDV_DMAR(32) ZT_BWD_DKDV_DMAR(64) ZT_BWD_DKDV_DMAR(96) ZT_BWD_DKDV_DMAR(128)
-// The same reading the forward's scores: each part's wave loads its own
-// row tile's score tile and writes dS over it.
-#define ZT_BWD_DKDV_DMARS(DP)                                                                      \
-    extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv_dmars_d##DP(BwdArgs a) {       \
-        bwd_dkdv_dma_body<DP, 2, true, true>(a);                                                   \
-    }
-ZT_BWD_DKDV_DMARS(32) ZT_BWD_DKDV_DMARS(64) ZT_BWD_DKDV_DMARS(96) ZT_BWD_DKDV_DMARS(128)
+// The same reading the forward's scores.
+ZT_BWD_SPLIT_32(zt_bwd_dkdv_dmars_d32)
+ZT_BWD_SPLIT_64(zt_bwd_dkdv_dmars_d64)
+ZT_BWD_SPLIT_96(zt_bwd_dkdv_dmars_d96)
+ZT_BWD_SPLIT_128(zt_bwd_dkdv_dmars_d128)
 ZT_BWD_DKDV_DMA(32, 4)
 ZT_BWD_DKDV_DMA(64, 4)
 ZT_BWD_DKDV_DMA(96, 4)
@@ -1399,7 +1770,8 @@ ZT_BWD_DKDV8PD1(64) ZT_BWD_DKDV8PD1(128)
 #else
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
-ZT_BWD_DQ_PF(32) ZT_BWD_DQ_LSE(32) ZT_BWD_DKDV8(32) ZT_BWD_DKDV8S(128)
+ZT_BWD_DQ_PF(32) ZT_BWD_DQ_LSE(32) ZT_BWD_DKDV8(32)
+ZT_BWD_SPLIT_128(zt_bwd_dkdv8s_d128_hs2)
 #endif
 
 // delta[row] = sum_d o[row, d] * dout[row, d] over the B*T*H rows of dim

@@ -166,7 +166,7 @@ int launch(DeviceState *st, const char *name, unsigned blocks, const Args &args,
 enum Tune {
     kTuneBK, kTuneFwdW, kTuneFPF, kTuneFPair, kTuneQPF, kTuneDqW, kTuneHS, kTuneW8, kTunePF, kTuneDMA, kTuneBPair,
     kTuneDSplit, kTuneRSplit, kTuneDecWgs, kTuneGemmTile, kTuneGemmSk, kTuneGemmSkTile, kTuneDqdsTile, kTuneRowG,
-    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneFShape, kTuneCount
+    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneFShape, kTuneBShape, kTuneCount
 };
 struct TuneSpec {
     const char *name;
@@ -198,6 +198,7 @@ const TuneSpec kTuneSpecs[kTuneCount] = {
     {"ZT_DQDS_K", {1, 2}, 2},
     {"ZT_ATTN_RSCORES", {0, 1}, 2},
     {"ZT_ATTN_FSHAPE", {11, 12, 14, 21, 22}, 5},
+    {"ZT_ATTN_BSHAPE", {1, 2, 4}, 3},
 };
 std::atomic<int> g_tune[kTuneCount] = {};  // 0 = unset (no allowed value is 0 except a flag, stored as value + 1)
 
@@ -920,6 +921,24 @@ static float *ws_tiles(void *workspace, int B, int T, int n_heads) {
     return reinterpret_cast<float *>(static_cast<char *>(workspace) + align256((size_t)B * T * n_heads * sizeof(float)));
 }
 
+// The split-operand dk/dv kernel's shape: 16-key blocks per workgroup and the
+// parts its (head, 32-row block) items are dealt to.  Four blocks share each
+// staged tile between most keys; fewer give more workgroups with shorter item
+// lists where 64-key tiles leave CUs idle.  Measured on MI355X with delta (us,
+// blocks 4 / 2 / 1): 4 over 2 heads at d = 32, T = 4096 406 / 213 / 130, T = 256
+// 31 / 19 / 14; 12 over 4 heads at d = 64, 4 x 512 rows 96 / 63 / 72; 32 over 8 at d =
+// 128, T = 512 182 / 177, T = 4096 1517 / 2784.
+static void dkdv_split_shape(int B, int T, int n_kv_heads, int dp, int cus, int *parts, int *kblocks) {
+    const long long wgs = (long long)((T + 63) / 64) * n_kv_heads * B;  // 64 keys each
+    int kb = 4;
+    if (2 * wgs <= cus || (dp == 32 && wgs <= cus)) kb = 2;
+    if ((4 * wgs <= cus && dp <= 64) || (dp == 32 && 2 * wgs <= cus)) kb = 1;
+    const int forced = tuned(kTuneBShape, kb);
+    kb = forced == 1 && dp > 64 ? 2 : forced;
+    *kblocks = kb;
+    *parts = dp > 64 ? 2 : kb == 4 ? 2 : kb == 2 ? 4 : dp == 32 ? 8 : 4;
+}
+
 // Which workspaces hold scores, and of what.  zt_attn_forward_train_ws stamps
 // the workspace it wrote scores into with the call's device, q, k and shape;
 // the first backward stage 1 that consumes them (ZT_WS_SCORES) checks the
@@ -1055,29 +1074,35 @@ int zt_attn_backward_train_ws(const float *q, const float *k, const float *v, co
                 "       Refusing rather than reading stale tiles: run the forward again, or drop ZT_WS_SCORES.\n");
         return 1;
     }
-    if (read_scores && sk == ScoreKernel::RowSplit) {
-        // The row-split kernel the statistics path chose (backward_prepare
-        // set its grid), reading the scores instead of forming Q K^T.
-        snprintf(name_b, sizeof name_b, "zt_bwd_dkdv_dmars_d%d", dp);
-    } else if (read_scores) {
-        // The forward left the scores in the dS tiles: a kernel that reads
-        // them, 2 head halves x 64 keys (eight waves, d <= 128) or x 32 keys
-        // (wider heads: eight waves splitting the columns, or four waves with
-        // asynchronous staging) per workgroup.  (Unaligned q / dout rows form
-        // Q K^T again.)
-        a.HS = 2;
-        const int keys = dp <= 128 ? 64 : 32;
-        const bool dsplit = dp > 128 && dkdv_dsplit(dp, st->lds_limit);
+    if (read_scores && dp <= 128) {
+        // The forward left the scores in the dS tiles: the split-operand kernel,
+        // whose shape follows the grid.
+        dkdv_split_shape(B, T, n_kv_heads, dp, st->cus, &a.parts, &a.kblocks);
+        const int keys = 16 * a.kblocks;
         a.n_key_tiles = (T + keys - 1) / keys;
         a.pair = tuned(kTuneBPair, pair_pays((unsigned long long)a.n_key_tiles * n_kv_heads * B, st->cus));
         const unsigned long long blocks =
             (unsigned long long)(a.pair ? (a.n_key_tiles + 1) / 2 : a.n_key_tiles) * n_kv_heads * B;
-        threads_b = dp <= 128 || dsplit ? 512 : 256;
+        threads_b = 64u * a.parts * a.kblocks;
         if (!grid_ok(blocks, threads_b)) return 1;
         blocks_b = (unsigned)blocks;
         snprintf(name_b, sizeof name_b,
-                 dp <= 128 ? "zt_bwd_dkdv8s_d%d_hs2" : dsplit ? "zt_bwd_dkdv8sd_d%d_hs2" : "zt_bwd_dkdv_dmas_d%d_hs2",
-                 dp);
+                 sk == ScoreKernel::RowSplit ? "zt_bwd_dkdv_dmars_d%d" : "zt_bwd_dkdv8s_d%d_hs2", dp);
+    } else if (read_scores) {
+        // Wider heads, 2 head halves x 32 keys: eight waves splitting the columns,
+        // or four waves with asynchronous staging.  (Unaligned q / dout rows form
+        // Q K^T again.)
+        a.HS = 2;
+        const int keys = 32;
+        const bool dsplit = dkdv_dsplit(dp, st->lds_limit);
+        a.n_key_tiles = (T + keys - 1) / keys;
+        a.pair = tuned(kTuneBPair, pair_pays((unsigned long long)a.n_key_tiles * n_kv_heads * B, st->cus));
+        const unsigned long long blocks =
+            (unsigned long long)(a.pair ? (a.n_key_tiles + 1) / 2 : a.n_key_tiles) * n_kv_heads * B;
+        threads_b = dsplit ? 512 : 256;
+        if (!grid_ok(blocks, threads_b)) return 1;
+        blocks_b = (unsigned)blocks;
+        snprintf(name_b, sizeof name_b, dsplit ? "zt_bwd_dkdv8sd_d%d_hs2" : "zt_bwd_dkdv_dmas_d%d_hs2", dp);
     }
     if (stage & 1) {
         // Stage 1 writes dS over the tiles: whatever scores they held are gone.
