@@ -168,8 +168,15 @@ def test_dkdv_with_large_operands(gpu, zt, where):
     args = {"q": q, "k": k, "v": v, "do": do, where: x}
     got = _train(gpu, zt, args["q"], args["k"], args["v"], args["do"], T, H, Hkv, D)
     want = attention_backward_f64(*(host(args[n]) for n in ("q", "k", "v", "do")), T, H, Hkv, D)
-    for g, w, o, heads in zip(got, want, good, (H, Hkv, Hkv)):
+    for n, g, w, o, heads in zip(("dq", "dk", "dv"), got, want, good, (H, Hkv, Hkv)):
         g, w, o = (np.asarray(y).reshape(T, heads, D) for y in (g, w, o))
         assert np.all(np.isfinite(g))
-        assert np.max(np.abs(g - w)) <= 1e-5 * np.abs(w).max()
+        err, tol = np.abs(g - w), np.full(D, 1e-5 * np.abs(w).max())
+        if where == "q" and n == "dk":
+            # Row S's softmax is one-hot, so its dS = dP - delta is exactly 0, as the
+            # difference of two f32 sums of the same D products dO V, each off by up to
+            # D 2^-24 of the sum of their magnitudes; column 3 of dk takes it times 2^70.
+            mags = np.abs(host(do).reshape(T, H, D)[S, -1] * host(v).reshape(T, Hkv, D)[:, -1]).sum(1).max()
+            tol[3] += 2 * D * 2.0 ** -24 * mags * 2.0 ** 70 / np.sqrt(D)
+        assert np.all(err <= tol)
         assert np.array_equal(g[:, :heads // 2].view(np.uint32), o[:, :heads // 2].astype(np.float32).view(np.uint32))
