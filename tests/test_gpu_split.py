@@ -180,3 +180,29 @@ def test_dkdv_with_large_operands(gpu, zt, where):
             tol[3] += 2 * D * 2.0 ** -24 * mags * 2.0 ** 70 / np.sqrt(D)
         assert np.all(err <= tol)
         assert np.array_equal(g[:, :heads // 2].view(np.uint32), o[:, :heads // 2].astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("where", ["", "do", "k"])
+@pytest.mark.parametrize("T,H,Hkv,D", [(2, 2, 1, 128), (33, 4, 2, 96), (129, 2, 1, 36), (161, 4, 4, 128),
+                                       (300, 4, 2, 192)])
+def test_dq_product_on_split_operands(gpu, zt, tune, T, H, Hkv, D, where):
+    """The 128-tile dq = dS K product: edges of tiles, slabs and columns, a row
+    of dO with an entry of 2^70 (its dS is past the split's range) and a column of
+    K with one (Q holds 0 there, so the scores do not).  Same gate as the shapes
+    of dk/dv above, over the entries the large value reaches and over the rest."""
+    tune({"ZT_DQDS_TILE": 128, "ZT_DQDS_K": 1})
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    do = dev_normal(gpu, zt, T * H * D, SEED_DO)
+    S, reached = T // 2, np.zeros((T, H, D), bool)
+    if where == "do":
+        do.view(T, H, D)[S, -1, 3] = 2.0 ** 70
+        reached[S, -1] = True
+    if where == "k":
+        q.view(T, H, D)[:, :, 3] = 0.0
+        k.view(T, Hkv, D)[S, -1, 3] = 2.0 ** 70
+        reached[S:, H - H // Hkv:, 3] = True
+    want = np.asarray(attention_backward_f64(*(host(x) for x in (q, k, v, do)), T, H, Hkv, D)[0]).reshape(T, H, D)
+    got = _train(gpu, zt, q, k, v, do, T, H, Hkv, D)[0].reshape(T, H, D)
+    for part in (reached, ~reached):
+        if part.any():
+            assert np.max(np.abs(got[part] - want[part])) <= 1e-5 * max(1.0, np.abs(want[part]).max())

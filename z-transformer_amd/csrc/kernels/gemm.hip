@@ -1,4 +1,5 @@
-// f32 GEMM on FP32 MFMA for the model's dense products (gfx950):
+// f32 GEMM for the model's dense products (gfx950), on FP32 MFMA and, for the
+// 128 and whole 64 tiles, on split operands (gemm_split_tile below):
 //   zt_gemm_nn: C  = A B      src/tensor.zig:78-106 (tensor.matmul)
 //   zt_gemm_tn: C += A^T B    src/autograd.zig:958-972 (weightGrad: w += input^T dout)
 //   zt_gemm_nt: C += A B^T    src/autograd.zig:999-1022 (inputGrad: d input += dout w^T)
@@ -523,7 +524,9 @@ DEVI void gemm_sk_body(const GemmArgs &g) {
 // unaligned instantiations.
 template <int BT, int KSP>
 DEVI float *dq_ds_slabs() {
-    __shared__ __attribute__((aligned(16))) float slabs[KSP * 2 * BK * Tile<BT>::LIC];
+    constexpr int kF32 = KSP * 2 * BK * Tile<BT>::LIC * 4;
+    constexpr int kSplit = BT == 128 && KSP == 1 ? 2 * slab_bytes<128, false>() + 16 : 0;  // dq_ds_split_tile
+    __shared__ __attribute__((aligned(16))) float slabs[(kF32 > kSplit ? kF32 : kSplit) / 4];
     return slabs;
 }
 // KSP key parts (KSP = 2: eight waves, for grids that give a workgroup of four
@@ -672,6 +675,168 @@ DEVI void dq_ds_tile(const DqDsArgs &g, const int tm, const int tn, const int bh
         }
 }
 
+// The 128 tile on split operands (split.h), for 16-byte k rows: the slab loop of
+// gemm_split_tile with both operands index-contiguous, a dS chunk being four
+// queries at one key (eight bytes per part; 16 keys x 4 chunks of a tile cover
+// the banks twice, the least that 512 bytes take).  Loads stay unconditional and
+// in bounds as in dq_ds_tile.  Bound by power and by the splitting of the slabs
+// beside the products, as gemm_split_tile, two workgroups per CU.  32 over 8 heads,
+// d = 128, T = 4096: 558 us on f32 MFMAs (123 TFLOP/s), 458 us here (150 TFLOP/s);
+// that shape's training step 2780 -> 2715 us, 2 x 2048 rows of 16 over 4 heads at
+// d = 256 1791 -> 1733 us.
+DEVI void dq_ds_split_tile(const DqDsArgs &g, const int tm, const int tn, const int bh) {
+    constexpr int BT = 128, TW = Tile<BT>::TW, WT = Tile<BT>::WT, NA = BT * BK / 4 / NTHR, NB = NA / 2;
+    constexpr int S = split_stride<BT>();
+    char *const As = reinterpret_cast<char *>(dq_ds_slabs<BT, 1>()), *const Bs = As + slab_bytes<BT, false>();
+    // The slab id (k0 + 1) whose dS (K) holds a big value.
+    int *const flags = reinterpret_cast<int *>(Bs + slab_bytes<BT, false>());
+    const int tid = (int)threadIdx.x, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = WT * (w >> 1), wn = WT * (w & 1);
+    const int b = bh / g.H, h = bh % g.H, kvh = h / (g.H / g.Hkv);
+    const int m0 = tm * BT, n0 = tn * BT;
+    const size_t qld = (size_t)g.H * g.dim, kld = (size_t)g.Hkv * g.dim;
+    const int nt = (g.T + 15) >> 4;
+    const float *A = g.ds + (size_t)bh * zt_tri_count(nt) * 256;
+    const float *Bm = g.k + (size_t)b * g.T * kld + (size_t)kvh * g.dim;
+    float *C = g.dq + (size_t)b * g.T * qld + (size_t)h * g.dim;
+    const int kend = min(g.T, m0 + BT);
+    if (tid < 2) flags[tid] = 0;
+
+    f4 acc[TW][TW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int j = 0; j < TW; ++j) acc[i][j] = zero4();
+
+    f4 pa[NA], pb[NB][2];
+    auto fetch_a = [&](int k0) {
+#pragma unroll
+        for (int n = 0; n < NA; ++n) {
+            const int e = tid + n * NTHR;
+            const int tile = e >> 6, c = e & 63;
+            const int tb = (m0 >> 4) + tile % (BT / 16), sb = (k0 >> 4) + tile / (BT / 16);
+            const int tc = min(tb, nt - 1), sc = min(sb, tc);
+            const f4 x = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(A + zt_tri_index(tc, sc) * 256) + c);
+            pa[n] = sb <= tb && tb < nt ? x : zero4();
+        }
+    };
+    auto fetch_b = [&](int k0) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const int e = tid + n * NTHR;
+            const float *row = Bm + (size_t)min(k0 + e / (BT / 8), kend - 1) * kld;
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                pb[n][x] = *reinterpret_cast<const f4 *>(row + min(n0 + 8 * (e % (BT / 8)) + 4 * x, g.dim - 4));
+        }
+    };
+    fetch_a(0);
+    fetch_b(0);
+#pragma unroll 1
+    for (int k0 = 0; k0 < kend; k0 += BK) {
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < NA; ++n) {
+            const int e = tid + n * NTHR;
+            const int tile = e >> 6, c = e & 63;
+            float y[4] = {pa[n][0], pa[n][1], pa[n][2], pa[n][3]};
+            if (any_big(max_abs(y))) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = small_part(y[i]);
+                if (lane == 0) flags[0] = k0 + 1;
+            }
+            u2 hi, mi, lo;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                unsigned x0, x1, x2;
+                split2(y[2 * i], y[2 * i + 1], x0, x1, x2);
+                hi[i] = x0; mi[i] = x1; lo[i] = x2;
+            }
+            char *p = As + (16 * (tile / (BT / 16)) + (c & 15)) * S + 2 * (16 * (tile % (BT / 16)) + 4 * (c >> 4));
+            *reinterpret_cast<u2 *>(p) = hi;
+            *reinterpret_cast<u2 *>(p + BK * S) = mi;
+            *reinterpret_cast<u2 *>(p + 2 * BK * S) = lo;
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const int e = tid + n * NTHR;
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = pb[n][i / 4][i % 4];
+            if (any_big(max_abs(y))) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
+                if (lane == 0) flags[1] = k0 + 1;
+            }
+            put_tri<BT>(Bs, BK, e / (BT / 8), e % (BT / 8) * 8, split8(y));
+        }
+        __syncthreads();
+        if (k0 + BK < kend) {
+            fetch_a(k0 + BK);
+            fetch_b(k0 + BK);
+        }
+        const bool abig = __builtin_amdgcn_readfirstlane(flags[0]) == k0 + 1;
+        const bool bbig = __builtin_amdgcn_readfirstlane(flags[1]) == k0 + 1;
+        if (!(abig && bbig)) {
+            Tri bt[TW];
+#pragma unroll
+            for (int j = 0; j < TW; ++j) {
+                bt[j].l = get_col<BT>(Bs, BK, 0, wn + 16 * j, lane, 0);
+                bt[j].m = get_col<BT>(Bs, BK, 0, wn + 16 * j, lane, 1);
+                bt[j].h = get_col<BT>(Bs, BK, 0, wn + 16 * j, lane, 2);
+            }
+            f4 t[TW];
+            stream_parts<TW, 3>([&](int i, int part) { return get_col<BT>(As, BK, 0, wm + 16 * i, lane, part); },
+                                [&](int i, auto part, u4 x) {
+                                    if constexpr (part == 0) {
+#pragma unroll
+                                        for (int j = 0; j < TW; ++j) t[j] = zero4();
+                                    }
+                                    mfma_parts<part>(t, x, [&](int j) -> const Tri & { return bt[j]; });
+                                    if constexpr (part == 2) {
+#pragma unroll
+                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j];
+                                    }
+                                });
+        }
+        if (abig || bbig) {
+            // Products with a big operand from the full values (both: the whole slab).
+            const int ll = opaque(lane), li = ll & 15, lg = ll >> 4;
+#pragma unroll 1
+            for (int kk = 0; kk < 8; ++kk) {
+                const int k = k0 + 4 * kk + lg, sb = k >> 4;
+                float av[TW], bv[TW];
+#pragma unroll
+                for (int i = 0; i < TW; ++i) {
+                    const int tb = ((m0 + wm) >> 4) + i, n = n0 + wn + 16 * i + li;
+                    av[i] = sb <= tb && tb < nt
+                                ? A[zt_tri_index(tb, sb) * 256 + ((li >> 2) * 16 + (k & 15)) * 4 + (li & 3)] : 0.f;
+                    bv[i] = n < g.dim && k < kend ? Bm[(size_t)k * kld + n] : 0.f;
+                    if (!bbig) av[i] = big_part(av[i]);
+                    if (!abig) bv[i] = big_part(bv[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < TW; ++i)
+#pragma unroll
+                    for (int j = 0; j < TW; ++j) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = m0 + wm + 16 * i + 4 * grp + r;
+            if (t >= g.T) continue;
+            float *crow = C + (size_t)t * qld + n0 + wn + l16;
+#pragma unroll
+            for (int j = 0; j < TW; ++j)
+                if (n0 + wn + 16 * j + l16 < g.dim)
+                    crow[16 * j] = ZT_PLANT == 16 ? acc[i][j][r] : acc[i][j][r] * g.scale;
+        }
+}
+
 // A workgroup takes row tiles tiles_m - 1 - p and p one after the other, so
 // every workgroup has the same causal work (C3: 0.64 -> 0.58 ms against one
 // row tile per workgroup, heaviest first).
@@ -683,10 +848,14 @@ DEVI void dq_ds_body(const DqDsArgs &g) {
     const int bh = rem % (g.B * g.H);
     const int p = rem / (g.B * g.H);
     if (KSP > 1 || g.vec) {  // (the host takes the key-split kernels only with vec)
-        dq_ds_tile<BT, true, KSP>(g, g.tiles_m - 1 - p, tn, bh);
+        const auto tile = [&](int tm) {
+            if constexpr (BT == 128 && KSP == 1) dq_ds_split_tile(g, tm, tn, bh);
+            else dq_ds_tile<BT, true, KSP>(g, tm, tn, bh);
+        };
+        tile(g.tiles_m - 1 - p);
         if (p < g.tiles_m - 1 - p) {  // workgroup-uniform
             __syncthreads();  // the first tile's last LDS reads before the second's writes
-            dq_ds_tile<BT, true, KSP>(g, p, tn, bh);
+            tile(p);
         }
     } else {
         dq_ds_tile<BT, false>(g, g.tiles_m - 1 - p, tn, bh);
@@ -723,7 +892,7 @@ ZT_GEMM(32)
 ZT_GEMM_SK(1, 16)
 ZT_GEMM_SK(2, 32)
 
-extern "C" __global__ void __launch_bounds__(256) zt_gemm_dqds_128(DqDsArgs g) { dq_ds_body<128>(g); }
+extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_dqds_128(DqDsArgs g) { dq_ds_body<128>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_dqds_64(DqDsArgs g) { dq_ds_body<64>(g); }
 // Two key parts, eight waves (grids of at most one four-wave workgroup per CU).
 extern "C" __global__ void __launch_bounds__(512) zt_gemm_dqds2_64(DqDsArgs g) { dq_ds_body<64, 2>(g); }
