@@ -1,4 +1,6 @@
-// Fused causal grouped-query attention, forward, f32 on FP32 MFMA (gfx950).
+// Fused causal grouped-query attention, forward, f32 (gfx950): on FP32 MFMA, and
+// on split operands (split.h, the second half of the file) wherever rows are whole
+// 16-byte chunks and the width allows.
 //
 // Computes what src/cuda/attn_kernels.cu:197-369 (fusedAttnForward) computes
 // -- O = softmax(Q K^T / sqrt(d), causal) V with query row t at absolute
