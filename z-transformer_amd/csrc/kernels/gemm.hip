@@ -877,6 +877,9 @@ DEVI void dq_ds_body(const DqDsArgs &g) {
 
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nn_128(GemmArgs g) { gemm_split_body<128, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_128(GemmArgs g) { gemm_split_body<128, false, false>(g); }
+// f32 MFMA forms, for the products where the split loses (zt_attn.cpp, gemm_impl).
+extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_128f(GemmArgs g) { gemm_body<128, false, false>(g); }
+extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_64f(GemmArgs g) { gemm_body<64, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_128(GemmArgs g) { gemm_split_body<128, true, true>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_nn_64(GemmArgs g) { gemm_body<64, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_64(GemmArgs g) { gemm_split_body<64, false, false>(g); }

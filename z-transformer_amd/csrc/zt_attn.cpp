@@ -1667,8 +1667,17 @@ static int gemm_impl(const char *name, const char *what, const float *a, int lda
     g.vec_a = lda % 4 == 0 && (uintptr_t)a % 16 == 0;
     g.vec_b = ldb % 4 == 0 && (uintptr_t)b % 16 == 0;
     g.vec_c = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
+    // The f32 MFMA form of the weight gradient (..f) where splitting the slabs is not
+    // paid back (us, f32 / split, M x N x K): few slabs, 4096 x 4096 x 128 55.6 / 60.6 (x 250
+    // 91.6 / 86.4); at most a workgroup per CU (or 64 tiles) below 2048 deep, 4096 x 1024 x
+    // 128 17.9 / 25.0, x 1024 80 / 84, x 1500 125 / 129 (x 2048 150 / 134).
+    const bool tn = strcmp(name, "zt_gemm_tn") == 0;
+    const bool whole64 = g.vec_a && g.vec_b && M % 64 == 0 && N % 64 == 0 && K % 32 == 0;
+    const bool f32 = tn && !sk && tuned(kTuneGemmTile, 0) == 0 &&
+                     ((bt == 64 && !(whole64 && K >= 2048)) ||
+                      (bt == 128 && (K < 192 || (blocks <= (unsigned long long)st->cus && K < 2048))));
     char kname[32];
-    snprintf(kname, sizeof kname, sk ? "%s_sk%d" : "%s_%d", name, bt);
+    snprintf(kname, sizeof kname, sk ? "%s_sk%d" : f32 ? "%s_%df" : "%s_%d", name, bt);
     return launch(st, kname, (unsigned)blocks, g, stream, threads);
 }
 
