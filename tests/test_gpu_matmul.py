@@ -176,3 +176,22 @@ def test_split_k_is_deterministic_and_chosen_for_the_model_shapes(gpu, zt):
         assert np.array_equal(outs[0], outs[1])
     assert zt.gemm_kernel(256, 512, 128) == "zt_gemm_nn_sk16"
     assert zt.gemm_kernel(4096, 4096, 4096) == "zt_gemm_nn_128"
+
+
+@pytest.mark.parametrize("M,N", [(2048, 2048), (1024, 2048), (1024, 1024), (2049, 2050)])
+@pytest.mark.parametrize("op", ["nn", "tn", "nt"])
+def test_an_empty_contraction_reads_nothing(gpu, zt, op, M, N):
+    """K = 0 on grids of whole and ragged 128, 64 and 32 tiles, with null
+    operands as the ABI allows: matmul writes zeros, the accumulating products
+    leave their output as it was."""
+    empty = gpu.empty(0, device="cuda")
+    c = gpu.randn(M * N, device="cuda") + 10.0
+    before = c.clone()
+    if op == "nn":
+        zt.matmul(empty, empty, c, M, 0, N)
+    elif op == "tn":
+        zt.weight_grad(c, empty, empty, 0, M, N)
+    else:
+        zt.input_grad(c, empty, empty, M, 0, N)
+    gpu.cuda.synchronize()
+    assert gpu.equal(c, gpu.zeros_like(c) if op == "nn" else before)
