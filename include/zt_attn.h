@@ -271,8 +271,9 @@ int zt_rope_qk_backward(const float *dq, const float *dk, float *dq_out, float *
 
 /* ---- Dense products of the model step (no reference C entry point) ----
  * src/tensor.zig:78-106 (tensor.matmul) on the device: out[M,N] = a[M,K] b[K,N],
- * row-major f32, products on the matrix cores at f32 precision (FP32 MFMA, or
- * three exact bf16 parts per operand) with f32 accumulation (the reference reduces in f32
+ * row-major f32, products on the matrix cores at f32 precision over f32's whole
+ * range (FP32 MFMA, or three bf16 parts per operand that add up to it exactly) with
+ * f32 accumulation (the reference reduces in f32
  * too, src/tensor_test.zig:185-273; only the rounding order differs).  K = 0
  * writes zeros; M = 0 or N = 0 writes nothing.  The reference's
  * DimensionMismatch is the caller's shape check (sizes are explicit here). */

@@ -1,7 +1,8 @@
 """The kernels that form f32 products from three bf16 parts per operand
 (csrc/kernels/split.h): every wave shape of the forward against a float64
-reference, at tile edges and remainders, and operands too large for the split
-(infinities, magnitudes of 2^60 and more), which take f32 products instead.
+reference, at tile edges and remainders, operands too large for the split
+(infinities, magnitudes of 2^40 and more), which take f32 products instead, and
+operands near the bottom of f32's range, which keep all their bits.
 
 Gate: an output is a convex combination of V rows (|V| up to about 5 here), so
 an error of 2^-22 in a weight's exponent and 2^-22 in its product are below
@@ -206,3 +207,52 @@ def test_dq_product_on_split_operands(gpu, zt, tune, T, H, Hkv, D, where):
     for part in (reached, ~reached):
         if part.any():
             assert np.max(np.abs(got[part] - want[part])) <= 1e-5 * max(1.0, np.abs(want[part]).max())
+
+
+def _scaled(gpu, x, e):
+    """x 2^e, rounded once to f32 (denormal values kept)."""
+    return (x.double().cpu() * 2.0 ** e).float().cuda()
+
+
+@pytest.mark.parametrize("op", ["nn", "tn", "nt"])
+@pytest.mark.parametrize("e", [-116, -124, -135])
+@pytest.mark.parametrize("which", ["a", "b"])
+def test_small_operands_keep_their_bits_in_products(gpu, zt, tune, op, e, which):
+    """One operand near or in f32's denormal range: test_split_products' bound
+    (relative to the sum of the products' magnitudes), plus the results' own
+    denormal rounding, 2^-150 an addition."""
+    tune({"ZT_GEMM_TILE": 128})
+    M, K, N = 130, 96, 128
+    gen = gpu.Generator(device="cuda").manual_seed(11)
+    a, b = (gpu.randn(s, device="cuda", generator=gen) for s in ((M, K), (K, N)))
+    a, b = (_scaled(gpu, a, e), b) if which == "a" else (a, _scaled(gpu, b, e))
+    want = a.double().cpu() @ b.double().cpu()
+    n = 34 + K / 32
+    bound = (a.double().abs().cpu() @ b.double().abs().cpu()) * (n * 2.0 ** -24) + n * 2.0 ** -150
+    assert gpu.all((_product(gpu, zt, op, a, b).double().cpu() - want).abs() <= bound)
+
+
+@pytest.mark.parametrize("shape", [12, 21])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_small_values_keep_their_bits_in_the_forward(gpu, zt, tune, shape, D):
+    """V scaled by 2^-124: the output is the same combination, to the same relative gate."""
+    tune({"ZT_ATTN_FSHAPE": shape})
+    T, H, Hkv = 100, 4, 2
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    v = _scaled(gpu, v, -124)
+    want = attention_f64(host(q), host(k), host(v), T, H, Hkv, D).ravel()
+    assert np.max(np.abs(_forward(gpu, zt, q, k, v, T, H, Hkv, D) - want)) <= TOL * 2.0 ** -124
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_small_gradients_keep_their_bits(gpu, zt, tune, D):
+    """dO scaled by 2^-124 scales every gradient by it: test_every_dkdv_shape's
+    gate relative to the gradient (with the dq product on split operands too)."""
+    tune({"ZT_DQDS_TILE": 128, "ZT_DQDS_K": 1})
+    T, H, Hkv = 161, 4, 2
+    q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+    do = _scaled(gpu, dev_normal(gpu, zt, T * H * D, SEED_DO), -124)
+    want = attention_backward_f64(*(host(x) for x in (q, k, v, do)), T, H, Hkv, D)
+    for got, w in zip(_train(gpu, zt, q, k, v, do, T, H, Hkv, D), want):
+        w = np.asarray(w).ravel()
+        assert np.max(np.abs(got - w)) <= 1e-5 * np.abs(w).max()

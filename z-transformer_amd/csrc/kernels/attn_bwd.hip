@@ -1441,9 +1441,11 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
         if (live) fetch(a.q, r0, hd);
         f4 ds[2];
         if (active) {
-            // dP starts at -delta (C layout: rows 16 j + 4 grp + r).
 #pragma unroll
-            for (int j = 0; j < 2; ++j) ds[j] = *reinterpret_cast<const f4 *>(st_del + 16 * j + 4 * grp);
+            for (int j = 0; j < 2; ++j) ds[j] = zero4();
+            f4 del[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) del[j] = *reinterpret_cast<const f4 *>(st_del + 16 * j + 4 * grp);
             const bool dobig = __builtin_amdgcn_readfirstlane(flags[0]) == sid;
             if (!(dobig && vbig))
                 stream_parts<2 * NKS, 6>(
@@ -1453,6 +1455,9 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
                         mfma_parts<prt>(t, x, [&](int) -> const Tri & { return v[i >> 1]; });
                         ds[i & 1] = t[0];
                     });
+            // dP - delta (C layout: rows 16 j + 4 grp + r).
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ds[j] = ds[j] * kUnscale + del[j];
             if (dobig || vbig) {  // products with a big operand, from the full values
                 const int ol = opaque(lane), li = ol & 15, lg = ol >> 4;
                 const float *vr = a.v + ((size_t)b * a.T + min(key0 + li, a.T - 1)) * kld + (size_t)kvr * a.dim;
@@ -1497,14 +1502,14 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
 #pragma unroll
                 for (int i = 0; i < 8; ++i) ps[i] = small_part(ps[i]);
             }
-            const Tri pt = split8(ps);
+            const Tri pt = split8_as_is(ps);
             if (!(dobig && pbig)) {
                 f4 t[1];
                 stream_parts<NT, 6>([&](int i, int prt) { return get_col<DP>(dOs, 32, 0, 16 * i, lane, prt); },
                                     [&](int i, auto prt, u4 x) {
                                         if constexpr (prt == 0) t[0] = zero4();
                                         mfma_parts<prt>(t, x, [&](int) -> const Tri & { return pt; });
-                                        if constexpr (prt == 2) dv[i] += t[0];
+                                        if constexpr (prt == 2) dv[i] += t[0] * kUnscale1;
                                     });
             }
             if (dobig || pbig) {
@@ -1555,7 +1560,7 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
                                     [&](int i, auto prt, u4 x) {
                                         if constexpr (prt == 0) t[0] = zero4();
                                         mfma_parts<prt>(t, x, [&](int) -> const Tri & { return dt; });
-                                        if constexpr (prt == 2) dk[i] += t[0];
+                                        if constexpr (prt == 2) dk[i] += t[0] * kUnscale;
                                     });
             }
             if (dsbig || qbig) {

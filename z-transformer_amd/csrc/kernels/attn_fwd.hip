@@ -380,7 +380,7 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
             x[n][1] = *reinterpret_cast<const f4 *>(p + (r + vcol2[n % NC]));
         }
     };
-    auto put = [&](const f4 (&x)[NP][2], char *t, int *flag, int id) {
+    auto put = [&](const f4 (&x)[NP][2], char *t, int *flag, int id, auto split) {
 #pragma unroll
         for (int n = 0; n < NP; ++n) {
             const int e = tid + n * NTH;
@@ -398,7 +398,7 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
                 for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
                 if (lane == 0) *flag = id;
             }
-            put_tri<DP>(t, ROWS, e / CPR, c, split8(y));
+            put_tri<DP>(t, ROWS, e / CPR, c, split(y));
         }
     };
 
@@ -427,7 +427,7 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = small_part(y[i]);
             }
-            q[ks][n] = split8(y);
+            q[ks][n] = split8_as_is(y);
         }
     }
     const bool qbig = any_big(qmax);
@@ -515,10 +515,12 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
     // loads' latency for small tiles.
     constexpr bool DEEP = NQ == 1 || DW <= 64;
     f4 px[NP][2], py[DEEP ? NP : 1][2];
-    auto stage_k = [&](int id) { put(px, ktile(id), kflag(id), id); };
+    const auto as_is = [](const float (&y)[8]) { return split8_as_is(y); };
+    const auto scaled = [](const float (&y)[8]) { return split8(y); };
+    auto stage_k = [&](int id) { put(px, ktile(id), kflag(id), id, as_is); };
     auto stage_v = [&](int id) {
-        if constexpr (DEEP) put(py, vtile(id), vflag(id), id);
-        else put(px, vtile(id), vflag(id), id);
+        if constexpr (DEEP) put(py, vtile(id), vflag(id), id, scaled);
+        else put(px, vtile(id), vflag(id), id, scaled);
     };
     const int klast = (kend_wg - 1) / ROWS * ROWS;  // the last step's first key
     fetch(px, kb, 0);
@@ -619,7 +621,7 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
                 float y[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) y[i] = s[(i / 4) * NQ + n][i % 4];
-                p[n] = split8(y);
+                p[n] = split8_as_is(y);
             }
             f4 t[NQ];
             stream_parts<NT, 3>(
@@ -632,7 +634,7 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
                     mfma_parts<part>(t, x, [&](int n) -> const Tri & { return p[n]; });
                     if constexpr (part == 2) {
 #pragma unroll
-                        for (int n = 0; n < NQ; ++n) o[i][n] += t[n];
+                        for (int n = 0; n < NQ; ++n) o[i][n] += t[n] * kUnscale1;
                     }
                 });
             if (__builtin_amdgcn_readfirstlane(*vflag(sid)) == sid) {

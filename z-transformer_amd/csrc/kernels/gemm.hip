@@ -360,7 +360,7 @@ DEVI void gemm_split_tile(const GemmArgs &g, char *smem) {
                                     mfma_parts<part>(t, x, [&](int j) -> const Tri & { return b[j]; });
                                     if constexpr (part == 2) {
 #pragma unroll
-                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j];
+                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j] * kUnscale;
                                     }
                                 });
         }
@@ -751,7 +751,7 @@ DEVI void dq_ds_split_tile(const DqDsArgs &g, const int tm, const int tn, const 
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 unsigned x0, x1, x2;
-                split2(y[2 * i], y[2 * i + 1], x0, x1, x2);
+                split2(scale_up(y[2 * i]), scale_up(y[2 * i + 1]), x0, x1, x2);
                 hi[i] = x0; mi[i] = x1; lo[i] = x2;
             }
             char *p = As + (16 * (tile / (BT / 16)) + (c & 15)) * S + 2 * (16 * (tile % (BT / 16)) + 4 * (c >> 4));
@@ -797,7 +797,7 @@ DEVI void dq_ds_split_tile(const DqDsArgs &g, const int tm, const int tn, const 
                                     mfma_parts<part>(t, x, [&](int j) -> const Tri & { return bt[j]; });
                                     if constexpr (part == 2) {
 #pragma unroll
-                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j];
+                                        for (int j = 0; j < TW; ++j) acc[i][j] += t[j] * kUnscale;
                                     }
                                 });
         }

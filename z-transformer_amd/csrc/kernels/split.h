@@ -19,15 +19,29 @@
 // (fewer roundings of the long accumulator), so a chain of at most 256 terms
 // accumulates in the MFMA and a longer one adds 32-term sums on the vector ALU.
 //
-// Range: an operand of magnitude 2^60 or more, infinities among them, would
-// overflow or turn into NaN in the split (inf - inf), so it enters the split
+// Range, below: bf16's smallest bit is 2^-133 and f32's 2^-149, so l loses bits of
+// an x under 2^-110 (the error of a product against 64-bit sums, 2.0e-7 on f32 MFMAs,
+// was 2.2e-6 with an operand of 2^-116 and 5.7e-4 at 2^-124).  Operands are
+// therefore split as 2^16 x (split8), which makes the split exact for denormal
+// values too (the conversion and the MFMA keep bf16 denormals; 5.6e-8 at every
+// scale), and the f32 add that takes a sum of products into its accumulator is a
+// multiply-add with 2^-32.  Scores and softmax weights are split without the
+// factor (split8_as_is), since only their absolute error counts: the exponential
+// sees the scores', under 2^-80, and the weights', 2^-134, is below the 2^-126 under
+// which the exponential returns 0.  (With it on the weights 333 rows over 2340
+// keys, 32 over 8 heads, d = 128, took 131 us instead of 128.)
+// What the factor costs (us, without / with): nothing in the forward; 32 over 8
+// heads, d = 128, T = 4096, dk/dv 1515 / 1531, dq product 439 / 445; MHA d = 64, 4 x 1024
+// rows x 8 heads, dk/dv 82.9 / 85.6.
+//
+// Range, above: an operand of magnitude 2^40 or more, infinities among them, could
+// overflow so scaled or turn into NaN in the split (inf - inf), so it enters the split
 // as 0 and its products are added by f32 MFMAs from the full value ("big"
 // below; NaN needs no care, every part of it is NaN).  Kernels flag a staged
 // tile that holds one, and only flagged tiles take that slow path; elements
 // that are not big keep the same arithmetic, bit for bit, with or without one
 // beside them (but where both operands of a tile hold one, the whole tile's
-// product is formed in f32).  Below 2^-110 the parts reach f32's denormal range and lose
-// bits whose products with operands near 1 are under 2^-133.
+// product is formed in f32).
 #pragma once
 #include "common.h"
 #include <utility>
@@ -38,7 +52,10 @@ typedef unsigned u2 __attribute__((ext_vector_type(2)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 typedef short s4i __attribute__((ext_vector_type(4)));
 
-constexpr float kBig = 0x1p60f;
+constexpr int kSplitExp = 16;         // a split operand is 2^16 x
+constexpr float kUnscale = 0x1p-32f;  // takes that back off a product of two
+constexpr float kUnscale1 = 0x1p-16f; // off a product with one operand as it is
+constexpr float kBig = 0x1p40f;       // 256 products of such operands, scaled: 2^120
 
 // x again, as a value the compiler knows nothing about: what a rarely taken
 // branch computes from it stays in the branch instead of being hoisted out of
@@ -66,7 +83,8 @@ DEVI void split2(float x0, float x1, unsigned &h, unsigned &m, unsigned &l) {
     x1 -= __uint_as_float(m & 0xffff0000u);
     l = pack_bf16(x0, x1);
 }
-DEVI Tri split8(const float (&x)[8]) {
+DEVI float scale_up(float x) { return __builtin_amdgcn_ldexpf(x, kSplitExp); }  // (an inline constant: no register)
+DEVI Tri split8_as_is(const float (&x)[8]) {
     Tri t;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -75,6 +93,13 @@ DEVI Tri split8(const float (&x)[8]) {
         t.h[i] = h; t.m[i] = m; t.l[i] = l;
     }
     return t;
+}
+
+DEVI Tri split8(const float (&x)[8]) {
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = scale_up(x[i]);
+    return split8_as_is(y);
 }
 
 // The f32 value whose parts are in the low (hi = 0) or high halves of h, m, l.
