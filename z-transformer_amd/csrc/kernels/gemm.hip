@@ -233,10 +233,11 @@ template <int BT, bool A_KC, bool B_KC>
 DEVI void gemm_body(const GemmArgs &g) {
     // Workgroup-uniform: the whole product is in full tiles (vec_c as well,
     // so the C rows take 16-byte stores), and a k-contiguous operand's chunk
-    // offsets (up to M lda or N ldb floats) fit the 32-bit offsets.  K = 0 has
-    // no slab, and A and B may be null there: the guarded loads read nothing.
+    // offsets (up to M lda or N ldb floats) fit the 32-bit offsets.  (K = 0 has no
+    // slab to load: the host clears vec_a and vec_b there.  Testing K here as well
+    // cost the 64 and 32 tiles 2 to 4 %.)
     constexpr unsigned long long kOff = 1ull << 32;
-    const bool full = g.vec_a && g.vec_b && g.vec_c && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0 && g.K > 0 &&
+    const bool full = g.vec_a && g.vec_b && g.vec_c && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0 &&
                       (!A_KC || (unsigned long long)g.M * (unsigned)g.lda < kOff) &&
                       (!B_KC || (unsigned long long)g.N * (unsigned)g.ldb < kOff);
     if (full) gemm_tile<BT, A_KC, B_KC, true>(g);
@@ -407,8 +408,8 @@ DEVI void gemm_split_tile(const GemmArgs &g, char *smem) {
 template <int BT, bool A_KC, bool B_KC>
 DEVI void gemm_split_body(const GemmArgs &g) {
     __shared__ __attribute__((aligned(16))) char smem[slab_bytes<BT, A_KC>() + slab_bytes<BT, B_KC>() + 16];
-    // Workgroup-uniform: every chunk inside its matrix, 16-byte rows (K = 0 has no slab to load, as in gemm_body).
-    const bool full = g.vec_a && g.vec_b && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0 && g.K > 0;
+    // Workgroup-uniform: every chunk inside its matrix, 16-byte rows (never K = 0, as in gemm_body).
+    const bool full = g.vec_a && g.vec_b && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0;
     if (full) gemm_split_tile<BT, A_KC, B_KC, true>(g, smem);
     else if constexpr (BT == 128) gemm_split_tile<BT, A_KC, B_KC, false>(g, smem);
     else gemm_tile<BT, A_KC, B_KC, false>(g);

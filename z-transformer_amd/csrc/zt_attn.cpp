@@ -1664,8 +1664,10 @@ static int gemm_impl(const char *name, const char *what, const float *a, int lda
     g.M = M; g.N = N; g.K = K;
     g.lda = lda; g.ldb = ldb; g.ldc = ldc;
     g.accumulate = accumulate;
-    g.vec_a = lda % 4 == 0 && (uintptr_t)a % 16 == 0;
-    g.vec_b = ldb % 4 == 0 && (uintptr_t)b % 16 == 0;
+    // K = 0: A and B may be null, and the whole-tile loaders, which read a first slab
+    // unconditionally, need vec_a and vec_b; the guarded ones then read nothing.
+    g.vec_a = K > 0 && lda % 4 == 0 && (uintptr_t)a % 16 == 0;
+    g.vec_b = K > 0 && ldb % 4 == 0 && (uintptr_t)b % 16 == 0;
     g.vec_c = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
     // The f32 MFMA form of the weight gradient (..f) where splitting the slabs is not
     // paid back (us, f32 / split, M x N x K): few slabs, 4096 x 4096 x 128 55.6 / 60.6 (x 250
