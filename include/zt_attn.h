@@ -283,11 +283,15 @@ int zt_weight_grad(float *w, const float *input, const float *dout, int T, int I
 /* src/autograd.zig:999-1022 (inputGrad): din[T,I] += dout[T,J] w[I,J]^T. */
 int zt_input_grad(float *din, const float *dout, const float *w, int T, int J, int I, hipStream_t stream);
 /* The kernel zt_matmul launches for an M x K x N product on the current device
- * ("zt_gemm_nn_<tile>" slab kernel or "zt_gemm_nn_sk<tile>" split-K kernel;
- * the two gradients take the same choice for the same output shape and
- * reduction length), into name[len].  0, or 1 if there is no usable device,
+ * ("zt_gemm_nn_<tile>" slab kernel, an f after the tile naming the f32 MFMA form of
+ * one that also has a split-operand form, or "zt_gemm_nn_sk<tile>" split-K kernel;
+ * 16-byte aligned operands), into name[len].  0, or 1 if there is no usable device,
  * the shape is empty or name is too short.  No reference counterpart. */
 int zt_matmul_plan(int M, int K, int N, char *name, int len);
+/* The same for any of the three products over K: 0 zt_matmul (M, K, N), 1
+ * zt_weight_grad ("zt_gemm_tn_..": M = I, K = T, N = J), 2 zt_input_grad
+ * ("zt_gemm_nt_..": M = T, K = J, N = I).  No reference counterpart. */
+int zt_product_plan(int product, int M, int K, int N, char *name, int len);
 
 /* Roofline calibration (no reference counterpart): the FP32 MFMA rate this
  * device sustains (two interleaved v_mfma_f32_16x16x4_f32 chains per wave,
@@ -341,7 +345,9 @@ int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_til
  *   none), ZT_ATTN_FSHAPE 11|12|14|21|22 (the forward's wave shape on split
  *   operands, 16-row blocks per wave then key parts; one the kernel does not
  *   hold falls back to one it does), ZT_ATTN_BSHAPE 1|2|4 (16-key blocks per
- *   workgroup of the score-reading dk/dv kernel, head_dim <= 128).
+ *   workgroup of the score-reading dk/dv kernel, head_dim <= 128), ZT_GEMM_SPLIT
+ *   0|1 (the f32 or split-operand form of a dense product's slab tile; a form
+ *   the tile does not have falls back to the one it has).
  * Returns 0, or 1 (reason on stderr) for an unknown name or value.  The
  * process environment is never read.  Not synchronised with launches in
  * flight on other threads: set before launching. */

@@ -195,3 +195,40 @@ def test_an_empty_contraction_reads_nothing(gpu, zt, op, M, N):
         zt.input_grad(c, empty, empty, M, 0, N)
     gpu.cuda.synchronize()
     assert gpu.equal(c, gpu.zeros_like(c) if op == "nn" else before)
+
+
+# Both sides of every line of the rule (a 256-CU device), whole and ragged.
+FORMS = [
+    ("nn", 1024, 64, 4096, "128"), ("nn", 1024, 256, 2048, "64"),
+    ("tn", 4096, 191, 2048, "128f"), ("tn", 4096, 192, 2048, "128"), ("tn", 2048, 2016, 2048, "128f"),
+    ("tn", 2048, 2080, 2048, "128"), ("tn", 1024, 32, 2048, "64"), ("tn", 1600, 128, 2048, "64"),
+    ("tn", 1600, 130, 2048, "64f"), ("tn", 1030, 256, 2040, "64f"),
+    ("nt", 1000, 64, 4096, "128"), ("nt", 1024, 64, 2048, "64"), ("nt", 1536, 256, 2048, "64"),
+    ("nt", 777, 128, 4096, "64f"), ("nt", 777, 100, 4096, "64f"), ("nt", 1024, 96, 2046, "64f"),
+]
+
+
+@pytest.mark.parametrize("op,M,K,N,form", FORMS)
+def test_the_form_the_rule_picks_passes_the_gate(gpu, zt, op, M, K, N, form):
+    """The f32 and the split form of each slab tile, unforced: the kernel the
+    rule names, and its result.  (Ragged 64 tiles never take the split kernel,
+    whose LDS would halve the f32 form's waves.)"""
+    assert zt.gemm_kernel(M, K, N, op) == f"zt_gemm_{op}_{form}"
+    gen = gpu.Generator(device="cuda").manual_seed(M + K)
+    a, b = (gpu.rand(s, device="cuda", generator=gen) * 2 - 1 for s in ((M, K), (K, N)))
+    c0 = gpu.rand(M, N, device="cuda", generator=gen) * 2 - 1
+    c = c0.clone().view(-1)
+    aa = (a.t() if op == "tn" else a).contiguous().view(-1)
+    bb = (b.t() if op == "nt" else b).contiguous().view(-1)
+    if op == "nn":
+        zt.matmul(aa, bb, c, M, K, N)
+        c0.zero_()
+    elif op == "tn":
+        zt.weight_grad(c, aa, bb, K, M, N)
+    else:
+        zt.input_grad(c, aa, bb, M, K, N)
+    gpu.cuda.synchronize()
+    exact, abs_sum = c0.double() + a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    # _divergence's gate: a rounding of each of the K products and sums, and of the add into C.
+    err = (c.view(M, N).double() - exact).abs() / gpu.maximum(abs_sum + c0.abs(), gpu.ones_like(abs_sum))
+    assert float(err.max()) < K * EPS32

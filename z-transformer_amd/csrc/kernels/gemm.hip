@@ -401,18 +401,20 @@ DEVI void gemm_split_tile(const GemmArgs &g, char *smem) {
             }
         }
 }
-// The 64-tile takes the split only for whole tiles (2048 x 4096 x 1024: weightGrad
-// 150 -> 134 us, inputGrad 161 -> 128 us; ragged 1000^3 would lose, 42 -> 47 us and 36
-// -> 45 us), and zt_gemm_nn_64 not at all (142 -> 174 us): its staging is shared by
-// half as many products.
+// The gradients' 64 tiles have the split for whole tiles only, where the launcher
+// picks it (1536 x 2048 x 2048, M x N x K: weightGrad 118 -> 105 us, inputGrad 123 -> 104
+// us): ragged tiles lose (1000^3 42 -> 47 us and 36 -> 45 us), and zt_gemm_nn_64 has
+// none (142 -> 174 us): its staging is shared by half as many products.  The f32 form
+// of a ragged product is a kernel of its own, for the LDS: one kernel with both takes
+// both their slabs', 55 KB and not 37 (ragged 3000 x 1024 x 4096 360 us for 265, and
+// the whole 1536 x 2048 x 2048 131 us).
 template <int BT, bool A_KC, bool B_KC>
 DEVI void gemm_split_body(const GemmArgs &g) {
     __shared__ __attribute__((aligned(16))) char smem[slab_bytes<BT, A_KC>() + slab_bytes<BT, B_KC>() + 16];
     // Workgroup-uniform: every chunk inside its matrix, 16-byte rows (never K = 0, as in gemm_body).
-    const bool full = g.vec_a && g.vec_b && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0;
+    const bool full = BT == 64 || (g.vec_a && g.vec_b && g.M % BT == 0 && g.N % BT == 0 && g.K % BK == 0);
     if (full) gemm_split_tile<BT, A_KC, B_KC, true>(g, smem);
     else if constexpr (BT == 128) gemm_split_tile<BT, A_KC, B_KC, false>(g, smem);
-    else gemm_tile<BT, A_KC, B_KC, false>(g);
 }
 
 // Split-K variant for products too small to fill the device with slab tiles
@@ -870,22 +872,22 @@ DEVI void dq_ds_body(const DqDsArgs &g) {
 
 }  // namespace
 
-// Kernel names: zt_gemm_<op>_<tile>.
+// Kernel names: zt_gemm_<op>_<tile>; with an f, the f32 MFMA form of a tile that also
+// has a split one (zt_attn.cpp, gemm_plan, picks).
 #define ZT_GEMM(BT)                                                                                \
     extern "C" __global__ void __launch_bounds__(256) zt_gemm_nn_##BT(GemmArgs g) { gemm_body<BT, true, false>(g); } \
     extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_##BT(GemmArgs g) { gemm_body<BT, false, false>(g); } \
     extern "C" __global__ void __launch_bounds__(256) zt_gemm_nt_##BT(GemmArgs g) { gemm_body<BT, true, true>(g); }
 
-
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nn_128(GemmArgs g) { gemm_split_body<128, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_128(GemmArgs g) { gemm_split_body<128, false, false>(g); }
-// f32 MFMA forms, for the products where the split loses (zt_attn.cpp, gemm_impl).
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_128f(GemmArgs g) { gemm_body<128, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_64f(GemmArgs g) { gemm_body<64, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_128(GemmArgs g) { gemm_split_body<128, true, true>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_nn_64(GemmArgs g) { gemm_body<64, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_64(GemmArgs g) { gemm_split_body<64, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_64(GemmArgs g) { gemm_split_body<64, true, true>(g); }
+extern "C" __global__ void __launch_bounds__(256) zt_gemm_nt_64f(GemmArgs g) { gemm_body<64, true, true>(g); }
 ZT_GEMM(32)
 
 // Split-K kernels: zt_gemm_<op>_sk<16 TW>, 64 NW threads (NW = 4, 8 or 16).

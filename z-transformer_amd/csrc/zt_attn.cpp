@@ -166,7 +166,7 @@ int launch(DeviceState *st, const char *name, unsigned blocks, const Args &args,
 enum Tune {
     kTuneBK, kTuneFwdW, kTuneFPF, kTuneFPair, kTuneQPF, kTuneDqW, kTuneHS, kTuneW8, kTunePF, kTuneDMA, kTuneBPair,
     kTuneDSplit, kTuneRSplit, kTuneDecWgs, kTuneGemmTile, kTuneGemmSk, kTuneGemmSkTile, kTuneDqdsTile, kTuneRowG,
-    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneFShape, kTuneBShape, kTuneCount
+    kTuneRowW, kTuneFKS, kTuneDqdsK, kTuneRScores, kTuneFShape, kTuneBShape, kTuneGemmSplit, kTuneCount
 };
 struct TuneSpec {
     const char *name;
@@ -199,6 +199,7 @@ const TuneSpec kTuneSpecs[kTuneCount] = {
     {"ZT_ATTN_RSCORES", {0, 1}, 2},
     {"ZT_ATTN_FSHAPE", {11, 12, 14, 21, 22}, 5},
     {"ZT_ATTN_BSHAPE", {1, 2, 4}, 3},
+    {"ZT_GEMM_SPLIT", {0, 1}, 2},
 };
 std::atomic<int> g_tune[kTuneCount] = {};  // 0 = unset (no allowed value is 0 except a flag, stored as value + 1)
 
@@ -1636,8 +1637,42 @@ static void gemm_choose(int M, int N, int K, int n_cus, int *bt_out, int *sk_out
     *sk_out = sk;
 }
 
-// C (+)= op(A) op(B) with the kernel variant `name` (see gemm.hip).
-static int gemm_impl(const char *name, const char *what, const float *a, int lda, const float *b, int ldb, float *c,
+// The three products: C = A B, C += A^T B, C += A B^T.
+enum class Product { NN, TN, NT };
+
+// Whether a 128 tile of the weight gradient takes the split form: it is not paid
+// back (us, f32 / split, M x N x K) on few slabs, 4096 x 4096 x 128 55.6 / 60.6 (x 250
+// 91.6 / 86.4), and with at most a workgroup per CU below 2048 deep, 4096 x 1024 x
+// 128 17.9 / 25.0, x 1024 80 / 84, x 1500 125 / 129.
+static bool gemm_split_pays(unsigned long long blocks, int K, unsigned long long cus) {
+    return K >= 192 && (blocks > cus || K >= 2048);
+}
+
+// The kernel of a product and its workgroups; aligned: both operands' rows on 16 bytes.
+struct GemmPlan {
+    char name[32];
+    unsigned long long blocks;
+    unsigned threads;
+};
+static GemmPlan gemm_plan(Product op, int M, int N, int K, bool aligned, int n_cus) {
+    GemmPlan p{};
+    int bt = 0, sk = 0;
+    gemm_choose(M, N, K, n_cus, &bt, &sk);
+    p.blocks = (unsigned long long)((M + bt - 1) / bt) * (unsigned long long)((N + bt - 1) / bt);
+    p.threads = sk ? 64u * (unsigned)sk : kThreads;
+    const char *kind = op == Product::NN ? "nn" : op == Product::TN ? "tn" : "nt";
+    // 128 tiles have the split form, the weight gradient's the f32 form too; the gradients' 64 tiles take the split where whole (in every shape measured,
+    // 1024 x 2048 x 64 to 1984 x 2048 x 4096: 1.0 to 1.2 times the f32 form), else f32.
+    const bool whole = aligned && M % bt == 0 && N % bt == 0 && K % 32 == 0 && K > 0;
+    const bool both = !sk && ((bt == 128 && op == Product::TN) || (bt == 64 && op != Product::NN));
+    const bool pays = bt == 64 ? whole : tuned(kTuneGemmTile, 0) != 0 || gemm_split_pays(p.blocks, K, n_cus);
+    const bool f32 = both && (tuned(kTuneGemmSplit, pays) == 0 || (bt == 64 && !whole));
+    snprintf(p.name, sizeof p.name, sk ? "zt_gemm_%s_sk%d" : f32 ? "zt_gemm_%s_%df" : "zt_gemm_%s_%d", kind, bt);
+    return p;
+}
+
+// C (+)= op(A) op(B) (see gemm.hip).
+static int gemm_impl(Product op, const char *what, const float *a, int lda, const float *b, int ldb, float *c,
                      int ldc, int M, int N, int K, int accumulate, hipStream_t stream) {
     if (M < 0 || N < 0 || K < 0) {
         fprintf(stderr, "%s: a %d x %d x %d product is not launchable.\n", what, M, N, K);
@@ -1653,12 +1688,6 @@ static int gemm_impl(const char *name, const char *what, const float *a, int lda
         fprintf(stderr, "%s: no usable gfx950 device or code object.\n", what);
         return 1;
     }
-    int bt = 0, sk = 0;
-    gemm_choose(M, N, K, st->cus, &bt, &sk);
-    auto tiles = [&](int t) { return (unsigned long long)((M + t - 1) / t) * (unsigned long long)((N + t - 1) / t); };
-    const unsigned long long blocks = tiles(bt);
-    const unsigned threads = sk ? 64u * (unsigned)sk : kThreads;
-    if (!grid_ok(blocks, threads)) return 1;
     GemmArgs g{};
     g.a = a; g.b = b; g.c = c;
     g.M = M; g.N = N; g.K = K;
@@ -1669,40 +1698,34 @@ static int gemm_impl(const char *name, const char *what, const float *a, int lda
     g.vec_a = K > 0 && lda % 4 == 0 && (uintptr_t)a % 16 == 0;
     g.vec_b = K > 0 && ldb % 4 == 0 && (uintptr_t)b % 16 == 0;
     g.vec_c = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
-    // The f32 MFMA form of the weight gradient (..f) where splitting the slabs is not
-    // paid back (us, f32 / split, M x N x K): few slabs, 4096 x 4096 x 128 55.6 / 60.6 (x 250
-    // 91.6 / 86.4); at most a workgroup per CU (or 64 tiles) below 2048 deep, 4096 x 1024 x
-    // 128 17.9 / 25.0, x 1024 80 / 84, x 1500 125 / 129 (x 2048 150 / 134).
-    const bool tn = strcmp(name, "zt_gemm_tn") == 0;
-    const bool whole64 = g.vec_a && g.vec_b && M % 64 == 0 && N % 64 == 0 && K % 32 == 0;
-    const bool f32 = tn && !sk && tuned(kTuneGemmTile, 0) == 0 &&
-                     ((bt == 64 && !(whole64 && K >= 2048)) ||
-                      (bt == 128 && (K < 192 || (blocks <= (unsigned long long)st->cus && K < 2048))));
-    char kname[32];
-    snprintf(kname, sizeof kname, sk ? "%s_sk%d" : f32 ? "%s_%df" : "%s_%d", name, bt);
-    return launch(st, kname, (unsigned)blocks, g, stream, threads);
+    const GemmPlan p = gemm_plan(op, M, N, K, g.vec_a && g.vec_b, st->cus);
+    if (!grid_ok(p.blocks, p.threads)) return 1;
+    return launch(st, p.name, (unsigned)p.blocks, g, stream, p.threads);
 }
 
 int zt_matmul(const float *a, const float *b, float *out, int M, int K, int N, hipStream_t stream) {
-    return gemm_impl("zt_gemm_nn", "zt_matmul", a, K, b, N, out, N, M, N, K, 0, stream);
+    return gemm_impl(Product::NN, "zt_matmul", a, K, b, N, out, N, M, N, K, 0, stream);
 }
 
 int zt_weight_grad(float *w, const float *input, const float *dout, int T, int I, int J, hipStream_t stream) {
-    return gemm_impl("zt_gemm_tn", "zt_weight_grad", input, I, dout, J, w, J, I, J, T, 1, stream);
+    return gemm_impl(Product::TN, "zt_weight_grad", input, I, dout, J, w, J, I, J, T, 1, stream);
 }
 
 int zt_input_grad(float *din, const float *dout, const float *w, int T, int J, int I, hipStream_t stream) {
-    return gemm_impl("zt_gemm_nt", "zt_input_grad", dout, J, w, J, din, I, T, I, J, 1, stream);
+    return gemm_impl(Product::NT, "zt_input_grad", dout, J, w, J, din, I, T, I, J, 1, stream);
 }
 
-int zt_matmul_plan(int M, int K, int N, char *name, int len) {
+int zt_product_plan(int product, int M, int K, int N, char *name, int len) {
     DeviceState *st = device_state();
-    if (!st || !name || len < 1 || M < 1 || N < 1 || K < 0) return 1;
-    int bt = 0, sk = 0;
-    gemm_choose(M, N, K, st->cus, &bt, &sk);
-    const int n = sk ? snprintf(name, (size_t)len, "zt_gemm_nn_sk%d", bt) : snprintf(name, (size_t)len, "zt_gemm_nn_%d", bt);
+    if (!st || !name || len < 1 || product < 0 || product > 2 || M < 1 || N < 1 || K < 0) return 1;
+    const Product op = static_cast<Product>(product);
+    // Row lengths of the stored operands: M x K and K x N, K x M and K x N, M x K and N x K.
+    const int lda = op == Product::TN ? M : K, ldb = op == Product::NT ? K : N;
+    const GemmPlan p = gemm_plan(op, M, N, K, lda % 4 == 0 && ldb % 4 == 0, st->cus);
+    const int n = snprintf(name, (size_t)len, "%s", p.name);
     return n < 0 || n >= len;
 }
+int zt_matmul_plan(int M, int K, int N, char *name, int len) { return zt_product_plan(0, M, K, N, name, len); }
 
 int zt_attn_set_tuning(const char *name, int value) {
     for (int i = 0; name && i < kTuneCount; ++i) {

@@ -26,7 +26,7 @@ ABI_SYMBOLS = [
     "zt_attn_bwd_dq_train", "zt_attn_bwd_dkdv_train", "zt_attn_plan_train", "zt_calibrate",
     "zt_matmul", "zt_weight_grad", "zt_input_grad", "zt_attn_backward_train_workspace",
     "zt_attn_backward_train_ws", "zt_attn_forward_train_ws", "zt_attn_set_tuning", "zt_attn_get_tuning",
-    "zt_calibrate_launch", "zt_attn_decode_noalloc", "zt_matmul_plan",
+    "zt_calibrate_launch", "zt_attn_decode_noalloc", "zt_matmul_plan", "zt_product_plan",
 ]
 HOLDER_SYMBOLS = [
     "zt_bytes_for", "zt_to_cint", "zt_forward_bounds", "zt_holder_init", "zt_holder_deinit",
@@ -92,6 +92,7 @@ def load_library(path):
         "zt_weight_grad": (I, [P, P, P, I, I, I, P]),
         "zt_input_grad": (I, [P, P, P, I, I, I, P]),
         "zt_matmul_plan": (I, [I, I, I, P, I]),
+        "zt_product_plan": (I, [I, I, I, I, P, I]),
         "zt_calibrate": (I, [P, Z, P, Z, P, P, P]),
         "zt_calibrate_launch": (I, [ctypes.c_uint, ctypes.c_uint, I, P, P]),
         "zt_rope_forward": (I, [P, P, I, I, I, D, I, P]),
@@ -333,10 +334,10 @@ def matmul(a, b, out, M, K, N, stream=None):
     _check(lib().zt_matmul(_ptr(a), _ptr(b), _ptr(out), M, K, N, _stream(stream)), "zt_matmul")
 
 
-def gemm_kernel(M, K, N):
-    """The kernel zt_matmul launches for an M x K x N product."""
+def gemm_kernel(M, K, N, product="nn"):
+    """The kernel zt_matmul ("nn"), zt_weight_grad ("tn") or zt_input_grad ("nt") launches for an M x N result over K."""
     buf = ctypes.create_string_buffer(64)
-    _check(lib().zt_matmul_plan(M, K, N, buf, 64), "zt_matmul_plan")
+    _check(lib().zt_product_plan(("nn", "tn", "nt").index(product), M, K, N, buf, 64), "zt_product_plan")
     return buf.value.decode()
 
 
