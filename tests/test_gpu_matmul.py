@@ -199,8 +199,10 @@ def test_an_empty_contraction_reads_nothing(gpu, zt, op, M, N):
 
 # Both sides of every line of the rule (a 256-CU device), whole and ragged.
 FORMS = [
-    ("nn", 1024, 64, 4096, "128"), ("nn", 1024, 256, 2048, "64"),
-    ("tn", 4096, 191, 2048, "128f"), ("tn", 4096, 192, 2048, "128"), ("tn", 2048, 2016, 2048, "128f"),
+    ("nn", 1000, 64, 4096, "128f"), ("nn", 1000, 383, 4096, "128f"), ("nn", 1000, 384, 4096, "128"),
+    ("nn", 1024, 64, 4096, "128"), ("nn", 2048, 32, 4096, "128"), ("nn", 4096, 32, 4096, "128f"),
+    ("nn", 4096, 33, 4096, "128"), ("nn", 1024, 256, 2048, "64"),
+    ("tn", 4096, 191, 2048, "128f"), ("tn", 4096, 192, 2048, "128"), ("tn", 2048, 2048, 2048, "128f"),
     ("tn", 2048, 2080, 2048, "128"), ("tn", 1024, 32, 2048, "64"), ("tn", 1600, 128, 2048, "64"),
     ("tn", 1600, 130, 2048, "64f"), ("tn", 1030, 256, 2040, "64f"),
     ("nt", 1000, 64, 4096, "128"), ("nt", 1024, 64, 2048, "64"), ("nt", 1536, 256, 2048, "64"),

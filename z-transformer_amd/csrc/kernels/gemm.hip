@@ -881,6 +881,7 @@ DEVI void dq_ds_body(const DqDsArgs &g) {
 
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nn_128(GemmArgs g) { gemm_split_body<128, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_tn_128(GemmArgs g) { gemm_split_body<128, false, false>(g); }
+extern "C" __global__ void __launch_bounds__(256) zt_gemm_nn_128f(GemmArgs g) { gemm_body<128, true, false>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_128f(GemmArgs g) { gemm_body<128, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256) zt_gemm_tn_64f(GemmArgs g) { gemm_body<64, false, false>(g); }
 extern "C" __global__ void __launch_bounds__(256, 2) zt_gemm_nt_128(GemmArgs g) { gemm_split_body<128, true, true>(g); }

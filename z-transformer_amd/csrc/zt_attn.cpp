@@ -1640,12 +1640,18 @@ static void gemm_choose(int M, int N, int K, int n_cus, int *bt_out, int *sk_out
 // The three products: C = A B, C += A^T B, C += A B^T.
 enum class Product { NN, TN, NT };
 
-// Whether a 128 tile of the weight gradient takes the split form: it is not paid
-// back (us, f32 / split, M x N x K) on few slabs, 4096 x 4096 x 128 55.6 / 60.6 (x 250
-// 91.6 / 86.4), and with at most a workgroup per CU below 2048 deep, 4096 x 1024 x
-// 128 17.9 / 25.0, x 1024 80 / 84, x 1500 125 / 129.
-static bool gemm_split_pays(unsigned long long blocks, int K, unsigned long long cus) {
-    return K >= 192 && (blocks > cus || K >= 2048);
+// Whether a 128 tile takes the split form (see gemm.hip) where it has both.  The
+// split's staging costs more per slab, so it must be shared by enough products and
+// workgroups; measured on MI355X, us, f32 form / split, M x N x K:
+//  - weight gradient: few slabs 4096 x 4096 x 128 55.0 / 60.1 (x 192 70.7 / 70.8, x 256
+//    86.9 / 81.9); at most a workgroup per CU, 1024 x 4096 x 128 16.9 / 20.7, x 1024 80.0 /
+//    84.6, x 1536 114.4 / 117.7, x 2048 149.6 / 150.5 (x 3072 219.4 / 217.1).
+//  - matmul: ragged with at most a workgroup per CU, 1000 x 4096 x 128 16.3 / 17.1 (x 384
+//    36.6 / 36.8; whole 1024 x 4096 x 128 14.7 / 14.4); one slab and many tiles,
+//    4096 x 4096 x 32 18.7 / 21.1 (2048 x 4096 x 32 11.9 / 10.4).
+static bool gemm_split_pays(Product op, bool whole, unsigned long long blocks, int K, unsigned long long cus) {
+    if (op == Product::TN) return K >= 192 && (blocks > cus || K > 2048);
+    return !(blocks <= cus && !whole && K < 384) && !(blocks > 3 * cus && K <= 32);
 }
 
 // The kernel of a product and its workgroups; aligned: both operands' rows on 16 bytes.
@@ -1661,11 +1667,12 @@ static GemmPlan gemm_plan(Product op, int M, int N, int K, bool aligned, int n_c
     p.blocks = (unsigned long long)((M + bt - 1) / bt) * (unsigned long long)((N + bt - 1) / bt);
     p.threads = sk ? 64u * (unsigned)sk : kThreads;
     const char *kind = op == Product::NN ? "nn" : op == Product::TN ? "tn" : "nt";
-    // 128 tiles have the split form, the weight gradient's the f32 form too; the gradients' 64 tiles take the split where whole (in every shape measured,
+    // 128 tiles have the split form, matmul's and the weight gradient's the f32 form
+    // too; the gradients' 64 tiles take the split where whole (in every shape measured,
     // 1024 x 2048 x 64 to 1984 x 2048 x 4096: 1.0 to 1.2 times the f32 form), else f32.
     const bool whole = aligned && M % bt == 0 && N % bt == 0 && K % 32 == 0 && K > 0;
-    const bool both = !sk && ((bt == 128 && op == Product::TN) || (bt == 64 && op != Product::NN));
-    const bool pays = bt == 64 ? whole : tuned(kTuneGemmTile, 0) != 0 || gemm_split_pays(p.blocks, K, n_cus);
+    const bool both = !sk && ((bt == 128 && op != Product::NT) || (bt == 64 && op != Product::NN));
+    const bool pays = bt == 64 ? whole : tuned(kTuneGemmTile, 0) != 0 || gemm_split_pays(op, whole, p.blocks, K, n_cus);
     const bool f32 = both && (tuned(kTuneGemmSplit, pays) == 0 || (bt == 64 && !whole));
     snprintf(p.name, sizeof p.name, sk ? "zt_gemm_%s_sk%d" : f32 ? "zt_gemm_%s_%df" : "zt_gemm_%s_%d", kind, bt);
     return p;
