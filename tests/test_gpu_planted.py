@@ -102,6 +102,20 @@ def test_forward_gate_rejects_every_planted_forward(gpu, zt, oracle, planted, in
         assert err > FWD_TOL, name
 
 
+@pytest.mark.parametrize("shape", [11, 12, 14, 21, 22])
+def test_a_planted_forward_holds_every_wave_shape_the_launcher_picks(gpu, planted, inputs, shape):
+    """The launcher knows one table of shapes: a kernel without the one asked for
+    would return with its output unwritten."""
+    q, k, v, _ = inputs
+    for name in FWD_PLANTS:
+        L = planted[name]
+        assert L.zt_attn_set_tuning(b"ZT_ATTN_FSHAPE", shape) == 0
+        try:
+            assert not np.isnan(_forward(gpu, L, q, k, v)).any(), name
+        finally:
+            L.zt_attn_set_tuning(b"ZT_ATTN_FSHAPE", -1)
+
+
 def test_backward_gate_rejects_every_planted_backward_with_its_own_signature(gpu, zt, oracle, planted, inputs):
     q, k, v, do = inputs
     want = oracle.attention_backward(*(host(x) for x in (q, k, v, do)), B, T, H, Hkv, D)

@@ -1305,10 +1305,11 @@ __device__ __forceinline__ void bwd_dkdv_dma_body(const BwdArgs &a) {
 template <int DP, int NPART, int NKB>
 struct BwdSplit {
     static constexpr int NW = NPART * NKB, NT = DP / 16, NKS = DP / 32;
-    static constexpr int TILE = split_bytes<DP>(32);
+    static constexpr int TILE = split_bytes(DP, 32);
     static constexpr int STATS = NPART * 2 * TILE;         // lse log2(e), -delta of the 32 rows, per part
     static constexpr int FLAGS = STATS + NPART * 64 * 4;   // step ids whose dO (Q) tile holds a big value, per part
-    static constexpr int BYTES = FLAGS + NPART * 8;
+    static constexpr int BYTES = dkdv_lds(DP, {NPART, NKB});
+    static_assert(BYTES == FLAGS + NPART * 8, "LDS layout");
     static_assert((NPART - 1) * NKB * 64 * 2 * NT * 16 <= STATS, "the parts merge in the tiles' space");
     static_assert(BYTES <= 160 * 1024, "LDS");
 };
@@ -1618,42 +1619,35 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
     __syncthreads();  // the merge's reads before the next tile's staging
 }
 
-// Shapes (NPART, NKB) of one kernel, picked by the launch (BwdArgs::parts, kblocks).
+// One of a kernel's shapes (shapes.h), picked by the launch (BwdArgs::parts, kblocks).
 template <int DP, int NPART, int NKB>
-struct BwdShape {
-    static constexpr int BYTES = BwdSplit<DP, NPART, NKB>::BYTES;
-    DEVI static bool run(const BwdArgs &a, char *smem) {
-        if (a.parts != NPART || a.kblocks != NKB) return false;  // workgroup-uniform
-        if (threadIdx.x < 2 * NPART) reinterpret_cast<int *>(smem + BwdSplit<DP, NPART, NKB>::FLAGS)[threadIdx.x] = 0;
-        __syncthreads();
-        const int per = a.Hkv * a.B, rem = (int)blockIdx.x % per, p = (int)blockIdx.x / per;
-        const int kvh = rem % a.Hkv, b = rem / a.Hkv;
-        int sid = 0, kt = p;
-        const int second = a.n_key_tiles - 1 - p;
+DEVI bool dkdv_shape(const BwdArgs &a, char *smem) {
+    if (a.parts != NPART || a.kblocks != NKB) return false;  // workgroup-uniform
+    if (threadIdx.x < 2 * NPART) reinterpret_cast<int *>(smem + BwdSplit<DP, NPART, NKB>::FLAGS)[threadIdx.x] = 0;
+    __syncthreads();
+    const int per = a.Hkv * a.B, rem = (int)blockIdx.x % per, p = (int)blockIdx.x / per;
+    const int kvh = rem % a.Hkv, b = rem / a.Hkv;
+    int sid = 0, kt = p;
+    const int second = a.n_key_tiles - 1 - p;
 #pragma unroll 1
-        for (;;) {
-            dkdv_split_tile<DP, NPART, NKB>(a, kt, kvh, b, smem, sid);
-            ++sid;  // (ids of one tile's last staging are not met by the next's)
-            if (!a.pair || kt == second || second <= p) break;
-            kt = second;
-        }
-        return true;
+    for (;;) {
+        dkdv_split_tile<DP, NPART, NKB>(a, kt, kvh, b, smem, sid);
+        ++sid;  // (ids of one tile's last staging are not met by the next's)
+        if (!a.pair || kt == second || second <= p) break;
+        kt = second;
     }
-};
-template <class... S>
-constexpr int bwd_shapes_bytes() {
-    int m = 0;
-    ((m = S::BYTES > m ? S::BYTES : m), ...);
-    return m;
+    return true;
 }
-template <class... S>
-DEVI void bwd_shapes(const BwdArgs &a) {
-    __shared__ __attribute__((aligned(16))) char smem[bwd_shapes_bytes<S...>()];
-    (void)(S::run(a, smem) || ...);
+template <int DP>
+DEVI void dkdv_shapes(const BwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds(DP)];
+    constexpr BwdWavesList L = dkdv_waves(DP);
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (void)(dkdv_shape<DP, L.s[I].parts, L.s[I].kblocks>(a, smem) || ...);
+    }(std::make_integer_sequence<int, L.n>{});
 }
-#define ZT_BWD_SPLIT(NAME, ...)                                                                      \
-    extern "C" __global__ void __launch_bounds__(512, 2) NAME(BwdArgs a) { bwd_shapes<__VA_ARGS__>(a); }
-#define BS(DP, NPART, NKB) BwdShape<DP, NPART, NKB>
+#define ZT_BWD_SPLIT(NAME, DP)                                                                      \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME(BwdArgs a) { dkdv_shapes<DP>(a); }
 
 #define ZT_BWD_DQ(DP, BK)                                                                          \
     extern "C" __global__ void __launch_bounds__(256, (DP) <= ((BK) == 32 ? 192 : 128) ? 2 : 1)  \
@@ -1690,13 +1684,9 @@ DEVI void bwd_shapes(const BwdArgs &a) {
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8p_d##DP##_hs2(BwdArgs a) {    \
         bwd_dkdv_body<DP, 2, 4, true>(a);                                                          \
     }
-// dk/dv that reads the forward's scores, on split operands: one list of shapes
-// per width under two names, for head groups of two and more (dkdv8s) and for
-// one that cannot be halved (dmars).
-#define ZT_BWD_SPLIT_32(NAME) ZT_BWD_SPLIT(NAME, BS(32, 2, 4), BS(32, 4, 2), BS(32, 8, 1))
-#define ZT_BWD_SPLIT_64(NAME) ZT_BWD_SPLIT(NAME, BS(64, 2, 4), BS(64, 4, 2), BS(64, 4, 1))
-#define ZT_BWD_SPLIT_96(NAME) ZT_BWD_SPLIT(NAME, BS(96, 2, 4), BS(96, 2, 2))
-#define ZT_BWD_SPLIT_128(NAME) ZT_BWD_SPLIT(NAME, BS(128, 2, 4), BS(128, 2, 2))
+// dk/dv that reads the forward's scores, on split operands: one kernel under two
+// names, for head groups of two and more (dkdv8s) and for one that cannot be halved
+// (dmars), so that a profile tells the two apart.
 #define ZT_BWD_DKDV_DMA(DP, HS)                                                                    \
     extern "C" __global__ void __launch_bounds__(256) zt_bwd_dkdv_dma_d##DP##_hs##HS(BwdArgs a) { \
         bwd_dkdv_dma_body<DP, HS>(a);                                                              \
@@ -1715,10 +1705,10 @@ ZT_BWD_ALL(32)
 ZT_BWD_ALL(64)
 ZT_BWD_ALL(96)
 ZT_BWD_ALL(128)
-ZT_BWD_SPLIT_32(zt_bwd_dkdv8s_d32_hs2)
-ZT_BWD_SPLIT_64(zt_bwd_dkdv8s_d64_hs2)
-ZT_BWD_SPLIT_96(zt_bwd_dkdv8s_d96_hs2)
-ZT_BWD_SPLIT_128(zt_bwd_dkdv8s_d128_hs2)
+ZT_BWD_SPLIT(zt_bwd_dkdv8s_d32_hs2, 32)
+ZT_BWD_SPLIT(zt_bwd_dkdv8s_d64_hs2, 64)
+ZT_BWD_SPLIT(zt_bwd_dkdv8s_d96_hs2, 96)
+ZT_BWD_SPLIT(zt_bwd_dkdv8s_d128_hs2, 128)
 // The 4-way splits: the 160 KB LDS holds 4 parts' tiles (double-buffered for
 // the asynchronous variant) up to d = 128.
 ZT_BWD_DKDV(32, 4)
@@ -1733,10 +1723,10 @@ ZT_BWD_DKDV(128, 4)
     }
 ZT_BWD_DKDV_DMAR(32) ZT_BWD_DKDV_DMAR(64) ZT_BWD_DKDV_DMAR(96) ZT_BWD_DKDV_DMAR(128)
 // The same reading the forward's scores.
-ZT_BWD_SPLIT_32(zt_bwd_dkdv_dmars_d32)
-ZT_BWD_SPLIT_64(zt_bwd_dkdv_dmars_d64)
-ZT_BWD_SPLIT_96(zt_bwd_dkdv_dmars_d96)
-ZT_BWD_SPLIT_128(zt_bwd_dkdv_dmars_d128)
+ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d32, 32)
+ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d64, 64)
+ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d96, 96)
+ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d128, 128)
 ZT_BWD_DKDV_DMA(32, 4)
 ZT_BWD_DKDV_DMA(64, 4)
 ZT_BWD_DKDV_DMA(96, 4)
@@ -1776,7 +1766,7 @@ ZT_BWD_DKDV8PD1(64) ZT_BWD_DKDV8PD1(128)
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
 ZT_BWD_DQ_PF(32) ZT_BWD_DQ_LSE(32) ZT_BWD_DKDV8(32)
-ZT_BWD_SPLIT_128(zt_bwd_dkdv8s_d128_hs2)
+ZT_BWD_SPLIT(zt_bwd_dkdv8s_d128_hs2, 128)
 #endif
 
 // delta[row] = sum_d o[row, d] * dout[row, d] over the B*T*H rows of dim

@@ -287,21 +287,22 @@ __device__ __forceinline__ void attn_fwd_body(const FwdArgs &a) {
 // products): 512 rows of that first shape 70 / 34 us.  Two row blocks per wave (NQ = 2) read each K and V
 // operand from LDS once for 32 rows: at one block the operand reads alone
 // (49 KB per wave and tile at d = 128) would take as long as the MFMAs.
-template <int DP, int DS, int NW, int NQ, int KS>
+template <int DP, int NW, int NQ, int KS>
 struct FwdSplit {
+    static constexpr FwdWaves W{NW, NQ, KS};
+    static constexpr int DS = fwd_ds(DP);   // column halves
     static constexpr int DW = DP / DS;      // columns per wave
     static constexpr int NT = DW / 16;      // 16-wide output tiles per wave
     static constexpr int NKS = DW / 32;     // 32-wide contraction steps of the score product
     static constexpr int ROWS = 32 * KS;    // keys staged per step
-    static constexpr int TILE = split_bytes<DP>(ROWS);
-    static constexpr int XCHG = DS > 1 ? NW * 2 * NQ * 1024 : 0;  // partial scores of the column halves
+    static constexpr int TILE = split_bytes(DP, ROWS);
     static constexpr int MERGE = (KS - 1) * (NW / KS) * 64 * (4 * NQ * NT + 2 * NQ) * 4;
     // Alternating wave halves (below): two buffers each for K and V.
-    static constexpr bool ALT = NW == 8 && DS == 1 && 4 * TILE + 16 <= 160 * 1024;
-    static constexpr int BUFS = ALT ? 2 : 1;
-    static constexpr int FLAGS = 2 * BUFS * TILE + XCHG;  // offset of the big-value flags
-    static constexpr int BYTES = FLAGS + 16;
-    static_assert(MERGE <= 2 * BUFS * TILE, "the key parts merge in the tiles' space");
+    static constexpr bool ALT = fwd_alt(DP, W);
+    static constexpr int XCHG = fwd_tiles_lds(DP, W);  // offset of the column halves' partial scores
+    static constexpr int BYTES = fwd_lds(DP, W);
+    static constexpr int FLAGS = BYTES - 16;           // offset of the big-value flags
+    static_assert(MERGE <= XCHG, "the key parts merge in the tiles' space");
     static_assert(BYTES <= 160 * 1024, "LDS");
 };
 
@@ -318,12 +319,12 @@ DEVI f4 quad_transpose(f4 x, int lane) {
     return f4{o2 ? y2 : a0, o2 ? y3 : a1, o2 ? a2 : y0, o2 ? a3 : y1};
 }
 
-template <int DP, int DS, int NW, int NQ, int KS, int SC>
+template <int DP, int NW, int NQ, int KS, int SC>
 DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int &sid) {
-    using C = FwdSplit<DP, DS, NW, NQ, KS>;
-    constexpr int DW = C::DW, NT = C::NT, NKS = C::NKS, ROWS = C::ROWS, NTH = 64 * NW, NWR = NW / (KS * DS);
+    using C = FwdSplit<DP, NW, NQ, KS>;
+    constexpr int DS = C::DS, DW = C::DW, NT = C::NT, NKS = C::NKS, ROWS = C::ROWS, NTH = 64 * NW, NWR = NW / (KS * DS);
     constexpr bool ALT = C::ALT;
-    char *const xchg = smem + 2 * C::BUFS * C::TILE;
+    char *const xchg = smem + C::XCHG;
     // The K (V) tile of a step, and the flag that holds the step's id if the tile has a big value.
     auto ktile = [&](int id) { return smem + (ALT ? (id & 1) * 2 * C::TILE : 0); };
     auto vtile = [&](int id) { return ktile(id) + C::TILE; };
@@ -737,10 +738,10 @@ DEVI void fwd_split_tile(const FwdArgs &a, const int tile, char *const smem, int
     }
 }
 
-template <int DP, int DS, int NW, int NQ, int KS, int SC>
+template <int DP, int NW, int NQ, int KS, int SC>
 DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
     const int p = (int)blockIdx.x / (a.n_head_blocks * a.B);
-    using C = FwdSplit<DP, DS, NW, NQ, KS>;
+    using C = FwdSplit<DP, NW, NQ, KS>;
     if (threadIdx.x < 4) reinterpret_cast<int *>(smem + C::FLAGS)[threadIdx.x] = 0;
     __syncthreads();
     int sid = 0;
@@ -749,7 +750,7 @@ DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
     int tile = second;
 #pragma unroll 1
     for (;;) {  // workgroup-uniform (every tile ends after a barrier)
-        fwd_split_tile<DP, DS, NW, NQ, KS, SC>(a, tile, smem, sid);
+        fwd_split_tile<DP, NW, NQ, KS, SC>(a, tile, smem, sid);
         if (!a.pair || tile == p || p >= second) break;
         tile = p;
     }
@@ -761,42 +762,28 @@ DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
     extern "C" __global__ void __launch_bounds__(512) zt_fwd8_d##DP##_k##BK(FwdArgs a) {         \
         attn_fwd_body<DP, BK, 8, false>(a);                                                        \
     }
-// Kernels on split operands: one per role and width, each holding the wave
-// shapes (NQ, KS) the launcher picks from by the grid (FwdArgs::nq, ks).
-template <int DP, int DS, int NW, int NQ, int KS, int SC>
-struct FwdShape {
-    static constexpr int BYTES = FwdSplit<DP, DS, NW, NQ, KS>::BYTES;
-    DEVI static bool run(const FwdArgs &a, char *smem) {
-        if (a.nq != NQ || a.ks != KS || blockDim.x != 64 * NW) return false;  // workgroup-uniform
-        fwd_split_body<DP, DS, NW, NQ, KS, SC>(a, smem);
-        return true;
-    }
-};
-template <class... S>
-constexpr int fwd_shapes_bytes() {
-    int m = 0;
-    ((m = S::BYTES > m ? S::BYTES : m), ...);
-    return m;
-}
-template <class... S>
-DEVI void fwd_shapes(const FwdArgs &a) {
-    __shared__ __attribute__((aligned(16))) char smem[fwd_shapes_bytes<S...>()];
-    (void)(S::run(a, smem) || ...);
-}
+// Kernels on split operands: one per role and width, each holding the role's wave
+// shapes (shapes.h), of which the launcher picks by the grid (FwdArgs::nq, ks).
 // SC: 0 never keeps the scores, 1 always, 2 where s_out is set.
-// Roles: several heads of a kv group per workgroup; the same keeping the scores
-// (its own name, so that a profile tells the two apart); one head per workgroup
-// (also four waves, where forced); one head per workgroup on small grids.
-#define ZT_FWD_P8(NAME, DP, ...)                                                                     \
+template <int DP, int SC, int NW, int NQ, int KS>
+DEVI bool fwd_shape(const FwdArgs &a, char *smem) {
+    if (a.nq != NQ || a.ks != KS || blockDim.x != 64 * NW) return false;  // workgroup-uniform
+    fwd_split_body<DP, NW, NQ, KS, SC>(a, smem);
+    return true;
+}
+template <FwdRole R, int DP, int SC>
+DEVI void fwd_shapes(const FwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[fwd_lds(R, DP)];
+    constexpr FwdWavesList L = fwd_waves(R, DP);
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (void)(fwd_shape<DP, SC, L.s[I].nw, L.s[I].nq, L.s[I].ks>(a, smem) || ...);
+    }(std::make_integer_sequence<int, L.n>{});
+}
+// zt_fwd8ps_* is zt_fwd8p_* keeping the scores: its own name, so that a profile tells the two apart.
+#define ZT_FWD_SPLIT(NAME, ROLE, DP, SC)                                                             \
     extern "C" __global__ void __launch_bounds__(512, 2) NAME##_d##DP##_k32(FwdArgs a) {          \
-        fwd_shapes<__VA_ARGS__>(a);                                                                  \
+        fwd_shapes<FwdRole::ROLE, DP, SC>(a);                                                        \
     }
-#define SH(...) FwdShape<__VA_ARGS__>
-#define ZT_FWD_SPLIT_8(NAME, SC)                                                                         \
-    ZT_FWD_P8(NAME, 32, SH(32, 1, 8, 2, 1, SC), SH(32, 1, 8, 2, 2, SC), SH(32, 1, 8, 1, 2, SC), SH(32, 1, 8, 1, 4, SC))                  \
-    ZT_FWD_P8(NAME, 64, SH(64, 1, 8, 2, 1, SC), SH(64, 1, 8, 2, 2, SC), SH(64, 1, 8, 1, 2, SC))                                      \
-    ZT_FWD_P8(NAME, 96, SH(96, 1, 8, 2, 1, SC), SH(96, 1, 8, 1, 2, SC))                                      \
-    ZT_FWD_P8(NAME, 128, SH(128, 1, 8, 2, 1, SC), SH(128, 1, 8, 1, 2, SC))
 
 // Register-prefetched variants on f32 MFMA (32-key tiles; widths whose halves
 // are not whole 32-column groups).
@@ -818,24 +805,19 @@ ZT_FWD(192, 32) ZT_FWD(192, 64)
 ZT_FWD(224, 32) ZT_FWD(224, 64)
 ZT_FWD(256, 32) ZT_FWD(256, 64)
 ZT_FWD_PF(160) ZT_FWD_PF(224)
-ZT_FWD_SPLIT_8(zt_fwd8p, 0)
-ZT_FWD_SPLIT_8(zt_fwd8ps, 1)
-ZT_FWD_P8(zt_fwd8p, 192, SH(192, 2, 8, 2, 1, 2), SH(192, 2, 8, 1, 1, 2))
-ZT_FWD_P8(zt_fwd8p, 256, SH(256, 2, 8, 2, 1, 2), SH(256, 2, 8, 1, 1, 2))
-ZT_FWD_P8(zt_fwdp, 32, SH(32, 1, 8, 2, 1, 2), SH(32, 1, 8, 2, 2, 2), SH(32, 1, 8, 1, 2, 2), SH(32, 1, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdp, 64, SH(64, 1, 8, 2, 1, 2), SH(64, 1, 8, 2, 2, 2), SH(64, 1, 8, 1, 2, 2), SH(64, 1, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdp, 96, SH(96, 1, 8, 2, 1, 2), SH(96, 1, 8, 1, 2, 2), SH(96, 1, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdp, 128, SH(128, 1, 8, 2, 1, 2), SH(128, 1, 8, 1, 2, 2), SH(128, 1, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdp, 192, SH(192, 2, 8, 2, 1, 2), SH(192, 2, 8, 1, 1, 2), SH(192, 2, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdp, 256, SH(256, 2, 8, 2, 1, 2), SH(256, 2, 8, 1, 1, 2), SH(256, 2, 4, 2, 1, 2))
-ZT_FWD_P8(zt_fwdpk, 32, SH(32, 1, 8, 1, 2, 2), SH(32, 1, 8, 1, 4, 2))
-ZT_FWD_P8(zt_fwdpk, 64, SH(64, 1, 8, 1, 2, 2), SH(64, 1, 8, 1, 4, 2))
-ZT_FWD_P8(zt_fwdpk, 96, SH(96, 1, 8, 1, 2, 2))
-ZT_FWD_P8(zt_fwdpk, 128, SH(128, 1, 8, 1, 2, 2))
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 32, 0) ZT_FWD_SPLIT(zt_fwd8p, Heads, 64, 0)
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 96, 0) ZT_FWD_SPLIT(zt_fwd8p, Heads, 128, 0)
+ZT_FWD_SPLIT(zt_fwd8ps, Heads, 32, 1) ZT_FWD_SPLIT(zt_fwd8ps, Heads, 64, 1)
+ZT_FWD_SPLIT(zt_fwd8ps, Heads, 96, 1) ZT_FWD_SPLIT(zt_fwd8ps, Heads, 128, 1)
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 192, 2) ZT_FWD_SPLIT(zt_fwd8p, Heads, 256, 2)
+ZT_FWD_SPLIT(zt_fwdp, One, 32, 2) ZT_FWD_SPLIT(zt_fwdp, One, 64, 2)
+ZT_FWD_SPLIT(zt_fwdp, One, 96, 2) ZT_FWD_SPLIT(zt_fwdp, One, 128, 2)
+ZT_FWD_SPLIT(zt_fwdp, One, 192, 2) ZT_FWD_SPLIT(zt_fwdp, One, 256, 2)
+ZT_FWD_SPLIT(zt_fwdpk, Small, 32, 2) ZT_FWD_SPLIT(zt_fwdpk, Small, 64, 2)
+ZT_FWD_SPLIT(zt_fwdpk, Small, 96, 2) ZT_FWD_SPLIT(zt_fwdpk, Small, 128, 2)
 #else
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
-ZT_FWD_P8(zt_fwd8p, 32, SH(32, 1, 8, 2, 1, 0), SH(32, 1, 8, 1, 2, 0), SH(32, 1, 8, 1, 4, 0))
-ZT_FWD_P8(zt_fwd8p, 128, SH(128, 1, 8, 2, 1, 0), SH(128, 1, 8, 1, 2, 0))
-ZT_FWD_P8(zt_fwd8ps, 128, SH(128, 1, 8, 2, 1, 1), SH(128, 1, 8, 1, 2, 1))
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 32, 0) ZT_FWD_SPLIT(zt_fwd8p, Heads, 128, 0)
+ZT_FWD_SPLIT(zt_fwd8ps, Heads, 128, 1)
 #endif

@@ -258,7 +258,7 @@ DEVI void gemm_body(const GemmArgs &g) {
 // workgroups share a CU and cover each other's barriers.  4096^3: 1064 us on f32
 // MFMAs (129 TFLOP/s), 788 us (174 TFLOP/s); bound by power, as the forward.
 template <int BT, bool KC>
-constexpr int slab_bytes() { return KC ? split_bytes<32>(BT) : split_bytes<BT>(32); }
+constexpr int slab_bytes() { return KC ? split_bytes(32, BT) : split_bytes(BT, 32); }
 
 // Part P of the operand of indices c0 .. c0 + 15 of a slab.
 template <int BT, bool KC, bool HALVES>
@@ -266,7 +266,7 @@ DEVI u4 slab_operand(const char *t, int c0, int lane, int part) {
     const int l16 = lane & 15, grp = lane >> 4;
     if constexpr (!KC) return get_col<BT>(t, 32, 0, c0, lane, part);
     else if constexpr (!HALVES) return get_row<32>(t, BT, c0, 0, l16, grp, part);
-    const char *p = t + ((2 - part) * BT + c0 + l16) * split_stride<32>() + 8 * grp;
+    const char *p = t + ((2 - part) * BT + c0 + l16) * split_stride(32) + 8 * grp;
     const u2 x = *reinterpret_cast<const u2 *>(p), y = *reinterpret_cast<const u2 *>(p + 32);
     return u4{x.x, x.y, y.x, y.y};
 }
@@ -690,7 +690,7 @@ DEVI void dq_ds_tile(const DqDsArgs &g, const int tm, const int tn, const int bh
 // d = 256 1791 -> 1733 us.
 DEVI void dq_ds_split_tile(const DqDsArgs &g, const int tm, const int tn, const int bh) {
     constexpr int BT = 128, TW = Tile<BT>::TW, WT = Tile<BT>::WT, NA = BT * BK / 4 / NTHR, NB = NA / 2;
-    constexpr int S = split_stride<BT>();
+    constexpr int S = split_stride(BT);
     char *const As = reinterpret_cast<char *>(dq_ds_slabs<BT, 1>()), *const Bs = As + slab_bytes<BT, false>();
     // The slab id (k0 + 1) whose dS (K) holds a big value.
     int *const flags = reinterpret_cast<int *>(Bs + slab_bytes<BT, false>());

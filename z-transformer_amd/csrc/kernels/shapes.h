@@ -1,0 +1,78 @@
+// Wave shapes of the split-operand attention kernels and the LDS each takes: one
+// table for the kernels that hold the shapes (attn_fwd.hip, attn_bwd.hip) and the
+// launcher that picks among them (zt_attn.cpp), so that a shape the launcher asks
+// for is one its kernel has.
+#pragma once
+
+// Split tiles in LDS: row-major rows of dp bf16 values, one plane of `rows` rows
+// per part.  The row stride is 2 dp + 32 bytes, 8 banks beyond a multiple
+// of 16 (dp a multiple of 32): eight rows then cover the 64 banks, both for an
+// operand read along the row (a lane per row, 16 bytes) and for a transposed
+// read (four rows x 32 bytes per 16 lanes).
+constexpr int split_stride(int dp) { return 2 * dp + 32; }
+constexpr int split_bytes(int dp, int rows) { return 3 * rows * split_stride(dp); }
+
+// ---- Forward: nw waves, nq 16-row blocks per wave, ks key parts ----------------
+struct FwdWaves {
+    int nw, nq, ks;
+};
+struct FwdWavesList {
+    int n;
+    FwdWaves s[4];
+};
+// Several heads of a kv group per workgroup (zt_fwd8p_*, zt_fwd8ps_*); one
+// (zt_fwdp_*, also four waves, where forced); one on a small grid (zt_fwdpk_*).
+enum class FwdRole { Heads, One, Small };
+constexpr int fwd_ds(int dp) { return dp > 128 ? 2 : 1; }  // column halves
+
+constexpr FwdWavesList fwd_waves(FwdRole role, int dp) {
+    if (role == FwdRole::Small) return dp <= 64 ? FwdWavesList{2, {{8, 1, 2}, {8, 1, 4}}} : FwdWavesList{1, {{8, 1, 2}}};
+    if (role == FwdRole::One)
+        return dp <= 64    ? FwdWavesList{4, {{8, 2, 1}, {8, 2, 2}, {8, 1, 2}, {4, 2, 1}}}
+               : dp <= 128 ? FwdWavesList{3, {{8, 2, 1}, {8, 1, 2}, {4, 2, 1}}}
+                           : FwdWavesList{3, {{8, 2, 1}, {8, 1, 1}, {4, 2, 1}}};
+    return dp == 32    ? FwdWavesList{4, {{8, 2, 1}, {8, 2, 2}, {8, 1, 2}, {8, 1, 4}}}
+           : dp == 64  ? FwdWavesList{3, {{8, 2, 1}, {8, 2, 2}, {8, 1, 2}}}
+           : dp <= 128 ? FwdWavesList{2, {{8, 2, 1}, {8, 1, 2}}}
+                       : FwdWavesList{2, {{8, 2, 1}, {8, 1, 1}}};
+}
+// Alternating wave halves (fwd_split_tile): two buffers each for K and V.
+constexpr bool fwd_alt(int dp, FwdWaves s) {
+    return s.nw == 8 && fwd_ds(dp) == 1 && 4 * split_bytes(dp, 32 * s.ks) + 16 <= 160 * 1024;
+}
+constexpr int fwd_tiles_lds(int dp, FwdWaves s) { return (fwd_alt(dp, s) ? 4 : 2) * split_bytes(dp, 32 * s.ks); }
+// The tiles, the partial scores that the column halves exchange, and the big-value flags.
+constexpr int fwd_lds(int dp, FwdWaves s) { return fwd_tiles_lds(dp, s) + (fwd_ds(dp) > 1 ? s.nw * 2 * s.nq * 1024 : 0) + 16; }
+// What the kernel of a role takes, whichever of its shapes runs.
+constexpr int fwd_lds(FwdRole role, int dp) {
+    int most = 0;
+    for (int i = 0; i < fwd_waves(role, dp).n; ++i) {
+        const int x = fwd_lds(dp, fwd_waves(role, dp).s[i]);
+        most = x > most ? x : most;
+    }
+    return most;
+}
+
+// ---- dk/dv from the forward's scores: `parts` parts of `kblocks` 16-key blocks ---
+struct BwdWaves {
+    int parts, kblocks;
+};
+struct BwdWavesList {
+    int n;
+    BwdWaves s[3];
+};
+constexpr BwdWavesList dkdv_waves(int dp) {
+    return dp == 32   ? BwdWavesList{3, {{2, 4}, {4, 2}, {8, 1}}}
+           : dp == 64 ? BwdWavesList{3, {{2, 4}, {4, 2}, {4, 1}}}
+                      : BwdWavesList{2, {{2, 4}, {2, 2}}};
+}
+// A dO and a Q tile of 32 rows, their rows' statistics and the big-value flags, per part.
+constexpr int dkdv_lds(int dp, BwdWaves s) { return s.parts * (2 * split_bytes(dp, 32) + 64 * 4 + 8); }
+constexpr int dkdv_lds(int dp) {
+    int most = 0;
+    for (int i = 0; i < dkdv_waves(dp).n; ++i) {
+        const int x = dkdv_lds(dp, dkdv_waves(dp).s[i]);
+        most = x > most ? x : most;
+    }
+    return most;
+}

@@ -44,6 +44,7 @@
 // product is formed in f32).
 #pragma once
 #include "common.h"
+#include "shapes.h"
 #include <utility>
 
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
@@ -175,28 +176,18 @@ DEVI void stream_parts(Load load, Step step) {
     }
 }
 
-// Split tiles in LDS: row-major rows of DP bf16 values, one plane of `rows`
-// rows per part.  The row stride is 2 DP + 32 bytes, 8 banks beyond a multiple
-// of 16 (DP a multiple of 32): eight rows then cover the 64 banks, both for an
-// operand read along the row (a lane per row, 16 bytes) and for a transposed
-// read (four rows x 32 bytes per 16 lanes).
-template <int DP>
-constexpr int split_stride() { return 2 * DP + 32; }
-template <int DP>
-constexpr int split_bytes(int rows) { return 3 * rows * split_stride<DP>(); }
-
 template <int DP>
 DEVI void put_tri(char *tile, int rows, int row, int col, const Tri &t) {  // col a multiple of 8
-    char *p = tile + row * split_stride<DP>() + 2 * col;
+    char *p = tile + row * split_stride(DP) + 2 * col;
     *reinterpret_cast<u4 *>(p) = t.h;
-    *reinterpret_cast<u4 *>(p + rows * split_stride<DP>()) = t.m;
-    *reinterpret_cast<u4 *>(p + 2 * rows * split_stride<DP>()) = t.l;
+    *reinterpret_cast<u4 *>(p + rows * split_stride(DP)) = t.m;
+    *reinterpret_cast<u4 *>(p + 2 * rows * split_stride(DP)) = t.l;
 }
 // Part C (0 = l, 1 = m, 2 = h) of an operand with the contraction along the row:
 // lane l16 = row, k slot 8 grp + j = column c0 + 8 grp + j.
 template <int DP>
 DEVI u4 get_row(const char *tile, int rows, int row0, int c0, int l16, int grp, int part) {
-    return *reinterpret_cast<const u4 *>(tile + ((2 - part) * rows + row0 + l16) * split_stride<DP>() + 2 * (c0 + 8 * grp));
+    return *reinterpret_cast<const u4 *>(tile + ((2 - part) * rows + row0 + l16) * split_stride(DP) + 2 * (c0 + 8 * grp));
 }
 // gfx950's transposing LDS read: 16 lanes read four rows of 16 values (lane i
 // at row i / 4, values 4 (i % 4)) and lane i gets column i of the four.
@@ -211,7 +202,7 @@ DEVI u2 lds_tr16(const char *p) {
 template <int DP>
 DEVI u4 get_col(const char *tile, int rows, int r0, int c0, int lane, int part) {
     const int i = lane & 15, grp = lane >> 4;
-    constexpr int S = split_stride<DP>();
+    constexpr int S = split_stride(DP);
     const char *p = tile + ((2 - part) * rows + r0 + 4 * grp + (i >> 2)) * S + 2 * (c0 + 4 * (i & 3));
     const u2 x = lds_tr16(p), y = lds_tr16(p + 16 * S);
     return u4{x.x, x.y, y.x, y.y};

@@ -27,6 +27,7 @@
 
 #include "../../include/zt_attn.h"
 #include "kernels/args.h"
+#include "kernels/shapes.h"
 
 extern "C" {
 extern const unsigned char zt_co_fwd[], zt_co_fwd_end[];
@@ -266,14 +267,15 @@ int fwd_key_split(int B, int T, int n_heads, int hw, int dp, int dim, int bk, in
     return able ? tuned(kTuneFKS, wgs <= cus ? 2 : 1) : 1;
 }
 
-// Whether the kernel fwd_kernel_name names for p holds the wave shape p (the
-// lists in kernels/attn_fwd.hip).
+// The role of p's kernel, and whether that kernel holds p's wave shape.
+FwdRole fwd_role(const FwdPlan &p) {
+    return p.nw == 8 && p.hw > 1 ? FwdRole::Heads : p.small ? FwdRole::Small : FwdRole::One;
+}
 bool fwd_shape_built(const FwdPlan &p, int dp) {
-    if (p.nw == 4) return p.nq == 2 && p.ks == 1;
-    if (p.ds == 2) return p.ks == 1;
-    if (p.small) return p.nq == 1 && (p.ks == 2 || (p.ks == 4 && dp <= 64));
-    return (p.nq == 2 && p.ks == 1) || (p.nq == 1 && p.ks == 2) || (p.nq == 2 && p.ks == 2 && dp <= 64) ||
-           (p.nq == 1 && p.ks == 4 && dp == 32 && p.hw >= 2);
+    const FwdWavesList l = fwd_waves(fwd_role(p), dp);
+    for (int i = 0; i < l.n; ++i)
+        if (l.s[i].nw == p.nw && l.s[i].nq == p.nq && l.s[i].ks == p.ks) return true;
+    return false;
 }
 
 // Wave shapes on split operands, by how many workgroups the widest shape (two
@@ -299,7 +301,7 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
     if (!p.split) return p;
     p.nw = tuned(kTuneFwdW, 8);  // (C2 at four waves, two workgroups per CU: 77 us against 47)
     p.small = p.small && p.nw == 8;
-    p.ds = dp > 128 ? 2 : 1;
+    p.ds = fwd_ds(dp);
     p.nq = 2; p.ks = 1;
     while (p.nw / p.ds < p.hw) p.hw /= 2;  // (four waves forced, two column halves)
     const long long wide = (long long)((T + fwd_rows(p) - 1) / fwd_rows(p)) * (n_heads / p.hw) * B;
@@ -329,8 +331,8 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
 // whole 16-byte chunks or a forced 64-key tile (without).
 void fwd_kernel_name(char *name, size_t len, int dim, int dp, int bk, const FwdPlan &p, bool scores) {
     const bool pf = bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1;
-    if (p.split && p.nw == 8 && p.hw == 1)
-        snprintf(name, len, p.small ? "zt_fwdpk_d%d_k32" : "zt_fwdp_d%d_k32", dp);
+    if (p.split && fwd_role(p) != FwdRole::Heads)
+        snprintf(name, len, fwd_role(p) == FwdRole::Small ? "zt_fwdpk_d%d_k32" : "zt_fwdp_d%d_k32", dp);
     else if (pf && p.nw == 8)  // keeping scores: the same kernel, named for its role
         snprintf(name, len, scores && dp <= 128 ? "zt_fwd8ps_d%d_k32" : "zt_fwd8p_d%d_k32", dp);
     else if (pf)
@@ -934,10 +936,13 @@ static void dkdv_split_shape(int B, int T, int n_kv_heads, int dp, int cus, int 
     int kb = 4;
     if (2 * wgs <= cus || (dp == 32 && wgs <= cus)) kb = 2;
     if ((4 * wgs <= cus && dp <= 64) || (dp == 32 && 2 * wgs <= cus)) kb = 1;
-    const int forced = tuned(kTuneBShape, kb);
-    kb = forced == 1 && dp > 64 ? 2 : forced;
-    *kblocks = kb;
-    *parts = dp > 64 ? 2 : kb == 4 ? 2 : kb == 2 ? 4 : dp == 32 ? 8 : 4;
+    kb = tuned(kTuneBShape, kb);
+    // The shape of kb blocks, or the last (fewest blocks) where the kernel has none.
+    const BwdWavesList l = dkdv_waves(dp);
+    int i = 0;
+    while (i + 1 < l.n && l.s[i].kblocks != kb) ++i;
+    *kblocks = l.s[i].kblocks;
+    *parts = l.s[i].parts;
 }
 
 // Which workspaces hold scores, and of what.  zt_attn_forward_train_ws stamps
