@@ -55,7 +55,8 @@ int zt_attn_dim_ok(int dim);
  * counts: the LDS bytes per workgroup THIS library's kernel asks at head width
  * `dim` with its key tile capped at `tile` (a tile cap below 64 selects the
  * 32-key tile; `group_q` does not change this library's schedule and is
- * ignored here).  The dk/dv figure is the most that kernel asks at `dim`.
+ * ignored here).  The forward's and the dk/dv figure are the most that any of
+ * their kernels for `dim` asks, whichever the grid and the head group pick.
  * 0 for a width zt_attn_dim_ok refuses. */
 size_t zt_attn_forward_shmem(int dim, int tile, int group_q);
 size_t zt_attn_bwd_dq_shmem(int dim, int tile);

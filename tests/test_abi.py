@@ -6,6 +6,8 @@ reference does for a device whose ceiling cannot be read (:910-915)."""
 import ctypes
 import os
 import re
+import subprocess
+import tempfile
 
 import pytest
 
@@ -55,6 +57,52 @@ def test_shmem_counts(zt):
         assert 0 < L.zt_attn_bwd_dq_shmem(d, 32) <= L.zt_attn_bwd_dq_shmem(d, 64) <= 160 * 1024
         assert 0 < L.zt_attn_bwd_dkdv_shmem(d) <= 160 * 1024
     assert L.zt_attn_forward_shmem(33, 64, 1) == 0 and L.zt_attn_bwd_dkdv_shmem(300) == 0
+
+
+def _static_lds():
+    """kernel name -> static LDS bytes, from the metadata of the code objects that build.py leaves beside the library."""
+    lds = {}
+    for tag in ("fwd", "bwd"):
+        co = open(os.path.join(ROOT, "z-transformer_amd", "_build", f"{tag}.hsaco"), "rb").read()
+        with tempfile.NamedTemporaryFile(suffix=".elf") as f:
+            f.write(co[co.index(b"\x7fELF"):])  # (past the offload bundle's header)
+            f.flush()
+            readelf = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+            notes = subprocess.run([readelf, "--notes", f.name], check=True, stdout=subprocess.PIPE, text=True).stdout
+        for size, name in re.findall(r"\.group_segment_fixed_size: (\d+).*?\.name:\s+(zt_\w+)", notes, re.S):
+            lds[name] = int(size)
+    assert len(lds) > 100
+    return lds
+
+
+def test_shmem_counts_are_the_kernels_lds(zt):
+    """The most static LDS among the kernels that a width can launch: 16-byte
+    rows (dim % 4 == 0) take the split-operand and prefetching kernels, whole
+    widths (a multiple of 32) the asynchronously staged and column-split ones."""
+    L, lds = zt.lib(), _static_lds()
+
+    def most(pattern):
+        return max(size for name, size in lds.items() if re.fullmatch(pattern, name))
+
+    for dp in range(32, 257, 32):
+        for dim in (dp, dp - 4, dp - 2):
+            if dim < 32:
+                continue
+            rows16, whole = dim % 4 == 0, dim == dp
+            if rows16:
+                fwd32 = fwd64 = most(rf"zt_fwd(8p|8ps|p|pk)_d{dp}_k32")
+            else:
+                fwd32 = most(rf"zt_fwd8?_d{dp}_k32")
+                fwd64 = most(rf"zt_fwd8?_d{dp}_k{64 if dp <= 64 else 32}")
+            assert (L.zt_attn_forward_shmem(dim, 32, 1), L.zt_attn_forward_shmem(dim, 64, 1)) == (fwd32, fwd64), dim
+            assert L.zt_attn_bwd_dq_shmem(dim, 64) == most(rf"zt_bwd_dq(8|p|8p|l)?_d{dp}_k32"), dim
+            kinds = ["_d{0}_hs[124]"]
+            if dp <= 128:
+                kinds += ["8_d{0}_hs2"] + (["8p_d{0}_hs2", "8s_d{0}_hs2"] if rows16 else [])
+            if whole:
+                kinds += ["_dma_d{0}_hs[124]", "_dmar_d{0}", "_dmars_d{0}", "_dmas_d{0}_hs2", "8pd_d{0}_hs[12]",
+                          "8sd_d{0}_hs2"]
+            assert L.zt_attn_bwd_dkdv_shmem(dim) == most("zt_bwd_dkdv(" + "|".join(kinds).format(dp) + ")"), dim
 
 
 def _fwd(L, T=8, H=4, Hkv=2, dim=32, group_q=1, max_tile=64, q_offset=0, n_keys=8):

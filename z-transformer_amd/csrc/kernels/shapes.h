@@ -53,6 +53,14 @@ constexpr int fwd_lds(FwdRole role, int dp) {
     return most;
 }
 
+// The most any of a width's kernels takes (Small is built for dp <= 128).
+constexpr int fwd_lds(int dp) {
+    int most = fwd_lds(FwdRole::Heads, dp);
+    if (fwd_lds(FwdRole::One, dp) > most) most = fwd_lds(FwdRole::One, dp);
+    if (dp <= 128 && fwd_lds(FwdRole::Small, dp) > most) most = fwd_lds(FwdRole::Small, dp);
+    return most;
+}
+
 // ---- dk/dv from the forward's scores: `parts` parts of `kblocks` 16-key blocks ---
 struct BwdWaves {
     int parts, kblocks;

@@ -249,8 +249,11 @@ struct FwdPlan {
 int fwd_rows(const FwdPlan &p) { return 16 * p.nq * (p.nw / (p.ks * p.ds * p.hw)); }
 
 // Widths the split-operand forward is built for (a wave's columns are whole
-// 32-column groups); it loads whole 16-byte row chunks (dim % 4 == 0).
+// 32-column groups); it loads whole 16-byte row chunks (dim % 4 == 0) in 32-key tiles.
 bool fwd_split_width(int dp) { return dp <= 128 || dp == 192 || dp == 256; }
+bool fwd_splits(int dim, int dp, int bk) {
+    return bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1 && fwd_split_width(dp);
+}
 
 // Key parts of the forward: 1, or 2 for the key-split kernel (zt_fwdpk_*:
 // eight waves, 4 row blocks x 2 key parts merged at the end) for one query
@@ -297,7 +300,7 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
     p.small = ks > 1;
     p.nw = ks > 1 ? 8 : fwd_waves(p.hw);
     p.nq = 1; p.ks = ks; p.ds = 1;
-    p.split = bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1 && fwd_split_width(dp);
+    p.split = fwd_splits(dim, dp, bk);
     if (!p.split) return p;
     p.nw = tuned(kTuneFwdW, 8);  // (C2 at four waves, two workgroups per CU: 77 us against 47)
     p.small = p.small && p.nw == 8;
@@ -324,6 +327,11 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
     }
     while (p.nw / (p.ks * p.ds) < p.hw) p.hw /= 2;
     return p;
+}
+
+// The LDS its kernel takes per workgroup.
+size_t fwd_plan_lds(const FwdPlan &p, int dp, int bk) {
+    return p.split ? (size_t)fwd_lds(fwd_role(p), dp) : fwd_tile_bytes(dp, bk);
 }
 
 // Forward kernel name: the split-operand kernels, and the f32 MFMA kernels for
@@ -534,10 +542,11 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     const int dp = pad32(dim);
     int bk = key_tile(Tiled::Forward, dp, max_tile, dim);
     if (fwd_tile_bytes(dp, bk) > st->lds_limit) bk = 32;
-    if (fwd_tile_bytes(dp, bk) > st->lds_limit) {
+    const FwdPlan p = fwd_plan(B, T, n_heads, n_kv_heads, dp, dim, bk, st->cus);
+    if (fwd_plan_lds(p, dp, bk) > st->lds_limit) {
         fprintf(stderr, "zt_attn: head_dim %d needs %zu bytes of LDS per workgroup even at a 32-key tile, and\n"
                         "       this device grants %zu. Refusing.\n",
-                dim, fwd_tile_bytes(dp, bk), st->lds_limit);
+                dim, fwd_plan_lds(p, dp, bk), st->lds_limit);
         return 1;
     }
     if (!q || !k || !v || !out) {
@@ -549,7 +558,6 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     a.q = q; a.k = k; a.v = v; a.out = out; a.lse = lse; a.s_out = s_out;
     a.B = B; a.T = T; a.H = n_heads; a.Hkv = n_kv_heads; a.dim = dim;
     a.q_offset = q_offset; a.n_keys = n_keys; a.kv_rows = kv_rows;
-    const FwdPlan p = fwd_plan(B, T, n_heads, n_kv_heads, dp, dim, bk, st->cus);
     a.HW = p.hw; a.nq = p.nq; a.ks = p.ks;
     const int rows_per_wg = fwd_rows(p);
     a.n_row_tiles = (T + rows_per_wg - 1) / rows_per_wg;
@@ -763,8 +771,8 @@ int zt_attn_dim_ok(int dim) { return !(dim < kMinDim || dim > kMaxDim || (dim & 
 size_t zt_attn_forward_shmem(int dim, int tile, int group_q) {
     (void)group_q;
     if (!zt_attn_dim_ok(dim)) return 0;
-    const int dp = pad32(dim);
-    return fwd_tile_bytes(dp, key_tile(Tiled::Forward, dp, tile, dim));
+    const int dp = pad32(dim), bk = key_tile(Tiled::Forward, dp, tile, dim);
+    return fwd_splits(dim, dp, bk) ? (size_t)fwd_lds(dp) : fwd_tile_bytes(dp, bk);
 }
 
 size_t zt_attn_bwd_dq_shmem(int dim, int tile) {
@@ -776,13 +784,17 @@ size_t zt_attn_bwd_dq_shmem(int dim, int tile) {
 size_t zt_attn_bwd_dkdv_shmem(int dim) {
     if (!zt_attn_dim_ok(dim)) return 0;
     const int dp = pad32(dim);
-    size_t most = dkdv_bytes(dp, dp <= 128 ? 4 : 2);
-    if (dp <= 128) most = std::max(most, dkdv_bytes(dp, 2, 4, 32, 2));  // eight waves, two 32-row stage buffers
-    if (dp == 192 || dp == 256)  // column-split eight waves
-        most = std::max(most, std::max(dkdv_dspd_bytes(dp, 2), dkdv_dspd_bytes(dp, 1)));
-    if (dp == 64 || dp == 128) most = std::max(most, dkdv_dspd_bytes(dp, 1));
-    for (int hs : {1, 2, 4})
-        if (!(hs == 4 && dp > 128) && dkdv_dma_bytes(dp, hs) > most) most = dkdv_dma_bytes(dp, hs);
+    const int hs = dp <= 128 ? 4 : 2;  // most head parts
+    size_t most = dkdv_bytes(dp, hs);
+    if (dp <= 128) {  // eight waves: register-prefetched, and reading the forward's scores
+        most = std::max(most, dkdv_bytes(dp, 2, 4));
+        if (dim % 4 == 0) most = std::max(most, std::max(dkdv_bytes(dp, 2, 4, 16, 2), (size_t)dkdv_lds(dp)));
+    }
+    if (dim == dp) {  // whole-head rows: asynchronously staged, and column-split eight waves
+        most = std::max(most, dkdv_dma_bytes(dp, hs));
+        if (dp == 192 || dp == 256) most = std::max(most, dkdv_dspd_bytes(dp, 2));
+        if (dp == 64 || dp == 128) most = std::max(most, dkdv_dspd_bytes(dp, 1));
+    }
     return most;
 }
 
@@ -905,7 +917,7 @@ static ScoreKernel score_kernel(int B, int T, int dim, int n_heads, int n_kv_hea
     const int dp = pad32(dim);
     if (n_kv_heads <= 0 || n_heads % n_kv_heads != 0 || dim % 4 != 0) return ScoreKernel::None;
     if ((n_heads / n_kv_heads) % 2 == 0) {
-        const bool fits = dp <= 128 ? dkdv_bytes(dp, 2, 4, 32, 2) <= st->lds_limit
+        const bool fits = dp <= 128 ? (size_t)dkdv_lds(dp) <= st->lds_limit
                                     : dim == dp && dkdv_dma_bytes(dp, 2) <= st->lds_limit;
         return fits ? ScoreKernel::Split : ScoreKernel::None;
     }
@@ -913,7 +925,8 @@ static ScoreKernel score_kernel(int B, int T, int dim, int n_heads, int n_kv_hea
     const unsigned long long tiles = (unsigned long long)(T + 63) / 64;
     const bool dma_pays = (tiles + 1) / 2 * n_kv_heads * B <= (unsigned long long)st->cus;
     const bool rsplit = dim == dp && dp <= 128 && dkdv_dma_bytes(dp, 2) <= st->lds_limit &&
-                        tuned(kTuneDMA, dma_pays ? 1 : 0) == 1 && tuned(kTuneRSplit, 1) == 1;
+                        (size_t)dkdv_lds(dp) <= st->lds_limit && tuned(kTuneDMA, dma_pays ? 1 : 0) == 1 &&
+                        tuned(kTuneRSplit, 1) == 1;
     return rsplit && tuned(kTuneRScores, 1) == 1 ? ScoreKernel::RowSplit : ScoreKernel::None;
 }
 static bool scores_path(int B, int T, int dim, int n_heads, int n_kv_heads, const DeviceState *st) {
