@@ -475,13 +475,15 @@ __device__ __forceinline__ void bwd_dq_lse_tile(const BwdArgs &a, const int tile
 // waves fit per SIMD; the partner wave holding the other half (w ^ KW*HS)
 // shares the partial dP through LDS, both form dP = own + partner (f32
 // addition commutes: the two copies are identical) and the same P and dS.
-template <int DP, int HS, int KW, bool PF = false, int NU = 1, bool SIN = false, int DS = 1>
+template <int DP, int HS, int KW, bool PF = false, bool SIN = false, int DS = 1>
 __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile, const bool up) {
     static_assert(!SIN || PF, "the scores are prefetched with the stage's rows");
     static_assert(DS == 1 || (PF && DS == 2 && (DP / 32) % 2 == 0), "d-split: prefetching, whole 32-column halves");
     constexpr int LW = DP + 4, NTH = 64 * KW * HS * DS;
     constexpr int DPW = DP / DS, DQW = DPW / 4, NTW = DPW / 16;  // a wave's columns
-    constexpr int BQ = 16 * NU;  // query rows per stage: NU sub-tiles of 16
+    // Query rows per stage: NU sub-tiles of 16.  (Written for any NU; plain vectors
+    // instead of arrays of one take 288 registers and not 200 in zt_bwd_dkdv_d128_hs1.)
+    constexpr int NU = 1, BQ = 16 * NU;
     // Per head-split part: Q rows, dO rows, and the rows' m2, -delta and 1/l
     // (BQ floats each, so that a lane reads its four rows' values as one float4).
     // With the register prefetch (PF) two such stage buffers: stage s reads one
@@ -500,21 +502,6 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // in a scalar register: wave-uniform branches stay scalar
     const int kbw = w % KW, hs = (w / KW) % HS, dh = w / (KW * HS);  // dh: the wave's column half (DS = 2)
-    // Column block of the dP / S products (a lane per staged row, lane group grp
-    // reading 32 of the DP columns): grp with its two bits swapped, so that
-    // the lane groups a 128-bit LDS read serves together sit 64 columns (all
-    // 64 banks) apart.  With grp itself the reads of rows l16 and l16 - 8 of
-    // groups 0 and 1 meet in one bank: a probe of the bank-conflict counter
-    // on gfx950 shows 3.8 conflict cycles per read, and none with the swap
-    // (C3 dk/dv 1.776 -> 1.762 ms).  Needs DP % 128 == 0; only where the
-    // scores are read (the kernel that forms S again reads Q and dO this way
-    // too, and measured 2.268 -> 2.281 ms with the swap).  The dV / dK reads
-    // (a lane per 16-byte chunk of rows 4 grp + kk) keep 3.8: no ownership of
-    // chunks free of per-step address arithmetic removes them under every
-    // lane grouping the probe admits, and an XOR-swizzled layout that does
-    // cost more in registers and VALU than it saved (1.78 -> 1.81 ms).
-    constexpr bool PERM = SIN && DS == 1 && DP % 128 == 0;
-    const int cbk = PERM ? ((grp & 1) << 1) | (grp >> 1) : grp;
     const int per_tile = a.Hkv * a.B;
     const int rem = (int)blockIdx.x % per_tile;
     const int kvh = rem % a.Hkv, b = rem / a.Hkv;
@@ -531,9 +518,9 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
     const bool key_ok = my_key < a.T;
     float kr[SIN ? 1 : DQW], vr[DQW];  // with the forward's scores K is not needed
     if constexpr (!SIN)
-        load_row_seg<DQW>(kr, a.k + kvrd + (size_t)my_key * kld + dh * DPW, cbk * DQW, a.dim - dh * DPW, vec4, key_ok,
+        load_row_seg<DQW>(kr, a.k + kvrd + (size_t)my_key * kld + dh * DPW, grp * DQW, a.dim - dh * DPW, vec4, key_ok,
                           ZT_PLANT == 14 ? kLog2e : a.scale_log2e);
-    load_row_seg<DQW>(vr, a.v + kvrd + (size_t)my_key * kld + dh * DPW, cbk * DQW, a.dim - dh * DPW, vec4, key_ok,
+    load_row_seg<DQW>(vr, a.v + kvrd + (size_t)my_key * kld + dh * DPW, grp * DQW, a.dim - dh * DPW, vec4, key_ok,
                       1.f);
 
     f4 dka[NTW], dva[NTW];
@@ -708,18 +695,12 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
             s[u] = zero4();
         }
         if constexpr (SIN) {
-            // Scores from the forward; dP alone, as one chain per sub-tile with
-            // the sub-tiles' products interleaved (NU >= 2), else as two chains
-            // summed.  (Raising the second head half's wave priority through dP,
-            // so that the two waves of a SIMD leave it at different times, once
-            // gained 1%; with the dP column blocks of lane groups 1 and 2 swapped
-            // it costs 0.9%.)
-            constexpr bool TWO = NU < 2;
+            // Scores from the forward; dP alone, as two chains summed.
             f4 dp2[NU];
 #pragma unroll
             for (int u = 0; u < NU; ++u) { s[u] = sn[u]; dp2[u] = zero4(); }
             // dO operands read one group ahead of their products.
-            const float *dsw = ds + dh * DPW + cbk * DQW;
+            const float *dsw = ds + dh * DPW + grp * DQW;
             f4 dxn[NU];
 #pragma unroll
             for (int u = 0; u < NU; ++u) dxn[u] = *reinterpret_cast<const f4 *>(dsw + (16 * u + l16) * LW);
@@ -732,26 +713,17 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
                     if (kk + 4 < DQW) dxn[u] = *reinterpret_cast<const f4 *>(dsw + (16 * u + l16) * LW + kk + 4);
                 }
                 __builtin_amdgcn_sched_barrier(0);  // keeps the reads ahead of this group's products
-                if constexpr (TWO) {
 #pragma unroll
-                    for (int u = 0; u < NU; ++u) {
-                        dp[u] = mfma16(dx[u].x, vr[kk + 0], dp[u]);
-                        dp2[u] = mfma16(dx[u].y, vr[kk + 1], dp2[u]);
-                        dp[u] = mfma16(dx[u].z, vr[kk + 2], dp[u]);
-                        dp2[u] = mfma16(dx[u].w, vr[kk + 3], dp2[u]);
-                    }
-                } else {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-#pragma unroll
-                        for (int u = 0; u < NU; ++u) dp[u] = mfma16(dx[u][c], vr[kk + c], dp[u]);
+                for (int u = 0; u < NU; ++u) {
+                    dp[u] = mfma16(dx[u].x, vr[kk + 0], dp[u]);
+                    dp2[u] = mfma16(dx[u].y, vr[kk + 1], dp2[u]);
+                    dp[u] = mfma16(dx[u].z, vr[kk + 2], dp[u]);
+                    dp2[u] = mfma16(dx[u].w, vr[kk + 3], dp2[u]);
                 }
                 fetch_after(kk / 4);
             }
-            if constexpr (TWO) {
 #pragma unroll
-                for (int u = 0; u < NU; ++u) dp[u] += dp2[u];
-            }
+            for (int u = 0; u < NU; ++u) dp[u] += dp2[u];
             if constexpr (DS > 1) {
                 float *xch = smem + MAIN_F;
 #pragma unroll
@@ -766,7 +738,7 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
             for (int kk = 0; kk < DQW; kk += 4) {
 #pragma unroll
                 for (int u = 0; u < NU; ++u) {
-                    const int col = dh * DPW + cbk * DQW + kk;
+                    const int col = dh * DPW + grp * DQW + kk;
                     const f4 qx = *reinterpret_cast<const f4 *>(qs + (16 * u + l16) * LW + col);
                     const f4 dx = *reinterpret_cast<const f4 *>(ds + (16 * u + l16) * LW + col);
                     s[u] = mfma16(qx.x, kr[kk + 0], s[u]);
@@ -827,9 +799,7 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
             for (int u = 0; u < NU; ++u) {
                 // wave-uniform: a sub-tile past the last row or above the diagonal has no slot
                 if (t0 + 16 * u >= a.T || t0 + 16 * u + 15 < s0) continue;
-                // (ZT_PLANT 15 swaps the two sub-tiles' slots where both exist.)
-                const int us = (ZT_PLANT == 15 && NU == 2 && t0 + 16 < a.T && t0 + 15 >= s0) ? NU - 1 - u : u;
-                const size_t tile = cur.sblk + zt_tri_index((t0 >> 4) + us, s0 >> 4);
+                const size_t tile = cur.sblk + zt_tri_index((t0 >> 4) + u, s0 >> 4);
                 // Scalar tile base plus the lane's 32-bit byte offset.
                 __builtin_nontemporal_store(
                     dsv[u], reinterpret_cast<f4 *>(reinterpret_cast<char *>(a.ds_out + tile * 256) + lane * 16u));
@@ -838,14 +808,11 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
     };
 
     // The second half: dV^T += dO^T P and dK^T += Q^T dS from the stage's rows.
-    // mid: the scalar bookkeeping of the stage after next, placed among the
-    // products (at the loop's head it ran beside no MFMA).
-    auto back = [&](int stg, const StageAt cur, const f4 (&p)[NU], const f4 (&dsv)[NU], auto &&mid) {
+    auto back = [&](int stg, const StageAt cur, const f4 (&p)[NU], const f4 (&dsv)[NU]) {
         const int t0 = cur.t0;
         const float *qs = Qs + stage_off(stg) + hs * BQ * LW, *ds = Ds + stage_off(stg) + hs * BQ * LW;
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
-            if (u == 1) mid();
             if (t0 + 16 * u + 15 < s0) continue;  // wave-uniform: this sub-tile is wholly masked
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
@@ -862,7 +829,8 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
         }
     };
 
-    // One whole stage: the first half, then the second.
+    // One whole stage: the first half, then the second, then mid: the scalar
+    // bookkeeping of the stage after next.
     auto work = [&](int stg, const StageAt cur, const StageAt nx, auto &&mid) {
         if (!visible(cur)) {
             if constexpr (PF) fetch(nx);
@@ -872,8 +840,8 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
         }
         f4 p[NU], dsv[NU];
         front(stg, cur, nx, p, dsv);
-        back(stg, cur, p, dsv, mid);
-        if constexpr (NU < 2) mid();
+        back(stg, cur, p, dsv);
+        mid();
     };
 
     if constexpr (PF) {
@@ -972,7 +940,7 @@ __device__ __forceinline__ void bwd_dkdv_tile(const BwdArgs &a, const int ktile,
 // are summed as the head halves' are.
 template <int DP, int HS, bool SIN = false, bool RS = false>
 __device__ __forceinline__ void bwd_dkdv_dma_tile(const BwdArgs &a, const int ktile) {
-    static_assert(!RS || HS == 2, "row split: two parts");
+    static_assert(!RS || (HS == 2 && !SIN), "row split: two parts, S formed");
     constexpr int DQ = DP / 4, NT = DP / 16, KW = RS ? 4 : 4 / HS, BQ = 16, NW = KW * HS;
     constexpr int CPR = DP / 4;          // 16-byte chunks per row
     constexpr int TILE = BQ * DP;        // floats per (part, array) tile
@@ -1262,13 +1230,13 @@ __device__ __forceinline__ void bwd_dq_lse_body(const BwdArgs &a) {
     if ((a.dim & 3) == 0) bwd_dq_lse_pair<DP, BK, NW, true>(a);
     else bwd_dq_lse_pair<DP, BK, NW, false>(a);
 }
-template <int DP, int HS, int KW, bool PF = false, int NU = 1, bool SIN = false, int DS = 1>
+template <int DP, int HS, int KW, bool PF = false, bool SIN = false, int DS = 1>
 __device__ __forceinline__ void bwd_dkdv_body(const BwdArgs &a) {
     const int p = (int)blockIdx.x / (a.Hkv * a.B), n = a.n_key_tiles;
-    bwd_dkdv_tile<DP, HS, KW, PF, NU, SIN, DS>(a, p, false);
+    bwd_dkdv_tile<DP, HS, KW, PF, SIN, DS>(a, p, false);
     if (a.pair && n - 1 - p > p) {
         __syncthreads();  // the head-split sum reads LDS; the next tile's staging writes it
-        bwd_dkdv_tile<DP, HS, KW, PF, NU, SIN, DS>(a, n - 1 - p, true);
+        bwd_dkdv_tile<DP, HS, KW, PF, SIN, DS>(a, n - 1 - p, true);
     }
 }
 template <int DP, int HS, bool SIN = false, bool RS = false>
@@ -1697,7 +1665,7 @@ DEVI void dkdv_shapes(const BwdArgs &a) {
         bwd_dkdv_dma_body<DP, 2, true>(a);                                                         \
     }
 #define ZT_BWD_ALL(DP)                                                                             \
-    ZT_BWD_DQ(DP, 32) ZT_BWD_DQ(DP, 64) ZT_BWD_DQ_PF(DP) ZT_BWD_DQ_LSE(DP) ZT_BWD_DKDV(DP, 1) ZT_BWD_DKDV(DP, 2) ZT_BWD_DKDV8(DP)    \
+    ZT_BWD_DQ(DP, 32) ZT_BWD_DQ(DP, 64) ZT_BWD_DQ_PF(DP) ZT_BWD_DQ_LSE(DP) ZT_BWD_DKDV(DP, 1) ZT_BWD_DKDV(DP, 2)    \
     ZT_BWD_DKDV_DMA(DP, 1) ZT_BWD_DKDV_DMA(DP, 2)
 
 #if ZT_PLANT == 0
@@ -1705,6 +1673,7 @@ ZT_BWD_ALL(32)
 ZT_BWD_ALL(64)
 ZT_BWD_ALL(96)
 ZT_BWD_ALL(128)
+ZT_BWD_DKDV8(32) ZT_BWD_DKDV8(64) ZT_BWD_DKDV8(96) ZT_BWD_DKDV8(128)
 ZT_BWD_SPLIT(zt_bwd_dkdv8s_d32_hs2, 32)
 ZT_BWD_SPLIT(zt_bwd_dkdv8s_d64_hs2, 64)
 ZT_BWD_SPLIT(zt_bwd_dkdv8s_d96_hs2, 96)
@@ -1742,7 +1711,7 @@ ZT_BWD_DKDV_DMAS(160) ZT_BWD_DKDV_DMAS(192) ZT_BWD_DKDV_DMAS(224) ZT_BWD_DKDV_DM
 // are whole 32-column groups (d = 192, 256).
 #define ZT_BWD_DKDV8SD(DP)                                                                         \
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8sd_d##DP##_hs2(BwdArgs a) {   \
-        bwd_dkdv_body<DP, 2, 2, true, 1, true, 2>(a);                                              \
+        bwd_dkdv_body<DP, 2, 2, true, true, 2>(a);                                                 \
     }
 ZT_BWD_DKDV8SD(192) ZT_BWD_DKDV8SD(256)
 // The same column split for the kernel that forms S again (reference entry
@@ -1751,15 +1720,15 @@ ZT_BWD_DKDV8SD(192) ZT_BWD_DKDV8SD(256)
 // column halves of one part, also at d = 64 and 128.
 #define ZT_BWD_DKDV8PD(DP)                                                                         \
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8pd_d##DP##_hs2(BwdArgs a) {   \
-        bwd_dkdv_body<DP, 2, 2, true, 1, false, 2>(a);                                             \
+        bwd_dkdv_body<DP, 2, 2, true, false, 2>(a);                                                \
     }                                                                                              \
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8pd_d##DP##_hs1(BwdArgs a) {   \
-        bwd_dkdv_body<DP, 1, 4, true, 1, false, 2>(a);                                             \
+        bwd_dkdv_body<DP, 1, 4, true, false, 2>(a);                                                \
     }
 ZT_BWD_DKDV8PD(192) ZT_BWD_DKDV8PD(256)
 #define ZT_BWD_DKDV8PD1(DP)                                                                        \
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8pd_d##DP##_hs1(BwdArgs a) {   \
-        bwd_dkdv_body<DP, 1, 4, true, 1, false, 2>(a);                                             \
+        bwd_dkdv_body<DP, 1, 4, true, false, 2>(a);                                                \
     }
 ZT_BWD_DKDV8PD1(64) ZT_BWD_DKDV8PD1(128)
 #else
