@@ -256,3 +256,80 @@ def test_small_gradients_keep_their_bits(gpu, zt, tune, D):
     for got, w in zip(_train(gpu, zt, q, k, v, do, T, H, Hkv, D), want):
         w = np.asarray(w).ravel()
         assert np.max(np.abs(got - w)) <= 1e-5 * np.abs(w).max()
+
+
+@pytest.mark.parametrize("op,tile", [("nn", 128), ("tn", 128), ("nt", 128), ("tn", 64), ("nt", 64)])
+@pytest.mark.parametrize("which", ["a", "b", "ab", "ab apart"])
+def test_whole_tiles_with_large_values(gpu, zt, tune, op, tile, which):
+    """Infinities and magnitudes past the split's range in whole tiles, in one
+    operand, in both in the same slab, and in both in different slabs: the result is
+    what f32 arithmetic gives, with test_split_products' bound where it is finite."""
+    tune({"ZT_GEMM_TILE": tile})
+    M, K, N = 256, 96, 128
+    gen = gpu.Generator(device="cuda").manual_seed(tile)
+    a, b = (gpu.randn(s, device="cuda", generator=gen) for s in ((M, K), (K, N)))
+    if "a" in which:
+        a[7, 40], a[140, 41], a[255, 2] = float("inf"), -2.0 ** 45, 2.0 ** 80
+    if "b" in which:
+        k = 90 if "apart" in which else 43
+        b[k, 100], b[k + 1, 3] = float("-inf"), 2.0 ** 41
+    want = a.double().cpu() @ b.double().cpu()
+    got = _product(gpu, zt, op, a, b).double().cpu()
+    fin = gpu.isfinite(want)
+    assert gpu.equal(gpu.isnan(got), gpu.isnan(want))
+    assert gpu.equal(got[~fin & ~gpu.isnan(want)], want[~fin & ~gpu.isnan(want)])
+    bound = (a.double().abs().cpu() @ b.double().abs().cpu()) * ((34 + K / 32) * 2.0 ** -24)
+    assert gpu.all((got - want).abs()[fin] <= bound[fin])
+
+
+def _close_by_part(got, want, parts):
+    """1e-5 of the largest value (test_every_dkdv_shape's gate) within each part of the entries."""
+    for part in parts:
+        assert np.all(np.isfinite(got[part]))
+        assert np.max(np.abs(got[part] - want[part])) <= 1e-5 * max(1.0, np.abs(want[part]).max())
+
+
+@pytest.mark.parametrize("T,H,Hkv,D", [(90, 4, 2, 64), (90, 4, 4, 128), (161, 4, 2, 32)])
+def test_gradients_with_both_operands_large(gpu, zt, tune, T, H, Hkv, D):
+    """2^70 in both operands of a product, where the two do not meet, so that the
+    tile's whole product is formed in f32 and stays in its ordinary range."""
+    tune({"ZT_DQDS_TILE": 128, "ZT_DQDS_K": 1})
+    big, g = 2.0 ** 70, H // Hkv
+
+    def run(q, k, v, do):
+        want = attention_backward_f64(*(host(x) for x in (q, k, v, do)), T, H, Hkv, D)
+        got = _train(gpu, zt, q, k, v, do, T, H, Hkv, D)
+        return [(x.reshape(T, -1, D), np.asarray(w).reshape(T, -1, D)) for x, w in zip(got, want)]
+
+    def inputs():
+        q, k, v = _inputs(gpu, zt, T, H, Hkv, D)
+        return q, k, v, dev_normal(gpu, zt, T * H * D, SEED_DO)
+
+    # dP = dO V^T: column 3 of dO large and of V zero, column 5 the other way round.
+    q, k, v, do = inputs()
+    v.view(T, Hkv, D)[:, :, 3], do.view(T, H, D)[:, :, 5] = 0.0, 0.0
+    do.view(T, H, D)[50, -1, 3], v.view(T, Hkv, D)[40, -1, 5] = big, big
+    dq, dk, dv = run(q, k, v, do)
+    col = np.zeros((T, Hkv, D), bool)
+    col[:, -1, 3] = True  # dv of the large column
+    _close_by_part(*dq, [np.ones((T, H, D), bool)])
+    _close_by_part(*dk, [np.ones((T, Hkv, D), bool)])
+    _close_by_part(*dv, [col, ~col])
+
+    # dK = dS^T Q: row 50's dS large, row 52's Q large in a column where K is zero.
+    q, k, v, do = inputs()
+    k.view(T, Hkv, D)[:, :, 7] = 0.0
+    do.view(T, H, D)[50, -1, 3], q.view(T, H, D)[52, -1, 7] = big, big
+    dk = run(q, k, v, do)[1]
+    head = np.zeros((T, Hkv, D), bool)
+    head[:, -1] = True
+    _close_by_part(*dk, [head, ~head])
+
+    # dQ = dS K: row 50's dS large, key 52's K large (hidden from row 50) in a column where Q is zero.
+    q, k, v, do = inputs()
+    q.view(T, H, D)[:, :, 7] = 0.0
+    do.view(T, H, D)[50, -1, 3], k.view(T, Hkv, D)[52, -1, 7] = big, big
+    dq = run(q, k, v, do)[0]
+    row, col = np.zeros((T, H, D), bool), np.zeros((T, H, D), bool)
+    row[50, -1], col[52:, H - g:, 7] = True, True
+    _close_by_part(*dq, [row, col, ~(row | col)])
