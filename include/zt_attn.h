@@ -236,7 +236,7 @@ int zt_attn_backward_train_ws(const float *q, const float *k, const float *v, co
  * per kv head with head_dim % 4 == 0 and head_dim <= 128 or a multiple of 32;
  * and head groups that cannot be halved (MHA, odd groups) with head_dim 32,
  * 64, 96 or 128 where the grid gives at most one paired dk/dv workgroup per
- * CU (the row-split kernel's shapes).  For the others this is
+ * CU.  For the others this is
  * zt_attn_forward_train and ZT_WS_SCORES is ignored (so it is for q or dout
  * rows that are not 16-byte aligned).  The workspace is the
  * backward's (zt_attn_backward_train_workspace bytes).  No reference
@@ -339,9 +339,9 @@ int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_til
  *   64|128 (dq-from-dS product tile), ZT_ROW_G
  *   1|2|4|8 and ZT_ROW_W 4|8 (query heads and waves per workgroup of the
  *   one-row forward, T = 1), ZT_ATTN_FKS 1|2 (key parts of the forward for
- *   one query head per workgroup: 2 = the key-split eight-wave kernel),
+ *   one query head per workgroup: 2 = the small-grid kernel, keys in two or four parts),
  *   ZT_DQDS_K 1|2 (key parts of the dq-from-dS product), ZT_ATTN_RSCORES
- *   0|1 (the row-split dk/dv kernel reading the forward's scores for head
+ *   0|1 (dk/dv reading the forward's scores for head
  *   groups that cannot be halved; 0 = it forms S again and the forward keeps
  *   none), ZT_ATTN_FSHAPE 11|12|14|21|22 (the forward's wave shape on split
  *   operands, 16-row blocks per wave then key parts; one the kernel does not

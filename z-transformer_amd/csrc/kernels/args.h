@@ -18,7 +18,7 @@ struct FwdArgs {
     int q_offset, n_keys, kv_rows;
     int HW;            // query heads per workgroup (1, 2 or 4; divides H/Hkv)
     int nq, ks;        // split-operand kernels: 16-row blocks per wave, key parts
-    int n_row_tiles;   // ceil(T / (16 * 4 / HW))
+    int n_row_tiles;   // ceil(T / rows of a workgroup): 16 rows a wave and row block, HW heads and ks key parts sharing the waves
     int n_head_blocks; // H / HW
     float scale_log2e; // log2(e) / sqrt(dim)
 };
@@ -46,14 +46,14 @@ struct BwdArgs {
     // (nt = ceil(T/16)), 256 floats in lane order (lane l, element r) =
     // (t = 16 tb + 4 (l >> 4) + r, s = 16 sb + (l & 15)); masked pairs are 0.
     // Tiles above the diagonal have no slot and are never written.
-    // The score-reading dk/dv kernels (zt_bwd_dkdv8s_*, zt_bwd_dkdv_dmas_*)
+    // The score-reading dk/dv kernels (zt_bwd_dkdv8s_*, dmars_*, 8sd_*, dmas_*)
     // find the forward's scaled scores (FwdArgs::s_out) in ds_out on entry;
     // each tile is read before its dS replaces it.
     float *ds_out;
     int B, T, H, Hkv, dim;
     int HW, n_row_tiles, n_head_blocks;  // dq kernel decomposition (as the forward)
     int parts, kblocks;                  // dk/dv on split operands: parts and 16-key blocks per workgroup
-    int HS, n_key_tiles;                 // dk/dv kernel: head split, ceil(T / (16 * 4/HS))
+    int HS, n_key_tiles;                 // dk/dv kernel: head split, ceil(T / keys of a workgroup)
     int pair;                            // both kernels: a workgroup takes tiles p and n - 1 - p
     float scale, scale_log2e;
 };

@@ -1265,8 +1265,12 @@ __device__ __forceinline__ void bwd_dkdv_dma_body(const BwdArgs &a) {
 //     runs beside the other waves' products.
 //   * dV and dK take 32-row sums by f32 adds.
 //   * The parts' dK and dV are summed through LDS in part order: deterministic.
-// What bounds it: LDS operand reads and their latency (74 KB per wave and item at
-// d = 128, against 144 MFMAs of 16 cycles).  With delta, against the f32 MFMA
+// What bounds it (d = 128, T = 4096, counters): MFMAs busy 33 % of the time and vector
+// instructions, four of 4 cycles to each MFMA of 16, as long again; the rest is
+// the waits between dependent products and at barriers (43 % of the waves' cycles)
+// that two waves per SIMD do not cover (a loop of MFMAs with four vector instructions
+// beside each reaches 263 TFLOP/s of f32 products, this kernel 135).  Waits to issue an LDS access are 5 %, without
+// bank conflicts.  With delta, against the f32 MFMA
 // kernels before it: 32 over 8 heads, d = 128, T = 4096 1661 -> 1517 us, T = 512 214
 // -> 177; 4 over 2 heads, d = 32, T = 4096 277 -> 130, T = 256 23.8 -> 13.9; MHA d = 64,
 // 4 x 1024 rows x 8 heads 88 -> 78 us.

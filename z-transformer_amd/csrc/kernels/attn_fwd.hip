@@ -277,10 +277,13 @@ __device__ __forceinline__ void attn_fwd_body(const FwdArgs &a) {
 //     formed from the score registers.
 //   * O accumulates 32-key sums with f32 adds: four vector adds beside six
 //     MFMAs, and a long row takes T / 32 roundings instead of 6 T / 32.
-// What bounds it: on a full chip, power -- operands like these hold a loop of
-// nothing but these MFMAs to 1.8 PFLOP/s, 300 TFLOP/s of f32 products -- and the
-// vector work beside it (a 16 x 16 score block at d = 128 is 48 MFMAs of 16
-// cycles; its softmax and split about 70 vector instructions).  32 over 8 heads,
+// What bounds it: on a full chip the MFMAs, which are busy 55 % of the time, and the
+// vector work beside them, two instructions of 4 cycles to each MFMA of 16 (a 16 x 16
+// score block at d = 128 is 48 MFMAs; its softmax and split about 70 vector
+// instructions), at two waves per SIMD, with power holding the clock to 2.27 GHz (2.15
+// with the scores kept; counters).  A loop of such MFMAs on operands like these
+// reaches 371 TFLOP/s of f32 products alone and 312 with two vector instructions
+// beside each.  32 over 8 heads,
 // d = 128, T = 4096: 1012 us on f32 MFMAs, 614 us here (224 TFLOP/s), with the
 // scores kept 1053 / 705 us; d = 256, 2 x 2048 rows of 16 over 4 heads 538 / 437 us.
 // On small grids, the latency of a step (fetch, split, barrier, two dependent
@@ -745,7 +748,7 @@ DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
     if (threadIdx.x < 4) reinterpret_cast<int *>(smem + C::FLAGS)[threadIdx.x] = 0;
     __syncthreads();
     int sid = 0;
-    // One copy of the tile's code (two cost registers: 43 against 11 spilled at d = 128).
+    // One copy of the tile's code: a second one would cost registers, which at d = 128 spill as it is (2 to 22).
     const int second = a.n_row_tiles - 1 - p;
     int tile = second;
 #pragma unroll 1

@@ -256,7 +256,10 @@ DEVI void gemm_body(const GemmArgs &g) {
 // tile sums are added to the accumulators on the vector ALU, so that K / 32
 // roundings are made at the accumulators' magnitude and not 6 K / 32.  Two
 // workgroups share a CU and cover each other's barriers.  4096^3: 1064 us on f32
-// MFMAs (129 TFLOP/s), 788 us (174 TFLOP/s); bound by power, as the forward.
+// MFMAs (129 TFLOP/s), 760 to 835 us (165 to 181 TFLOP/s).  What bounds it (counters):
+// MFMAs busy 44 % of the time, 3.6 vector instructions of 4 cycles to each MFMA of 16, LDS
+// accesses that wait 13 % of the waves' cycles (6.3 conflict cycles each), and power,
+// which holds the clock to 2.09 GHz.
 template <int BT, bool KC>
 constexpr int slab_bytes() { return KC ? split_bytes(32, BT) : split_bytes(BT, 32); }
 
@@ -683,8 +686,8 @@ DEVI void dq_ds_tile(const DqDsArgs &g, const int tm, const int tn, const int bh
 // gemm_split_tile with both operands index-contiguous, a dS chunk being four
 // queries at one key (eight bytes per part; 16 keys x 4 chunks of a tile cover
 // the banks twice, the least that 512 bytes take).  Loads stay unconditional and
-// in bounds as in dq_ds_tile.  Bound by power and by the splitting of the slabs
-// beside the products, as gemm_split_tile, two workgroups per CU.  32 over 8 heads,
+// in bounds as in dq_ds_tile.  Bound as gemm_split_tile (MFMAs busy 39 %, 4.1 vector
+// instructions to each, 2.3 conflict cycles an LDS access, 2.29 GHz).  32 over 8 heads,
 // d = 128, T = 4096: 558 us on f32 MFMAs (123 TFLOP/s), 458 us here (150 TFLOP/s);
 // that shape's training step 2780 -> 2715 us, 2 x 2048 rows of 16 over 4 heads at
 // d = 256 1791 -> 1733 us.

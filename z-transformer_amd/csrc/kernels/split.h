@@ -2,8 +2,9 @@
 //
 // v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s on gfx950 and, as measured here,
 // shares the SIMD with the vector ALU; v_mfma_f32_16x16x32_bf16 runs at 16
-// times that rate (2.28-2.41 PFLOP/s measured with two waves per SIMD) beside
-// up to two vector instructions per MFMA.  So an f32 operand x is written as
+// times that rate: 2.24 PFLOP/s measured with two waves per SIMD on the parts of N(0, 1)
+// values (2.48 on zeros: power), 1.87 with two vector instructions beside each MFMA,
+// 1.58 with four.  So an f32 operand x is written as
 // x = h + m + l, three bf16 values of 8 significant bits each (h = bf16(x), m =
 // bf16(x - h), l = x - h - m: together all 24 bits of x, both subtractions
 // exact), and a product as the six partial products above 2^-24 of it,

@@ -231,12 +231,14 @@ int key_tile(Tiled which, int dp, int max_tile, int dim = 0) {
 size_t fwd_tile_bytes(int dp, int bk) { return (size_t)2 * bk * (dp + 4) * sizeof(float); }
 size_t kv_tile_bytes(int dp, int bk) { return (size_t)2 * bk * (dp + 4) * sizeof(float); }
 
-// Waves per forward / dq workgroup (4 or 8): eight waves share each staged K/V
-// tile between twice as many query rows.  Measured on MI355X: the forward
-// gains when four query heads share a kv group (C3 1.39 -> 1.33 ms, C5 0.84 ->
-// 0.76 ms) and, with the register prefetch, when two do (B = 4, T = 2048, 16
-// heads over 8, d = 128: 0.647 -> 0.581 ms; d = 256, B = 2: 0.711 -> 0.588 ms);
-// it loses for MHA (C2 0.057 -> 0.076 ms); the dq kernel loses at every shape tried.
+// Waves per workgroup of the f32 MFMA forward (d = 160, 224, and rows that are not
+// whole 16-byte chunks; split operands take eight, fwd_plan): eight waves share each
+// staged K/V tile between twice as many query rows.  Measured on MI355X (us, four /
+// eight waves): four heads of a kv group 2 x 2048 rows at d = 160 453 / 382, 4 x 1024 at d =
+// 66 203 / 174; two 2 x 2048 at d = 130 712 / 578; MHA 2 x 1024 at d = 160 113 / 180, d = 224
+// 160 / 241 (but d = 66 204 / 165, d = 250 461 / 398, and one sequence of 16 over 4
+// heads at d = 224 325 / 477: the line is the head group's, not the width's).  The dq
+// kernel loses with eight at every shape tried.
 int fwd_waves(int hw) { return tuned(kTuneFwdW, hw >= 2 ? 8 : 4); }
 
 // The forward's kernel and the work of its waves.  nw waves per workgroup,
@@ -255,14 +257,13 @@ bool fwd_splits(int dim, int dp, int bk) {
     return bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1 && fwd_split_width(dp);
 }
 
-// Key parts of the forward: 1, or 2 for the key-split kernel (zt_fwdpk_*:
-// eight waves, 4 row blocks x 2 key parts merged at the end) for one query
-// head per workgroup (HW = 1) where the four-wave kernel's grid, after
-// pairing, gives at most one workgroup per CU: one wave per SIMD there, and
-// the split doubles it for the same rows.  Measured on MI355X (training
-// forward): C2 60.8 -> 51.3 us, one 16-head sequence of 2048 rows at d = 64
-// 104.5 -> 85.5 us, 12 heads of 1024 rows at d = 128, B = 2, 94.9 -> 89.5 us.
-// Needs the prefetching kernel (32-key tiles, dim % 4 == 0) and d <= 128.
+// 2 where one query head per workgroup (HW = 1) takes the small-grid kernel on split
+// operands (zt_fwdpk_*: waves of one row block, two or four key parts merged at the
+// end), else 1: where paired 64-row tiles give at most one workgroup per CU.
+// Measured on MI355X (training forward, us, without / with): one sequence of 8
+// heads, 512 rows at d = 64 24.3 / 19.0, 1024 at d = 32 30.8 / 21.9; equal near the line, 4
+// x 1024 rows of 8 heads at d = 64 52.6 / 52.4, 2 x 1024 of 12 at d = 128 74.6 / 75.5; past it
+// 8 x 1024 of 8 at d = 64 71.7 / 91.9.  Needs 32-key tiles, dim % 4 == 0 and d <= 128.
 int fwd_key_split(int B, int T, int n_heads, int hw, int dp, int dim, int bk, int cus) {
     const bool able = hw == 1 && dp <= 128 && bk == 32 && dim % 4 == 0 && tuned(kTuneFPF, 1) == 1;
     const long long tiles = (T + 63) / 64;  // 64-row tiles (4 row blocks) per head
@@ -898,20 +899,19 @@ size_t zt_attn_backward_train_workspace(int B, int T, int n_heads, int n_kv_head
            (size_t)B * n_heads * (size_t)zt_tri_count(nt) * 256 * sizeof(float);
 }
 
-// Which dk/dv kernel takes the forward's scores instead of rebuilding them,
-// if any.  Split: an even head group (two-way head split) with 16-byte row
-// chunks (d % 4 == 0): up to d = 128 the eight-wave kernel with 32 query rows
-// per stage, above it the asynchronously staged kernel (whole-head rows: d a
-// multiple of 32).  RowSplit: a group that cannot be halved (MHA, odd groups)
-// where the statistics path takes the row-split asynchronously staged kernel
-// (whole-head rows up to d = 128, at most one paired workgroup per CU): the
-// same kernel reading the scores (ZT_ATTN_RSCORES=0 keeps it forming S
-// again).  Measured on MI355X (training step, scores against none): C2
-// 179.6 -> 171.8-177.9 us, one 16-head MHA sequence of 2048 rows at d = 128
-// 582 -> 530 us, B = 2, T = 1024, 12 over 4 heads at d = 64 320 -> 291 us,
-// one 8-head sequence of 1024 rows at d = 96 217 -> 202 us; the forward pays
-// 4-5 us for its score stores at each.  The forward writes scores only for
-// these.
+// Whether dk/dv takes the forward's scores instead of rebuilding them, with 16-byte
+// row chunks (d % 4 == 0) throughout; the forward writes scores only for these.  Up
+// to d = 128 the kernel that reads them is the split-operand one, whatever the group.
+// Split: an even head group; above d = 128 the column-split or asynchronously staged
+// kernel (whole-head rows: d a multiple of 32).  RowSplit: a group that cannot be
+// halved (MHA, odd groups), on the shapes where the statistics path takes its row-split
+// kernel (whole-head rows up to d = 128, at most one paired workgroup per CU): the line
+// that was measured for that kernel's own score-reading form, not yet for the one
+// that reads them now, which needs neither (ZT_ATTN_RSCORES=0: no scores).  Measured on
+// MI355X (training step, us, without / with scores): 4 x 1024 rows of 8 heads at d = 64
+// 189 / 169, one 16-head sequence of 2048 rows at d = 128 545 / 436, 2 x 1024 of 12 over 4
+// heads at d = 64 318 / 200, one 8-head sequence of 1024 rows at d = 96 205 / 164, of 512 at
+// d = 32 65 / 49.
 enum class ScoreKernel { None, Split, RowSplit };
 static ScoreKernel score_kernel(int B, int T, int dim, int n_heads, int n_kv_heads, const DeviceState *st) {
     const int dp = pad32(dim);
@@ -1082,7 +1082,7 @@ int zt_attn_backward_train_ws(const float *q, const float *k, const float *v, co
     const int dp = pad32(dim);
     const bool qd_aligned = (uintptr_t)q % 16 == 0 && (uintptr_t)dout % 16 == 0;
     const ScoreKernel sk = score_kernel(B, T, dim, n_heads, n_kv_heads, st);
-    // (RowSplit reads them on the grid backward_prepare sized for the row-split kernel.)
+    // (RowSplit: only where backward_prepare picked the row-split kernel as well, as score_kernel's line has it.)
     const bool read_scores = scores && (stage & 1) && sk != ScoreKernel::None && qd_aligned &&
                              (sk != ScoreKernel::RowSplit || strncmp(name_b, "zt_bwd_dkdv_dmar_d", 18) == 0);
     if (read_scores &&
