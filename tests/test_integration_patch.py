@@ -24,8 +24,9 @@ REFERENCE = "/root/reference"
 FILES = ["build.zig", "src/cuda/device.zig", "src/model.zig", "src/autograd.zig"]
 LIB = os.path.join(REPO, "z-transformer_amd", "_build", "libzt_attn.so")
 
-needs_reference = pytest.mark.skipif(not os.path.isdir(REFERENCE) or shutil.which("git") is None,
-                                     reason="the reference tree or git is absent")
+# (An empty directory where the tree would be is an absent tree.)
+HAS_REFERENCE = all(os.path.isfile(os.path.join(REFERENCE, f)) for f in FILES) and shutil.which("git") is not None
+needs_reference = pytest.mark.skipif(not HAS_REFERENCE, reason="the reference tree or git is absent")
 
 
 def _patched_files(patch_text):
@@ -51,7 +52,7 @@ def test_the_patch_touches_exactly_the_binding_files():
 
 @pytest.fixture(scope="module")
 def patched(tmp_path_factory):
-    if not os.path.isdir(REFERENCE) or shutil.which("git") is None:
+    if not HAS_REFERENCE:
         pytest.skip("the reference tree or git is absent")
     d = tmp_path_factory.mktemp("ref")
     for f in FILES:
