@@ -59,9 +59,9 @@ def test_shmem_counts(zt):
     assert L.zt_attn_forward_shmem(33, 64, 1) == 0 and L.zt_attn_bwd_dkdv_shmem(300) == 0
 
 
-def _static_lds():
-    """kernel name -> static LDS bytes, from the metadata of the code objects that build.py leaves beside the library."""
-    lds = {}
+def _kernel_metadata(field):
+    """kernel name -> a number of its metadata, from the code objects that build.py leaves beside the library."""
+    values = {}
     for tag in ("fwd", "bwd"):
         co = open(os.path.join(ROOT, "z-transformer_amd", "_build", f"{tag}.hsaco"), "rb").read()
         with tempfile.NamedTemporaryFile(suffix=".elf") as f:
@@ -69,17 +69,18 @@ def _static_lds():
             f.flush()
             readelf = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
             notes = subprocess.run([readelf, "--notes", f.name], check=True, stdout=subprocess.PIPE, text=True).stdout
-        for size, name in re.findall(r"\.group_segment_fixed_size: (\d+).*?\.name:\s+(zt_\w+)", notes, re.S):
-            lds[name] = int(size)
-    assert len(lds) > 100
-    return lds
+        for entry in notes.split("  - .agpr_count")[1:]:  # one per kernel
+            name = re.search(r"\.name:\s+(zt_\w+)", entry).group(1)
+            values[name] = int(re.search(rf"\.{field}:\s+(\d+)", entry).group(1))
+    assert len(values) > 100
+    return values
 
 
 def test_shmem_counts_are_the_kernels_lds(zt):
     """The most static LDS among the kernels that a width can launch: 16-byte
     rows (dim % 4 == 0) take the split-operand and prefetching kernels, whole
     widths (a multiple of 32) the asynchronously staged and column-split ones."""
-    L, lds = zt.lib(), _static_lds()
+    L, lds = zt.lib(), _kernel_metadata("group_segment_fixed_size")
 
     def most(pattern):
         return max(size for name, size in lds.items() if re.fullmatch(pattern, name))
@@ -90,7 +91,7 @@ def test_shmem_counts_are_the_kernels_lds(zt):
                 continue
             rows16, whole = dim % 4 == 0, dim == dp
             if rows16:
-                fwd32 = fwd64 = most(rf"zt_fwd(8p|8ps|p|pk)_d{dp}_k32")
+                fwd32 = fwd64 = most(rf"zt_fwd(8p|8ps|p|pk)_d{dp}_k32(_\d+)?")
             else:
                 fwd32 = most(rf"zt_fwd8?_d{dp}_k32")
                 fwd64 = most(rf"zt_fwd8?_d{dp}_k{64 if dp <= 64 else 32}")
@@ -98,11 +99,21 @@ def test_shmem_counts_are_the_kernels_lds(zt):
             assert L.zt_attn_bwd_dq_shmem(dim, 64) == most(rf"zt_bwd_dq(8|p|8p|l)?_d{dp}_k32"), dim
             kinds = ["_d{0}_hs[124]"]
             if dp <= 128:
-                kinds += ["8_d{0}_hs2"] + (["8p_d{0}_hs2", "8s_d{0}_hs2"] if rows16 else [])
+                kinds += ["8_d{0}_hs2"] + (["8p_d{0}_hs2", "8s_d{0}_hs2_[0-9]+"] if rows16 else [])
             if whole:
-                kinds += ["_dma_d{0}_hs[124]", "_dmar_d{0}", "_dmars_d{0}", "_dmas_d{0}_hs2", "8pd_d{0}_hs[12]",
+                kinds += ["_dma_d{0}_hs[124]", "_dmar_d{0}", "_dmars_d{0}_[0-9]+", "_dmas_d{0}_hs2", "8pd_d{0}_hs[12]",
                           "8sd_d{0}_hs2"]
             assert L.zt_attn_bwd_dkdv_shmem(dim) == most("zt_bwd_dkdv(" + "|".join(kinds).format(dp) + ")"), dim
+
+
+def test_two_workgroups_of_the_narrowest_head_share_a_cu():
+    """At d = 32 the shapes of the larger grids (one row block and two key parts;
+    four parts of two key blocks) rest on two eight-wave workgroups per CU: half of
+    its 160 KB of LDS each, and 128 of a SIMD's 512 registers per wave."""
+    lds, vgpr = _kernel_metadata("group_segment_fixed_size"), _kernel_metadata("vgpr_count")
+    for name in ("zt_fwd8p_d32_k32_812", "zt_fwd8ps_d32_k32_812", "zt_fwdp_d32_k32_812", "zt_bwd_dkdv8s_d32_hs2_42",
+                 "zt_bwd_dkdv_dmars_d32_42"):
+        assert 2 * lds[name] <= 160 * 1024 and vgpr[name] <= 128, name
 
 
 def _fwd(L, T=8, H=4, Hkv=2, dim=32, group_q=1, max_tile=64, q_offset=0, n_keys=8):

@@ -17,7 +17,6 @@ struct FwdArgs {
     int B, T, H, Hkv, dim;
     int q_offset, n_keys, kv_rows;
     int HW;            // query heads per workgroup (1, 2 or 4; divides H/Hkv)
-    int nq, ks;        // split-operand kernels: 16-row blocks per wave, key parts
     int n_row_tiles;   // ceil(T / rows of a workgroup): 16 rows a wave and row block, HW heads and ks key parts sharing the waves
     int n_head_blocks; // H / HW
     float scale_log2e; // log2(e) / sqrt(dim)
@@ -52,7 +51,6 @@ struct BwdArgs {
     float *ds_out;
     int B, T, H, Hkv, dim;
     int HW, n_row_tiles, n_head_blocks;  // dq kernel decomposition (as the forward)
-    int parts, kblocks;                  // dk/dv on split operands: parts and 16-key blocks per workgroup
     int HS, n_key_tiles;                 // dk/dv kernel: head split, ceil(T / keys of a workgroup)
     int pair;                            // both kernels: a workgroup takes tiles p and n - 1 - p
     float scale, scale_log2e;

@@ -1591,10 +1591,10 @@ DEVI void dkdv_split_tile(const BwdArgs &a, const int kt, const int kvh, const i
     __syncthreads();  // the merge's reads before the next tile's staging
 }
 
-// One of a kernel's shapes (shapes.h), picked by the launch (BwdArgs::parts, kblocks).
+// A kernel per width and shape (shapes.h), of which the launcher picks by the grid.
 template <int DP, int NPART, int NKB>
-DEVI bool dkdv_shape(const BwdArgs &a, char *smem) {
-    if (a.parts != NPART || a.kblocks != NKB) return false;  // workgroup-uniform
+DEVI void dkdv_split_kernel(const BwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds(DP, {NPART, NKB})];
     if (threadIdx.x < 2 * NPART) reinterpret_cast<int *>(smem + BwdSplit<DP, NPART, NKB>::FLAGS)[threadIdx.x] = 0;
     __syncthreads();
     const int per = a.Hkv * a.B, rem = (int)blockIdx.x % per, p = (int)blockIdx.x / per;
@@ -1608,18 +1608,23 @@ DEVI bool dkdv_shape(const BwdArgs &a, char *smem) {
         if (!a.pair || kt == second || second <= p) break;
         kt = second;
     }
-    return true;
 }
-template <int DP>
-DEVI void dkdv_shapes(const BwdArgs &a) {
-    __shared__ __attribute__((aligned(16))) char smem[dkdv_lds(DP)];
-    constexpr BwdWavesList L = dkdv_waves(DP);
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-        (void)(dkdv_shape<DP, L.s[I].parts, L.s[I].kblocks>(a, smem) || ...);
-    }(std::make_integer_sequence<int, L.n>{});
-}
-#define ZT_BWD_SPLIT(NAME, DP)                                                                      \
-    extern "C" __global__ void __launch_bounds__(512, 2) NAME(BwdArgs a) { dkdv_shapes<DP>(a); }
+// Bounds of 512 threads for four waves too: given 512 registers per wave the compiler
+// keeps values in accumulation registers, at a copy per use (d = 128, 32 over 8 heads,
+// T = 512: 180 us, 193 with bounds of 256).
+#define ZT_DKDV_K(NAME, DP, NPART, NKB)                                                             \
+    extern "C" __global__ void __launch_bounds__(512, 2)                                    \
+    NAME##_##NPART##NKB(BwdArgs a) {                                                                 \
+        dkdv_split_kernel<DP, NPART, NKB>(a);                                                        \
+    }
+#define ZT_8S_32(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv8s_d32_hs2, 32, NPART, NKB)
+#define ZT_8S_64(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv8s_d64_hs2, 64, NPART, NKB)
+#define ZT_8S_96(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv8s_d96_hs2, 96, NPART, NKB)
+#define ZT_8S_128(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv8s_d128_hs2, 128, NPART, NKB)
+#define ZT_RS_32(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv_dmars_d32, 32, NPART, NKB)
+#define ZT_RS_64(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv_dmars_d64, 64, NPART, NKB)
+#define ZT_RS_96(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv_dmars_d96, 96, NPART, NKB)
+#define ZT_RS_128(NPART, NKB) ZT_DKDV_K(zt_bwd_dkdv_dmars_d128, 128, NPART, NKB)
 
 #define ZT_BWD_DQ(DP, BK)                                                                          \
     extern "C" __global__ void __launch_bounds__(256, (DP) <= ((BK) == 32 ? 192 : 128) ? 2 : 1)  \
@@ -1656,8 +1661,8 @@ DEVI void dkdv_shapes(const BwdArgs &a) {
     extern "C" __global__ void __launch_bounds__(512) zt_bwd_dkdv8p_d##DP##_hs2(BwdArgs a) {    \
         bwd_dkdv_body<DP, 2, 4, true>(a);                                                          \
     }
-// dk/dv that reads the forward's scores, on split operands: one kernel under two
-// names, for head groups of two and more (dkdv8s) and for one that cannot be halved
+// dk/dv that reads the forward's scores, on split operands: the same kernels under two
+// names (8S, RS above), for head groups of two and more (dkdv8s) and for one that cannot be halved
 // (dmars), so that a profile tells the two apart.
 #define ZT_BWD_DKDV_DMA(DP, HS)                                                                    \
     extern "C" __global__ void __launch_bounds__(256) zt_bwd_dkdv_dma_d##DP##_hs##HS(BwdArgs a) { \
@@ -1678,10 +1683,10 @@ ZT_BWD_ALL(64)
 ZT_BWD_ALL(96)
 ZT_BWD_ALL(128)
 ZT_BWD_DKDV8(32) ZT_BWD_DKDV8(64) ZT_BWD_DKDV8(96) ZT_BWD_DKDV8(128)
-ZT_BWD_SPLIT(zt_bwd_dkdv8s_d32_hs2, 32)
-ZT_BWD_SPLIT(zt_bwd_dkdv8s_d64_hs2, 64)
-ZT_BWD_SPLIT(zt_bwd_dkdv8s_d96_hs2, 96)
-ZT_BWD_SPLIT(zt_bwd_dkdv8s_d128_hs2, 128)
+ZT_DKDV_32(ZT_8S_32)
+ZT_DKDV_64(ZT_8S_64)
+ZT_DKDV_96(ZT_8S_96)
+ZT_DKDV_128(ZT_8S_128)
 // The 4-way splits: the 160 KB LDS holds 4 parts' tiles (double-buffered for
 // the asynchronous variant) up to d = 128.
 ZT_BWD_DKDV(32, 4)
@@ -1696,10 +1701,10 @@ ZT_BWD_DKDV(128, 4)
     }
 ZT_BWD_DKDV_DMAR(32) ZT_BWD_DKDV_DMAR(64) ZT_BWD_DKDV_DMAR(96) ZT_BWD_DKDV_DMAR(128)
 // The same reading the forward's scores.
-ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d32, 32)
-ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d64, 64)
-ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d96, 96)
-ZT_BWD_SPLIT(zt_bwd_dkdv_dmars_d128, 128)
+ZT_DKDV_32(ZT_RS_32)
+ZT_DKDV_64(ZT_RS_64)
+ZT_DKDV_96(ZT_RS_96)
+ZT_DKDV_128(ZT_RS_128)
 ZT_BWD_DKDV_DMA(32, 4)
 ZT_BWD_DKDV_DMA(64, 4)
 ZT_BWD_DKDV_DMA(96, 4)
@@ -1739,7 +1744,7 @@ ZT_BWD_DKDV8PD1(64) ZT_BWD_DKDV8PD1(128)
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
 ZT_BWD_DQ_PF(32) ZT_BWD_DQ_LSE(32) ZT_BWD_DKDV8(32)
-ZT_BWD_SPLIT(zt_bwd_dkdv8s_d128_hs2, 128)
+ZT_DKDV_128(ZT_8S_128)
 #endif
 
 // delta[row] = sum_d o[row, d] * dout[row, d] over the B*T*H rows of dim

@@ -271,14 +271,13 @@ int fwd_key_split(int B, int T, int n_heads, int hw, int dp, int dim, int bk, in
     return able ? tuned(kTuneFKS, wgs <= cus ? 2 : 1) : 1;
 }
 
-// The role of p's kernel, and whether that kernel holds p's wave shape.
+// The role of p's kernel, and whether it is built in p's wave shape.
 FwdRole fwd_role(const FwdPlan &p) {
     return p.nw == 8 && p.hw > 1 ? FwdRole::Heads : p.small ? FwdRole::Small : FwdRole::One;
 }
 bool fwd_shape_built(const FwdPlan &p, int dp) {
-    const FwdWavesList l = fwd_waves(fwd_role(p), dp);
-    for (int i = 0; i < l.n; ++i)
-        if (l.s[i].nw == p.nw && l.s[i].nq == p.nq && l.s[i].ks == p.ks) return true;
+    for (const FwdWaves &s : fwd_waves(fwd_role(p), dp).s)
+        if (s.nw == p.nw && s.nq == p.nq && s.ks == p.ks) return true;
     return false;
 }
 
@@ -291,9 +290,13 @@ bool fwd_shape_built(const FwdPlan &p, int dp) {
 // 285 / 235, T = 4096 610 / 860 (kept); 4 over 2 heads at d = 32, T = 256
 // 20 / 9.2 (two key parts 11), T = 4096 237 / 64; MHA at d = 64, 4 x 1024 rows x 8
 // heads 56 (two row blocks, two key parts) / 47, one sequence of 512 rows
-// 30 / 16 (four key parts).  Up to d = 64 grids of half to one workgroup per CU
-// keep both row blocks and split the keys: 8 x 2048 rows of 4 over 2 heads at d
-// = 32 125 / 86 (one row block 111), 8 x 1024 of 8 MHA heads at d = 64 85 / 66 (84).
+// 30 / 16 (four key parts).  At d = 64 grids of half to one workgroup per CU
+// keep both row blocks and split the keys: 8 x 1024 of 8 MHA heads 85 / 66 (one row
+// block 84).  At d = 32 one row block and two key parts leave room for two workgroups
+// per CU (shapes.h) and win on larger grids as well: widest / chosen 8 x 1070 rows of
+// 8 MHA heads 97 / 61, one of 2060 rows of 32 over 8 heads 137 / 104; but with four
+// heads per workgroup not where the widest, paired, fill three quarters of the CUs to
+// all of them: 4 x 896 rows of 32 over 8 heads 71 / 83, one of 3355 233 / 255 (kept).
 FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int bk, int cus) {
     FwdPlan p{};
     p.hw = heads_per_wg(n_heads / n_kv_heads);
@@ -313,18 +316,22 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
         const long long rows32 = (long long)((T + 31) / 32) * n_heads * B;
         p.nq = 1;
         p.ks = dp <= 64 && rows32 <= cus ? 4 : 2;
-    } else if (p.nw == 8 && wide <= cus) {
+    } else if (p.nw == 8 && (wide <= cus || (dp == 32 && !(p.hw == 4 && 2 * wide > 3 * cus && wide <= 2 * cus)))) {
         p.nq = 1;
         p.ks = p.ds > 1 ? 1 : 2;
-        if (dp <= 64 && 2 * wide > cus) p.nq = 2;
+        if (dp == 64 && 2 * wide > cus) p.nq = 2;
         if (p.hw == 2 && dp == 32 && (long long)((T + 15) / 16) * (n_heads / p.hw) * B <= 2 * cus) p.ks = 4;
     }
     const int shape = tuned(kTuneFShape, 10 * p.nq + p.ks);
     p.nq = shape / 10;
     p.ks = shape % 10;
-    if (!fwd_shape_built(p, dp)) {  // a forced shape the kernel does not hold
-        p.nq = p.small ? 1 : 2;
-        p.ks = p.small ? 2 : 1;
+    if (!fwd_shape_built(p, dp)) {  // a forced shape that the role is not built in
+        for (const FwdWaves &s : fwd_waves(fwd_role(p), dp).s)
+            if (s.nw == p.nw) {
+                p.nq = s.nq;
+                p.ks = s.ks;
+                break;
+            }
     }
     while (p.nw / (p.ks * p.ds) < p.hw) p.hw /= 2;
     return p;
@@ -332,7 +339,7 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
 
 // The LDS its kernel takes per workgroup.
 size_t fwd_plan_lds(const FwdPlan &p, int dp, int bk) {
-    return p.split ? (size_t)fwd_lds(fwd_role(p), dp) : fwd_tile_bytes(dp, bk);
+    return p.split ? (size_t)fwd_lds(dp, FwdWaves{p.nw, p.nq, p.ks}) : fwd_tile_bytes(dp, bk);
 }
 
 // Forward kernel name: the split-operand kernels, and the f32 MFMA kernels for
@@ -559,7 +566,7 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     a.q = q; a.k = k; a.v = v; a.out = out; a.lse = lse; a.s_out = s_out;
     a.B = B; a.T = T; a.H = n_heads; a.Hkv = n_kv_heads; a.dim = dim;
     a.q_offset = q_offset; a.n_keys = n_keys; a.kv_rows = kv_rows;
-    a.HW = p.hw; a.nq = p.nq; a.ks = p.ks;
+    a.HW = p.hw;
     const int rows_per_wg = fwd_rows(p);
     a.n_row_tiles = (T + rows_per_wg - 1) / rows_per_wg;
     a.n_head_blocks = n_heads / a.HW;
@@ -574,6 +581,10 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     if (!grid_ok(blocks, 64u * p.nw)) return 1;
     char name[64];
     fwd_kernel_name(name, sizeof name, dim, dp, bk, p, s_out != nullptr);
+    if (p.split) {  // the shape's kernel (shapes.h)
+        const size_t n = strlen(name);
+        snprintf(name + n, sizeof name - n, "_%d%d%d", p.nw, p.nq, p.ks);
+    }
     return launch(st, name, (unsigned)blocks, a, stream, 64u * p.nw);
 }
 
@@ -773,7 +784,7 @@ size_t zt_attn_forward_shmem(int dim, int tile, int group_q) {
     (void)group_q;
     if (!zt_attn_dim_ok(dim)) return 0;
     const int dp = pad32(dim), bk = key_tile(Tiled::Forward, dp, tile, dim);
-    return fwd_splits(dim, dp, bk) ? (size_t)fwd_lds(dp) : fwd_tile_bytes(dp, bk);
+    return fwd_splits(dim, dp, bk) ? (size_t)fwd_lds_most(dp) : fwd_tile_bytes(dp, bk);
 }
 
 size_t zt_attn_bwd_dq_shmem(int dim, int tile) {
@@ -789,7 +800,7 @@ size_t zt_attn_bwd_dkdv_shmem(int dim) {
     size_t most = dkdv_bytes(dp, hs);
     if (dp <= 128) {  // eight waves: register-prefetched, and reading the forward's scores
         most = std::max(most, dkdv_bytes(dp, 2, 4));
-        if (dim % 4 == 0) most = std::max(most, std::max(dkdv_bytes(dp, 2, 4, 16, 2), (size_t)dkdv_lds(dp)));
+        if (dim % 4 == 0) most = std::max(most, std::max(dkdv_bytes(dp, 2, 4, 16, 2), (size_t)dkdv_lds_most(dp)));
     }
     if (dim == dp) {  // whole-head rows: asynchronously staged, and column-split eight waves
         most = std::max(most, dkdv_dma_bytes(dp, hs));
@@ -917,7 +928,7 @@ static ScoreKernel score_kernel(int B, int T, int dim, int n_heads, int n_kv_hea
     const int dp = pad32(dim);
     if (n_kv_heads <= 0 || n_heads % n_kv_heads != 0 || dim % 4 != 0) return ScoreKernel::None;
     if ((n_heads / n_kv_heads) % 2 == 0) {
-        const bool fits = dp <= 128 ? (size_t)dkdv_lds(dp) <= st->lds_limit
+        const bool fits = dp <= 128 ? (size_t)dkdv_lds_most(dp) <= st->lds_limit
                                     : dim == dp && dkdv_dma_bytes(dp, 2) <= st->lds_limit;
         return fits ? ScoreKernel::Split : ScoreKernel::None;
     }
@@ -925,7 +936,7 @@ static ScoreKernel score_kernel(int B, int T, int dim, int n_heads, int n_kv_hea
     const unsigned long long tiles = (unsigned long long)(T + 63) / 64;
     const bool dma_pays = (tiles + 1) / 2 * n_kv_heads * B <= (unsigned long long)st->cus;
     const bool rsplit = dim == dp && dp <= 128 && dkdv_dma_bytes(dp, 2) <= st->lds_limit &&
-                        (size_t)dkdv_lds(dp) <= st->lds_limit && tuned(kTuneDMA, dma_pays ? 1 : 0) == 1 &&
+                        (size_t)dkdv_lds_most(dp) <= st->lds_limit && tuned(kTuneDMA, dma_pays ? 1 : 0) == 1 &&
                         tuned(kTuneRSplit, 1) == 1;
     return rsplit && tuned(kTuneRScores, 1) == 1 ? ScoreKernel::RowSplit : ScoreKernel::None;
 }
@@ -943,19 +954,23 @@ static float *ws_tiles(void *workspace, int B, int T, int n_heads) {
 // lists where 64-key tiles leave CUs idle.  Measured on MI355X with delta (us,
 // blocks 4 / 2 / 1): 4 over 2 heads at d = 32, T = 4096 406 / 213 / 130, T = 256
 // 31 / 19 / 14; 12 over 4 heads at d = 64, 4 x 512 rows 96 / 63 / 72; 32 over 8 at d =
-// 128, T = 512 182 / 177, T = 4096 1517 / 2784.
+// 128, T = 512 182 / 177, T = 4096 1517 / 2784.  At d = 32 four parts of two blocks
+// leave room for two workgroups per CU (shapes.h) and win on every larger grid:
+// one sequence of 2060 rows of 32 over 8 heads 445 / 283, 4 x 896 218 / 179.
 static void dkdv_split_shape(int B, int T, int n_kv_heads, int dp, int cus, int *parts, int *kblocks) {
     const long long wgs = (long long)((T + 63) / 64) * n_kv_heads * B;  // 64 keys each
-    int kb = 4;
-    if (2 * wgs <= cus || (dp == 32 && wgs <= cus)) kb = 2;
+    int kb = dp == 32 ? 2 : 4;
+    if (2 * wgs <= cus && dp > 32) kb = 2;
     if ((4 * wgs <= cus && dp <= 64) || (dp == 32 && 2 * wgs <= cus)) kb = 1;
     kb = tuned(kTuneBShape, kb);
     // The shape of kb blocks, or the last (fewest blocks) where the kernel has none.
     const BwdWavesList l = dkdv_waves(dp);
-    int i = 0;
-    while (i + 1 < l.n && l.s[i].kblocks != kb) ++i;
-    *kblocks = l.s[i].kblocks;
-    *parts = l.s[i].parts;
+    for (const BwdWaves &s : l.s) {
+        if (!s.parts) break;
+        *kblocks = s.kblocks;
+        *parts = s.parts;
+        if (s.kblocks == kb) break;
+    }
 }
 
 // Which workspaces hold scores, and of what.  zt_attn_forward_train_ws stamps
@@ -1096,17 +1111,20 @@ int zt_attn_backward_train_ws(const float *q, const float *k, const float *v, co
     if (read_scores && dp <= 128) {
         // The forward left the scores in the dS tiles: the split-operand kernel,
         // whose shape follows the grid.
-        dkdv_split_shape(B, T, n_kv_heads, dp, st->cus, &a.parts, &a.kblocks);
-        const int keys = 16 * a.kblocks;
+        int parts = 0, kblocks = 0;
+        dkdv_split_shape(B, T, n_kv_heads, dp, st->cus, &parts, &kblocks);
+        const int keys = 16 * kblocks;
         a.n_key_tiles = (T + keys - 1) / keys;
         a.pair = tuned(kTuneBPair, pair_pays((unsigned long long)a.n_key_tiles * n_kv_heads * B, st->cus));
         const unsigned long long blocks =
             (unsigned long long)(a.pair ? (a.n_key_tiles + 1) / 2 : a.n_key_tiles) * n_kv_heads * B;
-        threads_b = 64u * a.parts * a.kblocks;
+        threads_b = 64u * parts * kblocks;
         if (!grid_ok(blocks, threads_b)) return 1;
         blocks_b = (unsigned)blocks;
         snprintf(name_b, sizeof name_b,
                  sk == ScoreKernel::RowSplit ? "zt_bwd_dkdv_dmars_d%d" : "zt_bwd_dkdv8s_d%d_hs2", dp);
+        const size_t n = strlen(name_b);
+        snprintf(name_b + n, sizeof name_b - n, "_%d%d", parts, kblocks);  // the shape's kernel (shapes.h)
     } else if (read_scores) {
         // Wider heads, 2 head halves x 32 keys: eight waves splitting the columns,
         // or four waves with asynchronous staging.  (Unaligned q / dout rows form
