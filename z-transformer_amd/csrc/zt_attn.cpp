@@ -959,9 +959,10 @@ static float *ws_tiles(void *workspace, int B, int T, int n_heads) {
 // one sequence of 2060 rows of 32 over 8 heads 445 / 283, 4 x 896 218 / 179.
 static void dkdv_split_shape(int B, int T, int n_kv_heads, int dp, int cus, int *parts, int *kblocks) {
     const long long wgs = (long long)((T + 63) / 64) * n_kv_heads * B;  // 64 keys each
-    int kb = dp == 32 ? 2 : 4;
-    if (2 * wgs <= cus && dp > 32) kb = 2;
-    if ((4 * wgs <= cus && dp <= 64) || (dp == 32 && 2 * wgs <= cus)) kb = 1;
+    int kb = 4;
+    if (dp == 32) kb = 2 * wgs <= cus ? 1 : 2;
+    else if (dp == 64) kb = 4 * wgs <= cus ? 1 : wgs < cus ? 2 : 4;
+    else if (2 * wgs <= cus) kb = 2;
     kb = tuned(kTuneBShape, kb);
     // The shape of kb blocks, or the last (fewest blocks) where the kernel has none.
     const BwdWavesList l = dkdv_waves(dp);
