@@ -316,10 +316,11 @@ int zt_fill_uniform(float *dst, size_t n, uint64_t seed, double lo, double hi, h
 
 /* The kernel names this library launches for a forward and a backward at
  * this shape on the current device (for profilers and benchmarks), each
- * written NUL-terminated into a buffer of `len` bytes.  Kernels on split
- * operands are built once per wave shape: their symbols have the shape's
- * digits behind the name given here (zt_fwd8p_d64_k32_812).  1 if the shape
- * is refused or no device is usable. */
+ * written NUL-terminated into a buffer of `len` bytes.  Where
+ * each wave shape is a kernel of its own (the forward at head_dim 32, dk/dv
+ * reading the scores up to 128) its symbol has the shape's digits behind the
+ * name given here (zt_fwd8p_d32_k32_812).  1 if the shape is refused or no
+ * device is usable. */
 int zt_attn_plan(int B, int T, int n_heads, int n_kv_heads, int dim, int max_tile, char *fwd, char *dq,
                  char *dkdv, size_t len);
 

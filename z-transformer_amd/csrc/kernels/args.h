@@ -17,6 +17,7 @@ struct FwdArgs {
     int B, T, H, Hkv, dim;
     int q_offset, n_keys, kv_rows;
     int HW;            // query heads per workgroup (1, 2 or 4; divides H/Hkv)
+    int nq, ks;        // split-operand kernels: 16-row blocks per wave, key parts
     int n_row_tiles;   // ceil(T / rows of a workgroup): 16 rows a wave and row block, HW heads and ks key parts sharing the waves
     int n_head_blocks; // H / HW
     float scale_log2e; // log2(e) / sqrt(dim)

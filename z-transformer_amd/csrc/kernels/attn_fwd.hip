@@ -765,39 +765,42 @@ DEVI void fwd_split_body(const FwdArgs &a, char *smem) {
     extern "C" __global__ void __launch_bounds__(512) zt_fwd8_d##DP##_k##BK(FwdArgs a) {         \
         attn_fwd_body<DP, BK, 8, false>(a);                                                        \
     }
-// Kernels on split operands: one per role, width and wave shape (shapes.h), of which
-// the launcher picks by the grid.  SC: 0 never keeps the scores, 1 always, 2 where s_out is set.
+// Kernels on split operands: one per role and width, each holding the role's wave
+// shapes (shapes.h), of which the launcher picks by the grid (FwdArgs::nq, ks); at
+// d = 32 one per shape.
+// SC: 0 never keeps the scores, 1 always, 2 where s_out is set.
 template <int DP, int SC, int NW, int NQ, int KS>
-DEVI void fwd_split_kernel(const FwdArgs &a) {
+DEVI bool fwd_shape(const FwdArgs &a, char *smem) {
+    if (a.nq != NQ || a.ks != KS || blockDim.x != 64 * NW) return false;  // workgroup-uniform
+    fwd_split_body<DP, NW, NQ, KS, SC>(a, smem);
+    return true;
+}
+template <FwdRole R, int DP, int SC>
+DEVI void fwd_shapes(const FwdArgs &a) {
+    __shared__ __attribute__((aligned(16))) char smem[fwd_lds(R, DP)];
+    constexpr FwdWavesList L = fwd_waves(R, DP);
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (void)(fwd_shape<DP, SC, L.s[I].nw, L.s[I].nq, L.s[I].ks>(a, smem) || ...);
+    }(std::make_integer_sequence<int, L.n>{});
+}
+template <int DP, int SC, int NW, int NQ, int KS>
+DEVI void fwd_one_shape(const FwdArgs &a) {
     __shared__ __attribute__((aligned(16))) char smem[fwd_lds(DP, {NW, NQ, KS})];
     fwd_split_body<DP, NW, NQ, KS, SC>(a, smem);
 }
-#define ZT_FWD_K(NAME, DP, SC, NW, NQ, KS)                                                           \
-    extern "C" __global__ void __launch_bounds__(512, 2)                                     \
-    NAME##_d##DP##_k32_##NW##NQ##KS(FwdArgs a) {                                                     \
-        fwd_split_kernel<DP, SC, NW, NQ, KS>(a);                                                     \
-    }
 // zt_fwd8ps_* is zt_fwd8p_* keeping the scores: its own name, so that a profile tells the two apart.
-#define ZT_8P_32(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 32, 0, NW, NQ, KS)
-#define ZT_8P_64(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 64, 0, NW, NQ, KS)
-#define ZT_8P_96(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 96, 0, NW, NQ, KS)
-#define ZT_8P_128(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 128, 0, NW, NQ, KS)
-#define ZT_8P_192(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 192, 2, NW, NQ, KS)
-#define ZT_8P_256(NW, NQ, KS) ZT_FWD_K(zt_fwd8p, 256, 2, NW, NQ, KS)
-#define ZT_8PS_32(NW, NQ, KS) ZT_FWD_K(zt_fwd8ps, 32, 1, NW, NQ, KS)
-#define ZT_8PS_64(NW, NQ, KS) ZT_FWD_K(zt_fwd8ps, 64, 1, NW, NQ, KS)
-#define ZT_8PS_96(NW, NQ, KS) ZT_FWD_K(zt_fwd8ps, 96, 1, NW, NQ, KS)
-#define ZT_8PS_128(NW, NQ, KS) ZT_FWD_K(zt_fwd8ps, 128, 1, NW, NQ, KS)
-#define ZT_P_32(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 32, 2, NW, NQ, KS)
-#define ZT_P_64(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 64, 2, NW, NQ, KS)
-#define ZT_P_96(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 96, 2, NW, NQ, KS)
-#define ZT_P_128(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 128, 2, NW, NQ, KS)
-#define ZT_P_192(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 192, 2, NW, NQ, KS)
-#define ZT_P_256(NW, NQ, KS) ZT_FWD_K(zt_fwdp, 256, 2, NW, NQ, KS)
-#define ZT_PK_32(NW, NQ, KS) ZT_FWD_K(zt_fwdpk, 32, 2, NW, NQ, KS)
-#define ZT_PK_64(NW, NQ, KS) ZT_FWD_K(zt_fwdpk, 64, 2, NW, NQ, KS)
-#define ZT_PK_96(NW, NQ, KS) ZT_FWD_K(zt_fwdpk, 96, 2, NW, NQ, KS)
-#define ZT_PK_128(NW, NQ, KS) ZT_FWD_K(zt_fwdpk, 128, 2, NW, NQ, KS)
+#define ZT_FWD_SPLIT(NAME, ROLE, DP, SC)                                                             \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME##_d##DP##_k32(FwdArgs a) {          \
+        fwd_shapes<FwdRole::ROLE, DP, SC>(a);                                                        \
+    }
+#define ZT_FWD_SHAPE(NAME, SC, NW, NQ, KS)                                                           \
+    extern "C" __global__ void __launch_bounds__(512, 2) NAME##_d32_k32_##NW##NQ##KS(FwdArgs a) { \
+        fwd_one_shape<32, SC, NW, NQ, KS>(a);                                                        \
+    }
+#define ZT_8P_32(NW, NQ, KS) ZT_FWD_SHAPE(zt_fwd8p, 0, NW, NQ, KS)
+#define ZT_8PS_32(NW, NQ, KS) ZT_FWD_SHAPE(zt_fwd8ps, 1, NW, NQ, KS)
+#define ZT_P_32(NW, NQ, KS) ZT_FWD_SHAPE(zt_fwdp, 2, NW, NQ, KS)
+#define ZT_PK_32(NW, NQ, KS) ZT_FWD_SHAPE(zt_fwdpk, 2, NW, NQ, KS)
 
 // Register-prefetched variants on f32 MFMA (32-key tiles; widths whose halves
 // are not whole 32-column groups).
@@ -819,14 +822,19 @@ ZT_FWD(192, 32) ZT_FWD(192, 64)
 ZT_FWD(224, 32) ZT_FWD(224, 64)
 ZT_FWD(256, 32) ZT_FWD(256, 64)
 ZT_FWD_PF(160) ZT_FWD_PF(224)
-ZT_FWD_HEADS_32(ZT_8P_32) ZT_FWD_HEADS_64(ZT_8P_64) ZT_FWD_HEADS_96(ZT_8P_96) ZT_FWD_HEADS_128(ZT_8P_128)
-ZT_FWD_HEADS_192(ZT_8P_192) ZT_FWD_HEADS_256(ZT_8P_256)
-ZT_FWD_HEADS_32(ZT_8PS_32) ZT_FWD_HEADS_64(ZT_8PS_64) ZT_FWD_HEADS_96(ZT_8PS_96) ZT_FWD_HEADS_128(ZT_8PS_128)
-ZT_FWD_ONE_32(ZT_P_32) ZT_FWD_ONE_64(ZT_P_64) ZT_FWD_ONE_96(ZT_P_96) ZT_FWD_ONE_128(ZT_P_128)
-ZT_FWD_ONE_192(ZT_P_192) ZT_FWD_ONE_256(ZT_P_256)
-ZT_FWD_SMALL_32(ZT_PK_32) ZT_FWD_SMALL_64(ZT_PK_64) ZT_FWD_SMALL_96(ZT_PK_96) ZT_FWD_SMALL_128(ZT_PK_128)
+ZT_FWD_HEADS_32(ZT_8P_32) ZT_FWD_SPLIT(zt_fwd8p, Heads, 64, 0)
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 96, 0) ZT_FWD_SPLIT(zt_fwd8p, Heads, 128, 0)
+ZT_FWD_HEADS_32(ZT_8PS_32) ZT_FWD_SPLIT(zt_fwd8ps, Heads, 64, 1)
+ZT_FWD_SPLIT(zt_fwd8ps, Heads, 96, 1) ZT_FWD_SPLIT(zt_fwd8ps, Heads, 128, 1)
+ZT_FWD_SPLIT(zt_fwd8p, Heads, 192, 2) ZT_FWD_SPLIT(zt_fwd8p, Heads, 256, 2)
+ZT_FWD_ONE_32(ZT_P_32) ZT_FWD_SPLIT(zt_fwdp, One, 64, 2)
+ZT_FWD_SPLIT(zt_fwdp, One, 96, 2) ZT_FWD_SPLIT(zt_fwdp, One, 128, 2)
+ZT_FWD_SPLIT(zt_fwdp, One, 192, 2) ZT_FWD_SPLIT(zt_fwdp, One, 256, 2)
+ZT_FWD_SMALL_32(ZT_PK_32) ZT_FWD_SPLIT(zt_fwdpk, Small, 64, 2)
+ZT_FWD_SPLIT(zt_fwdpk, Small, 96, 2) ZT_FWD_SPLIT(zt_fwdpk, Small, 128, 2)
 #else
 // A planted-defect build (test-only): the kernels of the negative-control
 // shapes, d = 32 (the reference entry points) and d = 128 (the training path).
-ZT_FWD_HEADS_32(ZT_8P_32) ZT_FWD_HEADS_128(ZT_8P_128) ZT_FWD_HEADS_128(ZT_8PS_128)
+ZT_FWD_HEADS_32(ZT_8P_32) ZT_FWD_SPLIT(zt_fwd8p, Heads, 128, 0)
+ZT_FWD_SPLIT(zt_fwd8ps, Heads, 128, 1)
 #endif

@@ -271,13 +271,14 @@ int fwd_key_split(int B, int T, int n_heads, int hw, int dp, int dim, int bk, in
     return able ? tuned(kTuneFKS, wgs <= cus ? 2 : 1) : 1;
 }
 
-// The role of p's kernel, and whether it is built in p's wave shape.
+// The role of p's kernel, and whether it has p's wave shape.
 FwdRole fwd_role(const FwdPlan &p) {
     return p.nw == 8 && p.hw > 1 ? FwdRole::Heads : p.small ? FwdRole::Small : FwdRole::One;
 }
 bool fwd_shape_built(const FwdPlan &p, int dp) {
-    for (const FwdWaves &s : fwd_waves(fwd_role(p), dp).s)
-        if (s.nw == p.nw && s.nq == p.nq && s.ks == p.ks) return true;
+    const FwdWavesList l = fwd_waves(fwd_role(p), dp);
+    for (int i = 0; i < l.n; ++i)
+        if (l.s[i].nw == p.nw && l.s[i].nq == p.nq && l.s[i].ks == p.ks) return true;
     return false;
 }
 
@@ -325,13 +326,12 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
     const int shape = tuned(kTuneFShape, 10 * p.nq + p.ks);
     p.nq = shape / 10;
     p.ks = shape % 10;
-    if (!fwd_shape_built(p, dp)) {  // a forced shape that the role is not built in
-        for (const FwdWaves &s : fwd_waves(fwd_role(p), dp).s)
-            if (s.nw == p.nw) {
-                p.nq = s.nq;
-                p.ks = s.ks;
-                break;
-            }
+    if (!fwd_shape_built(p, dp)) {  // a forced shape that the role does not have: its first
+        const FwdWavesList l = fwd_waves(fwd_role(p), dp);
+        int i = 0;
+        while (i + 1 < l.n && l.s[i].nw != p.nw) ++i;
+        p.nq = l.s[i].nq;
+        p.ks = l.s[i].ks;
     }
     while (p.nw / (p.ks * p.ds) < p.hw) p.hw /= 2;
     return p;
@@ -339,7 +339,8 @@ FwdPlan fwd_plan(int B, int T, int n_heads, int n_kv_heads, int dp, int dim, int
 
 // The LDS its kernel takes per workgroup.
 size_t fwd_plan_lds(const FwdPlan &p, int dp, int bk) {
-    return p.split ? (size_t)fwd_lds(dp, FwdWaves{p.nw, p.nq, p.ks}) : fwd_tile_bytes(dp, bk);
+    if (!p.split) return fwd_tile_bytes(dp, bk);
+    return fwd_shape_kernels(dp) ? fwd_lds(dp, FwdWaves{p.nw, p.nq, p.ks}) : fwd_lds(fwd_role(p), dp);
 }
 
 // Forward kernel name: the split-operand kernels, and the f32 MFMA kernels for
@@ -566,7 +567,7 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     a.q = q; a.k = k; a.v = v; a.out = out; a.lse = lse; a.s_out = s_out;
     a.B = B; a.T = T; a.H = n_heads; a.Hkv = n_kv_heads; a.dim = dim;
     a.q_offset = q_offset; a.n_keys = n_keys; a.kv_rows = kv_rows;
-    a.HW = p.hw;
+    a.HW = p.hw; a.nq = p.nq; a.ks = p.ks;
     const int rows_per_wg = fwd_rows(p);
     a.n_row_tiles = (T + rows_per_wg - 1) / rows_per_wg;
     a.n_head_blocks = n_heads / a.HW;
@@ -581,7 +582,7 @@ int forward_impl(const float *q, const float *k, const float *v, float *out, int
     if (!grid_ok(blocks, 64u * p.nw)) return 1;
     char name[64];
     fwd_kernel_name(name, sizeof name, dim, dp, bk, p, s_out != nullptr);
-    if (p.split) {  // the shape's kernel (shapes.h)
+    if (p.split && fwd_shape_kernels(dp)) {  // the shape's kernel (shapes.h)
         const size_t n = strlen(name);
         snprintf(name + n, sizeof name - n, "_%d%d%d", p.nw, p.nq, p.ks);
     }
@@ -784,7 +785,7 @@ size_t zt_attn_forward_shmem(int dim, int tile, int group_q) {
     (void)group_q;
     if (!zt_attn_dim_ok(dim)) return 0;
     const int dp = pad32(dim), bk = key_tile(Tiled::Forward, dp, tile, dim);
-    return fwd_splits(dim, dp, bk) ? (size_t)fwd_lds_most(dp) : fwd_tile_bytes(dp, bk);
+    return fwd_splits(dim, dp, bk) ? (size_t)fwd_lds(dp) : fwd_tile_bytes(dp, bk);
 }
 
 size_t zt_attn_bwd_dq_shmem(int dim, int tile) {
@@ -956,7 +957,9 @@ static float *ws_tiles(void *workspace, int B, int T, int n_heads) {
 // 31 / 19 / 14; 12 over 4 heads at d = 64, 4 x 512 rows 96 / 63 / 72; 32 over 8 at d =
 // 128, T = 512 182 / 177, T = 4096 1517 / 2784.  At d = 32 four parts of two blocks
 // leave room for two workgroups per CU (shapes.h) and win on every larger grid:
-// one sequence of 2060 rows of 32 over 8 heads 445 / 283, 4 x 896 218 / 179.
+// one sequence of 2060 rows of 32 over 8 heads 445 / 283, 4 x 896 218 / 179.  At d = 64
+// two blocks win up to one 64-key workgroup per CU (8 heads over 4, one sequence of 3000
+// rows 358 / 236; MHA, 1200 rows of 8 heads 84 / 66, 2040 rows of 7 heads 134 / 97).
 static void dkdv_split_shape(int B, int T, int n_kv_heads, int dp, int cus, int *parts, int *kblocks) {
     const long long wgs = (long long)((T + 63) / 64) * n_kv_heads * B;  // 64 keys each
     int kb = 4;
