@@ -1,4 +1,6 @@
-// f32 products on the bf16 matrix cores, by an exact three-way split.
+// f32 products on the bf16 matrix cores, by an exact three-way split (the method of
+// Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype
+// For Higher-Precision Computations", ARITH 2019).
 //
 // v_mfma_f32_16x16x4_f32 peaks at 157 TFLOP/s on gfx950 and, as measured here,
 // shares the SIMD with the vector ALU; v_mfma_f32_16x16x32_bf16 runs at 16
